@@ -125,7 +125,7 @@ def main():
             sx.solve(msys, tf, tb, tu, tol_rel=tol, iters=False)
         torch.cuda.synchronize()
         prof = {}
-        for name in ("k_ess_gather", "k_condense", "k_assemble", "k_band_solve",
+        for name in ("k_ess_gather", "k_condense", "k_assemble", "k_tree", "k_band_solve",
                      "k_backsub", "k_pcg"):
             tot = C.c_double(); cnt = C.c_longlong()
             L.semx_profile_query(name.encode(), C.byref(tot), C.byref(cnt))
@@ -193,30 +193,28 @@ def main():
     u, _ = fresh_solve(S)
     err_exact = float(np.abs(u[:, :P.nPlane] - ue[:, :P.nPlane]).max())
 
-    # algorithmic bytes of k_band_solve per launch: every mode's band factor
-    # (nsolve x nband doubles) read once -- the Re and Im planes share it --
-    # plus the condensed RHS in and the boundary solution out, per plane;
-    # the two-sweep count (the factor streamed by the forward and again by
-    # the backward sweep, as dpbtrs does) is reported beside it
+    # algorithmic bytes of the boundary solve (the elimination tree's stages,
+    # k_tree): every mode's region matrices read once -- the Re and Im planes
+    # share them -- plus the condensed RHS in and the boundary solution out,
+    # per plane
     n0 = S.info["nsolve0"]
     ldab = S.info["ldab"]
-    bytes_factor = (nz // 2) * n0 * ldab * 8
+    bytes_factor = S.info["factor_kB"] * 1000
     bytes_rhs = nplanes * (P.nel * P.next + n0) * 8
     band_bytes = bytes_factor + bytes_rhs
-    band_bytes2 = 2 * bytes_factor + bytes_rhs
-    band_ms = kprof["k_band_solve"]
+    band_ms = kprof["k_tree"]
     achieved = band_bytes / (band_ms * 1e-3) / 1e9
-    # the whole all-mode solve's algorithmic bytes: factor once per mode,
+    # the whole all-mode solve's algorithmic bytes: matrices once per mode,
     # one condensed element-matrix set per mode (one geometric set), forcing
     # in and solution out per plane, BC lines
     nline = P.nbound * P.np
-    solve_bytes = 8 * ((nz // 2) * (n0 * ldab + P.nsets * (P.next * P.nint + P.nint ** 2))
-                       + nplanes * (2 * P.nPlane + nline))
+    solve_bytes = bytes_factor + 8 * (
+        (nz // 2) * P.nsets * (P.next * P.nint + P.nint ** 2) + nplanes * (2 * P.nPlane + nline))
 
-    # HBM bytes per k_band_solve launch from the committed rocprofv3 counter
-    # summary (FETCH_SIZE / WRITE_SIZE scaled by a plain copy kernel)
+    # HBM bytes per solve of the k_tree stages from the committed rocprofv3
+    # counter summary (FETCH_SIZE / WRITE_SIZE scaled by a plain copy kernel)
     traffic = None
-    tpath = os.path.join(ROOT, "profiles", "k_band_solve_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "k_tree_traffic.json")
     if os.path.exists(tpath):
         traffic = json.load(open(tpath)).get("traffic_bytes")
 
@@ -242,7 +240,7 @@ def main():
             "setup_s": round(t_setup, 3),
         },
         "roofline": {
-            "kernel": "k_band_solve",
+            "kernel": "k_tree",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
@@ -251,7 +249,6 @@ def main():
             "traffic": traffic,
             "bytes_per_launch": band_bytes,
             "avg_launch_ms": band_ms,
-            "frac_two_sweeps": band_bytes2 / (band_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
             "whole_solve_frac": solve_bytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
             "whole_solve_bytes": solve_bytes,
         },
@@ -553,7 +550,7 @@ def dns_bench(args, torch, sx, L):
     D.run(args.dns_steps, u, v, w, p)
     torch.cuda.synchronize()
     prof = {}
-    for name in ("k_band_solve", "k_condense", "k_assemble", "k_backsub", "k_dft_z",
+    for name in ("k_tree", "k_condense", "k_assemble", "k_backsub", "k_dft_z",
                  "k_grad_xy", "k_grad_nl", "k_grad_z", "k_smooth", "dns_nonlinear"):
         tot = C.c_double(); cnt = C.c_longlong()
         L.semx_profile_query(name.encode(), C.byref(tot), C.byref(cnt))
@@ -576,16 +573,10 @@ def dns_bench(args, torch, sx, L):
     ng1, nrep = D.graph_info()
     D.set_graph(False)
     progress(f"dns eager {ms:.3f} ms/step, graph replay {gms:.3f} ms/step ({ng1} graphs)")
-    # algorithmic HBM bytes of the band sweeps, which bound the step: the
-    # velocity and the pressure system, every mode's factor read by the
-    # forward and the backward sweep (nsolve x nband doubles per mode)
-    band_bytes = 2 * (nz // 2) * 2 * P.nsolve * P.nband * 8
-    band_ms = prof.get("k_band_solve", {}).get("ms_per_step", float("nan"))
-    # the whole step's algorithmic bytes: both systems' factors once per
-    # mode, and about 46 compulsory passes over a field (nonlinear terms 6,
-    # waveProp 21, setPForce 4, pressure 2, projection 7, velocity 6)
+    # the step's compulsory passes over a field, about 46 of them (nonlinear
+    # terms 6, waveProp 21, setPForce 4, pressure 2, projection 7, velocity 6)
     field_bytes = nz * P.planeSize * 8
-    step_bytes = 2 * (nz // 2) * P.nsolve * P.nband * 8 + 46 * field_bytes
+    step_bytes = 46 * field_bytes
     return {
         "metric": "DNS steps/s",
         "value": 1e3 / ms,
@@ -604,15 +595,7 @@ def dns_bench(args, torch, sx, L):
                           "graph per role assignment of the step's buffers"},
         "step_hbm": {"bytes_per_step": step_bytes,
                      "frac_of_peak": step_bytes / (ms * 1e-3) / 8e12,
-                     "what": "both systems' band factors once per mode plus 46 field passes "
-                             "over the measured step time"},
-        "band_hbm": {"bytes_per_step": band_bytes,
-                     "achieved_gb_s": band_bytes / (band_ms * 1e-3) / 1e9,
-                     "frac_of_peak_in_sweeps": band_bytes / (band_ms * 1e-3) / 8e12,
-                     "frac_of_peak_whole_step": band_bytes / (ms * 1e-3) / 8e12,
-                     "what": "algorithmic band-factor bytes (2 systems x modes x 2 sweeps x "
-                             "nsolve x nband x 8 B) over the sweeps' time and over the whole "
-                             "step (field traffic not counted)"},
+                     "what": "46 field passes over the measured step time"},
     }
 
 

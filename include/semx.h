@@ -190,14 +190,17 @@ int semx_helm_create_svv (semx_mesh mesh, double lambda2, double beta,
                           int nmode_total, semx_helm* helm);
 int semx_helm_destroy (semx_helm helm);
 /* info[8] = nmodes nz method nsolve(mode0) nband nblk(block size)
- *           bytes_per_solve_factor(MB*1000, int) singular(mode0)           */
+ *           bytes_per_solve_factor(MB*1000, int) singular(mode0); the factor
+ *           is the elimination tree's matrices or the band's factor        */
 int semx_helm_info (semx_helm helm, int* info);
 /* How the direct planes' band sweeps run; no counterpart in semtex (whose
  * dpbtrs is one call) -- and how the PCG planes run.  info[6] = partitions
  * per mode of the partitioned sweep (1: not available), the sweep variant
  * the first call picked for 1, 2 and 3 fields (0 before that call; 1-7 one
  * workgroup per mode, field or plane over the whole band, 8 the
- * partitioned sweep), workgroups per mode of the cooperative sweep (0: not
+ * partitioned sweep, 9 the elimination tree: regions of elements merged
+ * level by level, each eliminated with dense matrices; the default, with
+ * SEMX_TREE=0 or any of the sweeps' own switches selecting the sweeps), workgroups per mode of the cooperative sweep (0: not
  * used), workgroups per PCG plane in the last solve.                      */
 int semx_helm_sweep_info (semx_helm helm, int* info);
 /* Host copies of one element's condensed matrices for mode index m

@@ -50,6 +50,9 @@ int helm_solve(Helm& H, double* f, const double* bc, double* u, double tol_rel, 
 int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* bcs,
                       double* const* us, double tol_rel, int step_max, int* iters,
                       hipStream_t s);
+// The boundary systems of the direct modes through the elimination tree:
+// condensed right-hand sides d.Fb (pFb doubles per field) to d.sol (psol).
+int tree_solve(Helm& H, int nf, size_t pFb, size_t psol, hipStream_t s);
 // Device address (current device) of the static scratch array of the
 // allocation-free entry points; looked up once per device.
 int noalloc_scratch(double** out);

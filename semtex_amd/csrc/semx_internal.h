@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "semx.h"
+#include "semx_tree.h"
 
 namespace semx {
 
@@ -82,6 +83,8 @@ struct ModeSys {
   int nblk = 0;
 };
 
+struct TreeDev;
+
 struct HelmDev {
   double* hbi = nullptr;      // nmodes*nset*next*nint
   double* hii = nullptr;      // nmodes*nset*nint*nint
@@ -128,6 +131,8 @@ struct HelmDev {
   // PCG workgroup map (4 ints per workgroup: plane slot, part, parts, 0),
   // balanced by the planes' last iteration counts
   int* pwmap = nullptr;
+  // elimination tree: matrices, region tables, per-field scratch
+  TreeDev* tree = nullptr;
 };
 
 struct Helm {
@@ -206,6 +211,7 @@ struct Helm {
   std::vector<int> prow;
   std::vector<long long> spk_off;
   std::vector<double> spk;            // host, released after upload
+  Tree tree;                          // elimination tree (tree.on), else the band sweeps
   bool on_device = false;
   HelmDev d;
 };
@@ -232,6 +238,12 @@ int mesh_upload(Mesh& M);
 void mesh_release(Mesh& M);
 int helm_upload(Helm& H);
 void helm_release(Helm& H);
+
+// elimination tree on the device (semx_tree.hip): tables and matrices, the
+// scratch and launch lists for nf fields, and their release
+int tree_upload(Helm& H);
+int tree_scratch(Helm& H, int nf);
+void tree_release(Helm& H);
 
 }  // namespace semx
 

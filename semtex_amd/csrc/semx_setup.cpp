@@ -1165,6 +1165,14 @@ int helm_build(Helm& H) {
     S.n = S.singular ? M.nsolve - 1 : M.nsolve;
     if (S.kind == SEMX_DIRECT) {
       if (H.npass == 0) return SEMX_E_UNSUPPORTED;
+    }
+  }
+  // the elimination tree, or the band sweeps where it does not apply
+  tree_plan(H);
+  if (H.tree.on) { H.coop_mode = false; H.xcoop = false; }
+  for (int m = 0; m < nmodes && !H.tree.on; ++m) {
+    ModeSys& S = H.modes[m];
+    if (S.kind == SEMX_DIRECT) {
       S.nblk = (S.n + nb - 1) / nb;
       S.off_H = offH;
       S.off_L = offL;
@@ -1180,7 +1188,7 @@ int helm_build(Helm& H) {
   // the neighbouring partition).  SEMX_BAND_PARTS sets the count (1: off).
   H.npart = 1;
   H.prow.clear(); H.spk_off.clear(); H.spk.clear();
-  if (H.band_ext && nb == 32 && H.kd >= 1) {
+  if (H.band_ext && nb == 32 && H.kd >= 1 && !H.tree.on) {
     int ndirect = 0, nmin = INT32_MAX;
     for (int m = 0; m < nmodes; ++m)
       if (H.modes[m].kind == SEMX_DIRECT) { ++ndirect; nmin = std::min(nmin, H.modes[m].n); }
@@ -1259,6 +1267,7 @@ int helm_build(Helm& H) {
       if (st) { status[m] = st; return; }
     }
     if (S.kind == SEMX_DIRECT) {
+      if (H.tree.on) return;
       const int n = S.n, kd = H.kd, ldab = H.ldab, kdp = H.kdp;
       std::vector<double> band((size_t)std::max(n, 1) * ldab, 0.0);
       double* A = band.data();
@@ -1384,6 +1393,8 @@ int helm_build(Helm& H) {
     pool.emplace_back([&, t]() { for (int m = t; m < nmodes; m += nth) work(m); });
   for (auto& th : pool) th.join();
   for (int st : status) if (st) return st;
+  if (H.tree.on)
+    if (const int st = tree_factor(H)) return st;
   // plane list: every plane except the Nyquist plane 1, which only the
   // planes that start at mode 0 hold (ROOTONLY skip, field.cpp:566); with
   // base_mode > 0 plane 1 is Im of mode base_mode and is solved

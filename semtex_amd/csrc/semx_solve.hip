@@ -11,6 +11,9 @@
 //                   streamed as NB-column panels, the RHS in an LDS window
 //   k_band_coop     the same with several workgroups per mode in a lagged
 //                   pipeline (opt-in)
+//   k_tree_*        the same systems along the elimination tree (semx_tree.hip),
+//                   the default; the band sweeps above serve their own
+//                   switches and systems a tree does not fit
 //   k_backsub[_staged]
 //                   interior recovery u_i = hii F_i - hbi^T u_b and essential
 //                   re-imposition (Element::global2localSC, Field::setEssential)
@@ -2974,6 +2977,7 @@ int helm_upload(Helm& H) {
     if ((st = dev_upload(&H.d.pcg_plane, H.pcg_plane.data(), H.pcg_plane.size()))) return st;
   }
   if ((st = dev_upload(&H.d.plane_of, H.plane_of.data(), H.plane_of.size()))) return st;
+  if ((st = tree_upload(H))) return st;
   if ((st = coop_setup(H))) return st;
   if (H.npart > 1) {
     int nd = 0;
@@ -3010,6 +3014,7 @@ void helm_release(Helm& H) {
   dev_free(H.d.err);
   dev_free(H.d.spk); dev_free(H.d.spk_off); dev_free(H.d.prow); dev_free(H.d.pslot);
   dev_free(H.d.pctr); dev_free(H.d.pslot2); dev_free(H.d.pwmap);
+  tree_release(H);
   H.pcg_ws = 0;
   H.pcg_nwg = 0;
   H.nf_cap = 0;
@@ -3017,6 +3022,10 @@ void helm_release(Helm& H) {
 }
 
 int helm_scratch(Helm& H, int nf, hipStream_t s) {
+  if (H.tree.on) {
+    if (nf > H.nf_cap) HIPCHK(hipStreamSynchronize(s));
+    if (const int st = tree_scratch(H, nf)) return st;
+  }
   if (nf <= H.nf_cap) return SEMX_OK;
   Mesh& M = *H.M;
   HIPCHK(hipStreamSynchronize(s));
@@ -3194,7 +3203,10 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       hipLaunchKernelGGL(k_condense, eg, dim3(ELT_THREADS), lds_c, s, e);
     prof_end(s, "k_condense", ev);
   }
-  if (!H.dmode.empty()) {
+  if (!H.dmode.empty() && H.tree.on) {
+    if ((st = tree_solve(H, nf, pFb, psol, s))) return st;
+    H.band_pick[nf] = 9;
+  } else if (!H.dmode.empty()) {
     for (int i = 0; i < nf; ++i) {
       prof_begin(s, &ev);
       hipLaunchKernelGGL(k_assemble, dim3((M.nglobal + 255) / 256, H.nplanes), dim3(256), 0, s,
@@ -3925,7 +3937,8 @@ int semx_helm_info(semx_helm helm, int* info) {
   const Helm& H = helm->H;
   long long bytes = 0;
   for (const ModeSys& S : H.modes)
-    if (S.kind == SEMX_DIRECT) bytes += (long long)S.n * H.ldab * 8;
+    if (S.kind == SEMX_DIRECT)
+      bytes += H.tree.on ? H.tree.mstride * 8 : (long long)S.n * H.ldab * 8;
   info[0] = H.nmodes; info[1] = H.nz; info[2] = H.method;
   info[3] = H.modes.empty() ? 0 : H.modes[0].n;
   info[4] = H.ldab; info[5] = H.nb;
