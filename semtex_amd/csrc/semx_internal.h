@@ -84,6 +84,7 @@ struct ModeSys {
 };
 
 struct TreeDev;
+struct ChipDev;
 
 struct HelmDev {
   double* hbi = nullptr;      // nmodes*nset*next*nint
@@ -133,6 +134,9 @@ struct HelmDev {
   int* pwmap = nullptr;
   // elimination tree: matrices, region tables, per-field scratch
   TreeDev* tree = nullptr;
+  // on-chip PCG: tables, exchange slots (null: not built; see chip_tried)
+  ChipDev* chip = nullptr;
+  bool chip_tried = false;
 };
 
 struct Helm {

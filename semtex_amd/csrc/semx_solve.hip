@@ -32,6 +32,7 @@
 #include <map>
 #include <string>
 
+#include "semx_chip.h"
 #include "semx_hip.h"
 
 using namespace semx;
@@ -3015,6 +3016,14 @@ void helm_release(Helm& H) {
   dev_free(H.d.spk); dev_free(H.d.spk_off); dev_free(H.d.prow); dev_free(H.d.pslot);
   dev_free(H.d.pctr); dev_free(H.d.pslot2); dev_free(H.d.pwmap);
   tree_release(H);
+  if (ChipDev* C = H.d.chip) {
+    chip_release(C->plan);
+    dev_free(C->inst); dev_free(C->exch); dev_free(C->red); dev_free(C->ticket);
+    for (int2*& o : C->order) dev_free(o);
+    delete C;
+    H.d.chip = nullptr;
+  }
+  H.d.chip_tried = false;
   H.pcg_ws = 0;
   H.pcg_nwg = 0;
   H.nf_cap = 0;
@@ -3116,6 +3125,95 @@ int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, si
   H.pcg_nwg = (int)tot;
   H.pcg_wtop = std::max(2, *std::max_element(Wp.begin(), Wp.end()));
   return SEMX_OK;
+}
+
+// The on-chip PCG of a system's planes for nf fields: tables on first use,
+// slots for the largest field count met, and the order the planes are taken
+// in: as listed (low modes, which take the most iterations, first), or by
+// the iteration counts of the last solve that read them back.  H.d.chip
+// stays null where the on-chip iteration does not take the system; its own
+// switches (SEMX_PCG_WG, SEMX_PCG_OP, SEMX_PCG_CHIP=0) and BF16 refinement
+// select k_pcg.
+int chip_prepare(Helm& H, int nfields) {
+  Mesh& M = *H.M;
+  int nf = nfields;
+  const int npcg = (int)H.pcg_plane.size();
+  int st;
+  if (!H.d.chip_tried) {
+    H.d.chip_tried = true;
+    ChipPlan plan;
+    const ChipMesh* dm = nullptr;
+    if ((st = chip_plan(M, plan, &dm))) return st;
+    if (!plan.ok) return SEMX_OK;
+    ChipDev* C = new ChipDev();
+    H.d.chip = C;
+    C->plan = plan;
+    C->rank.resize(npcg);
+    for (int p = 0; p < npcg; ++p) C->rank[p] = p;
+    if ((st = dev_upload<unsigned>(&C->ticket, nullptr, 1))) return st;
+    if (!H.d.err && (st = dev_upload<int>(&H.d.err, nullptr, 1))) return st;
+  }
+  ChipDev* C = H.d.chip;
+  if (!C) return SEMX_OK;
+  const int W = C->plan.W;
+  if (nf > C->nf_cap || C->work != H.d.work) {
+    nf = std::max(nf, C->nf_cap);
+    dev_free(C->inst); dev_free(C->exch); dev_free(C->red);
+    C->nf_cap = 0;
+    const size_t np_ = (size_t)npcg * nf;
+    if ((st = dev_upload<double>(&C->exch, nullptr, np_ * 4 * C->plan.nif))) return st;
+    if ((st = dev_upload<double>(&C->red, nullptr, np_ * 12 * W))) return st;
+    std::vector<ChipInst> inst(npcg);
+    for (int i = 0; i < npcg; ++i) {
+      ChipInst& I = inst[i];
+      I.pidx = H.pcg_plane[i];
+      I.plane = H.plane_of[I.pidx];
+      const int m = I.plane >> 1;
+      I.mesh = (const ChipMesh*)C->plan.store;
+      I.pc = H.d.pc + (size_t)m * H.npts;
+      I.pc32 = H.d.pc32 + (size_t)m * H.npts;
+      I.mq = H.d.mq ? H.d.mq + (size_t)m * M.nset * M.npnp : nullptr;
+      I.work = H.d.work + (size_t)i * H.workstride;
+      I.hcon = M.cyl ? 1.0 : H.lambda2 + H.modes[m].betak2;
+      I.n = H.modes[m].n;
+      I.svv = H.lambda2 > EPSDP;
+      I.exch = (long long)i * 4 * C->plan.nif;
+      I.red = (long long)i * 12 * W;
+    }
+    if ((st = dev_upload(&C->inst, inst.data(), inst.size()))) return st;
+    C->nf_cap = nf;
+    C->work = H.d.work;
+  }
+  nf = nfields;
+  if (!C->order[nf]) {
+    std::vector<int2> o;
+    for (int p : C->rank)
+      for (int f = 0; f < nf; ++f)
+        for (int w = 0; w < W; ++w) o.push_back(make_int2(f * npcg + p, w));
+    if ((st = dev_upload(&C->order[nf], o.data(), o.size()))) return st;
+  }
+  int cus = 256, dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess)
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  H.pcg_w = C->ranked ? W : std::max(1, std::min(W, cus / npcg));
+  return SEMX_OK;
+}
+
+// the planes in decreasing order of their measured iteration counts
+void chip_rank(Helm& H, const std::vector<int>& it, int nf) {
+  ChipDev* C = H.d.chip;
+  if (H.pcg_frozen || !C) return;
+  const int npcg = (int)H.pcg_plane.size();
+  std::vector<int> cnt(npcg, 0), rank(npcg);
+  for (int f = 0; f < nf; ++f)
+    for (int p = 0; p < npcg; ++p)
+      cnt[p] = std::max(cnt[p], std::abs(it[(size_t)f * npcg + p]));
+  for (int p = 0; p < npcg; ++p) rank[p] = p;
+  std::stable_sort(rank.begin(), rank.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
+  C->ranked = true;
+  if (rank == C->rank) return;
+  C->rank = rank;
+  for (int2*& o : C->order) dev_free(o);
 }
 
 int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* bcs,
@@ -3541,7 +3639,48 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       prof_end(s, "k_backsub", ev);
     }
   }
-  if (!H.pcg_plane.empty()) {
+  bool chip = !H.pcg_plane.empty() && H.pcg_prec != SEMX_PCG_BF16_REFINED &&
+              !getenv("SEMX_PCG_WG") && !getenv("SEMX_PCG_OP") &&
+              !(getenv("SEMX_PCG_CHIP") && atoi(getenv("SEMX_PCG_CHIP")) == 0);
+  if (chip) {
+    if ((st = chip_prepare(H, nf))) return st;
+    chip = H.d.chip != nullptr;
+  }
+  if (chip) {
+    const ChipDev& C = *H.d.chip;
+    const int npcg = (int)H.pcg_plane.size(), W = C.plan.W;
+    ChipArgs ca{};
+    ca.inst = C.inst; ca.order = C.order[nf]; ca.ticket = C.ticket;
+    ca.exch = C.exch; ca.red = C.red;
+    ca.exchF = (long long)npcg * 4 * C.plan.nif; ca.redF = (long long)npcg * 12 * W;
+    ca.workF = (long long)npcg * H.workstride;
+    ca.iters = H.d.iters; ca.err = H.d.err; ca.count = npcg;
+    ca.planeSize = M.planeSize; ca.nzero = nzero;
+    ca.tol = tol_rel; ca.step_max = step_max;
+    ca.inner_tol = H.inner_tol; ca.max_outer = H.max_outer;
+    ca.Fb = H.d.Fb; ca.Fi = H.d.Fi; ca.g = H.d.g;
+    ca.FbF = (long long)pFb; ca.FiF = (long long)pFi; ca.gF = (long long)pg;
+    for (int i = 0; i < nf; ++i) ca.u[i] = us[i];
+    if ((st = chip_launch(ca, H.pcg_prec != SEMX_PCG_FP64, npcg * nf * W, C.plan.lds64,
+                          W > 1 ? (long long)npcg * nf * 4 * C.plan.nif : 0,
+                          W > 1 ? (long long)npcg * nf * 12 * W : 0, s)))
+      return st;
+    if (iters) {
+      std::vector<int> it((size_t)npcg * nf);
+      HIPCHK(hipMemcpyAsync(it.data(), H.d.iters, it.size() * sizeof(int),
+                            hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      int mx = 0;
+      bool limit = false;
+      for (int v : it) { limit |= v < 0; mx = std::max(mx, v < 0 ? -v : v); }
+      *iters = mx;
+      if (limit) {
+        const int st2 = helm_check(H, s);
+        return st2 ? st2 : SEMX_E_MAXITER;
+      }
+      chip_rank(H, it, nf);
+    }
+  } else if (!H.pcg_plane.empty()) {
     PcgArgs pa;
     pa.np = M.np; pa.npnp = M.npnp; pa.next = M.next; pa.nint = M.nint; pa.nel = M.nel;
     pa.nglobal = M.nglobal; pa.nsolve = M.nsolve; pa.nzero = nzero; pa.npts = H.npts;
@@ -3729,7 +3868,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
 // first check after it happened, whatever the caller passed for iters.
 int helm_check(Helm& H, hipStream_t s) {
   HIPCHK(hipStreamSynchronize(s));
-  if ((H.coop_w <= 0 && H.npart <= 1 && H.pcg_w <= 1) || !H.d.err) return SEMX_OK;
+  if ((H.coop_w <= 0 && H.npart <= 1 && H.pcg_w <= 1 && !H.d.chip) || !H.d.err) return SEMX_OK;
   int e = 0;
   HIPCHK(hipMemcpy(&e, H.d.err, sizeof(int), hipMemcpyDeviceToHost));
   if (!e) return SEMX_OK;
@@ -4022,12 +4161,24 @@ struct semx_batch_s {
   int count = 0, prec = SEMX_PCG_FP64, max_outer = 12;
   double inner_tol = 1e-5;
   size_t lds = 0;
+  // on-chip iteration (semx_pcg.hip): tables per distinct mesh, slots, order
+  bool chip = false;
+  std::map<const Mesh*, ChipPlan> plans;
+  ChipInst* cinst = nullptr;
+  double* exch = nullptr;
+  double* red = nullptr;
+  unsigned* ticket = nullptr;
+  int2* order = nullptr;
+  long long nexch = 0, nred = 0;
 };
 
 static void batch_free(semx_batch_s* b) {
   if (!b) return;
   dev_free(b->inst); dev_free(b->work); dev_free(b->iters); dev_free(b->ptrs);
   dev_free(b->wmap); dev_free(b->pctr); dev_free(b->pslot); dev_free(b->err);
+  for (auto& kv : b->plans) chip_release(kv.second);
+  dev_free(b->cinst); dev_free(b->exch); dev_free(b->red); dev_free(b->ticket);
+  dev_free(b->order);
   delete b;
 }
 
@@ -4092,6 +4243,72 @@ static int batch_layout(semx_batch_s* b, const std::vector<double>& cost) {
   return SEMX_OK;
 }
 
+// The order workgroups take an on-chip batch's problems in: longest first,
+// by the expected time (iterations growing with the elements per side and
+// np), then by the measured iterations; several-workgroup problems take
+// about twice the time of an iteration of the others.
+static int batch_chip_order(semx_batch_s* b, const std::vector<double>& its) {
+  std::vector<int> ord(b->count);
+  std::vector<double> cost(b->count);
+  for (int i = 0; i < b->count; ++i) {
+    ord[i] = i;
+    cost[i] = its[i] * (b->plans[b->helms[i]->H.M].W > 1 ? 2.0 : 1.0);
+  }
+  std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+  std::vector<int2> o;
+  for (int i : ord)
+    for (int w = 0; w < b->plans[b->helms[i]->H.M].W; ++w) o.push_back(make_int2(i, w));
+  dev_free(b->order);
+  b->nwg = (int)o.size();
+  return dev_upload(&b->order, o.data(), o.size());
+}
+
+// Tables of the on-chip iteration for every problem of a batch; b->chip
+// stays false where one of them does not fit it.
+static int batch_chip_setup(semx_batch_s* b) {
+  if (b->prec == SEMX_PCG_BF16_REFINED || getenv("SEMX_BATCH_OP") || getenv("SEMX_BATCH_WG") ||
+      (getenv("SEMX_PCG_CHIP") && atoi(getenv("SEMX_PCG_CHIP")) == 0))
+    return SEMX_OK;
+  for (semx_helm h : b->helms) if (!chip_workgroups(*h->H.M)) return SEMX_OK;
+  int st;
+  std::vector<ChipInst> inst(b->count);
+  std::vector<double> its(b->count);
+  size_t lds = 0;
+  long long nex = 0, nrd = 0;
+  for (int i = 0; i < b->count; ++i) {
+    Helm& H = b->helms[i]->H;
+    Mesh& M = *H.M;
+    if (!b->plans.count(&M)) {
+      const ChipMesh* dm = nullptr;
+      ChipPlan& P = b->plans[&M];
+      if ((st = chip_plan(M, P, &dm))) return st;
+      if (!P.ok) return SEMX_OK;
+    }
+    const ChipPlan& P = b->plans[&M];
+    ChipInst& I = inst[i];
+    I.mesh = (const ChipMesh*)P.store;
+    I.pc = H.d.pc; I.pc32 = H.d.pc32; I.mq = H.d.mq;
+    I.work = b->hinst[i].work;
+    I.hcon = b->hinst[i].op.hcon;
+    I.n = b->hinst[i].n;
+    I.svv = H.lambda2 > EPSDP;
+    I.plane = I.pidx = 0;
+    I.exch = nex; I.red = nrd;
+    if (P.W > 1) { nex += 4LL * P.nif; nrd += 12LL * P.W; b->nmulti++; }
+    lds = std::max(lds, P.lds64);
+    its[i] = std::sqrt((double)M.nel) * M.np;
+  }
+  if ((st = dev_upload(&b->cinst, inst.data(), inst.size()))) return st;
+  if ((st = dev_upload<double>(&b->exch, nullptr, (size_t)nex))) return st;
+  if ((st = dev_upload<double>(&b->red, nullptr, (size_t)nrd))) return st;
+  if ((st = dev_upload<unsigned>(&b->ticket, nullptr, 1))) return st;
+  b->nexch = nex; b->nred = nrd;
+  b->lds = lds;
+  b->chip = true;
+  b->tuned = true;
+  return batch_chip_order(b, its);
+}
+
 int semx_batch_create(int count, const semx_helm* helms, semx_batch* batch) {
   if (count < 1 || !helms || !batch) return SEMX_E_ARG;
   *batch = nullptr;
@@ -4146,12 +4363,15 @@ int semx_batch_create(int count, const semx_helm* helms, semx_batch* batch) {
   st = dev_upload(&b->inst, inst.data(), inst.size());
   if (st) { batch_free(b); return st; }
   b->hinst = inst;
-  std::vector<double> cost(count);
-  for (int i = 0; i < count; ++i) {
-    const Helm& H = helms[i]->H;
-    cost[i] = (double)H.npts * std::sqrt((double)H.M->nel) * H.M->np;
+  st = batch_chip_setup(b);
+  if (!st && !b->chip) {
+    std::vector<double> cost(count);
+    for (int i = 0; i < count; ++i) {
+      const Helm& H = helms[i]->H;
+      cost[i] = (double)H.npts * std::sqrt((double)H.M->nel) * H.M->np;
+    }
+    st = batch_layout(b, cost);
   }
-  st = batch_layout(b, cost);
   if (!st && !b->err) st = dev_upload<int>(&b->err, nullptr, 1);
   if (st) { batch_free(b); return st; }
   *batch = b;
@@ -4279,6 +4499,16 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
   if (stream_capturing(s)) b.frozen = true;   // a graph keeps the layout's buffers
   HIPCHK(hipMemcpyAsync(b.ptrs, ptrs.data(), ptrs.size() * sizeof(double*),
                         hipMemcpyHostToDevice, s));
+  if (b.chip) {
+    ChipArgs ca{};
+    ca.inst = b.cinst; ca.order = b.order; ca.ticket = b.ticket;
+    ca.exch = b.exch; ca.red = b.red; ca.iters = b.iters; ca.err = b.err;
+    ca.count = b.count; ca.tol = tol_rel; ca.inner_tol = b.inner_tol;
+    ca.step_max = step_max; ca.max_outer = b.max_outer;
+    ca.bf = b.ptrs; ca.bbc = b.ptrs + b.count; ca.bu = (double* const*)(b.ptrs + 2 * b.count);
+    if (const int st = chip_launch(ca, b.prec != SEMX_PCG_FP64, b.nwg, b.lds, b.nexch, b.nred, s))
+      return st;
+  }
   PcgBatchArgs a;
   a.wmap = b.wmap; a.pctr = b.pctr; a.pslot = b.pslot; a.err = b.err;
   a.inst = b.inst; a.f = b.ptrs; a.bc = b.ptrs + b.count;
@@ -4290,7 +4520,7 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
   const void* kfn = (const void*)k_pcg_batch<double, false, false>;
   if (b.prec == SEMX_PCG_FP32_REFINED) kfn = (const void*)k_pcg_batch<float, true, false>;
   if (b.prec == SEMX_PCG_BF16_REFINED) kfn = (const void*)k_pcg_batch<float, true, true>;
-  if (b.lds > 64 * 1024)
+  if (b.lds > 64 * 1024 && !b.chip)
     HIPCHK(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.lds));
   if (!b.tuned) {
     const int st = batch_tune(b, f, bc, u, kfn, s);
@@ -4301,7 +4531,7 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
   // the multi-workgroup problems' barrier counters back to zero (a fill
   // kernel: the launch may be captured into a graph); they are resident
   // together only if the kernel takes one CU per workgroup or less
-  if (b.nmulti > 0) {
+  if (b.nmulti > 0 && !b.chip) {
     int cus = 256, dev = 0, per_cu = 0;
     if (hipGetDevice(&dev) == hipSuccess)
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -4311,9 +4541,11 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
     hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((b.nmulti * 16 + 255) / 256)), dim3(256), 0,
                        s, b.pctr, (size_t)b.nmulti * 16);
   }
-  prof_begin(s, &ev);
-  HIPCHK(hipLaunchKernel(kfn, dim3((unsigned)b.nwg), dim3(PCG_THREADS), kargs, b.lds, s));
-  prof_end(s, "k_pcg_batch", ev);
+  if (!b.chip) {
+    prof_begin(s, &ev);
+    HIPCHK(hipLaunchKernel(kfn, dim3((unsigned)b.nwg), dim3(PCG_THREADS), kargs, b.lds, s));
+    prof_end(s, "k_pcg_batch", ev);
+  }
   HIPCHK(hipGetLastError());
   if (iters) {
     std::vector<int> it(b.count);
@@ -4334,6 +4566,11 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
     }
     if (limit) return SEMX_E_MAXITER;
     if (b.frozen) return SEMX_OK;
+    if (b.chip) {
+      std::vector<double> its(b.count);
+      for (int i = 0; i < b.count; ++i) its[i] = std::max(1, std::abs(it[i]));
+      return batch_chip_order(&b, its);
+    }
     std::vector<double> cost(b.count);
     for (int i = 0; i < b.count; ++i)
       cost[i] = (double)b.helms[i]->H.npts * std::max(1, std::abs(it[i]));
