@@ -50,6 +50,13 @@ int helm_solve(Helm& H, double* f, const double* bc, double* u, double tol_rel, 
 int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* bcs,
                       double* const* us, double tol_rel, int step_max, int* iters,
                       hipStream_t s);
+// Element right-hand sides (condensed for the direct modes) into d.Fb and,
+// for PCG planes, d.Fi; and the direct modes' element solutions from d.sol.
+// pFb, pFi, psol: strides between fields.
+int elem_condense(Helm& H, int nf, double* const* fs, const double* const* bcs, double* const* us,
+                  size_t pFb, size_t pFi, size_t psol, hipStream_t s);
+int elem_backsub(Helm& H, int nf, double* const* fs, const double* const* bcs, double* const* us,
+                 size_t pFb, size_t pFi, size_t psol, hipStream_t s);
 // The boundary systems of the direct modes through the elimination tree:
 // condensed right-hand sides d.Fb (pFb doubles per field) to d.sol (psol).
 int tree_solve(Helm& H, int nf, size_t pFb, size_t psol, hipStream_t s);

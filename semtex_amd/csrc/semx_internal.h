@@ -83,12 +83,11 @@ struct ModeSys {
   int nblk = 0;
 };
 
+struct ElemDev;
 struct TreeDev;
 struct ChipDev;
 
 struct HelmDev {
-  double* hbi = nullptr;      // nmodes*nset*next*nint
-  double* hii = nullptr;      // nmodes*nset*nint*nint
   double* Pf = nullptr;       // forward-sweep panels, all modes
   double* Pb = nullptr;       // backward-sweep panels, all modes
   double* Linv = nullptr;     // (U_JJ^T)^-1 blocks, row-major
@@ -112,8 +111,8 @@ struct HelmDev {
   int* err = nullptr;         // 1: a hand-off wait timed out
   // scratch
   double* Fb = nullptr;       // nplanes*nel*next
-  double* Fi = nullptr;       // nplanes*nel*nint
-  double* g = nullptr;        // nz*nzero essential values
+  double* Fi = nullptr;       // nplanes*nel*nint, systems with PCG planes
+  double* g = nullptr;        // nplanes*nzero essential values, likewise
   double* sol = nullptr;      // nplanes*solstride
   int* plane_of = nullptr;    // nplanes -> field plane
   double* hcon = nullptr;     // per mode: lambda2 + betak2 (betak2 with its SVV weight);
@@ -132,6 +131,8 @@ struct HelmDev {
   // PCG workgroup map (4 ints per workgroup: plane slot, part, parts, 0),
   // balanced by the planes' last iteration counts
   int* pwmap = nullptr;
+  // element matrices and groups, boundary-term scratch
+  ElemDev* elem = nullptr;
   // elimination tree: matrices, region tables, per-field scratch
   TreeDev* tree = nullptr;
   // on-chip PCG: tables, exchange slots (null: not built; see chip_tried)
@@ -242,6 +243,12 @@ int mesh_upload(Mesh& M);
 void mesh_release(Mesh& M);
 int helm_upload(Helm& H);
 void helm_release(Helm& H);
+
+// element condensation and recovery on the device (semx_elem.hip): matrices
+// and tables, scratch and element groups for nf fields, and their release
+int elem_upload(Helm& H);
+int elem_scratch(Helm& H, int nf);
+void elem_release(Helm& H);
 
 // elimination tree on the device (semx_tree.hip): tables and matrices, the
 // scratch and launch lists for nf fields, and their release

@@ -1,10 +1,9 @@
 // semx_solve.hip -- CDNA4 (gfx950) kernels and the C ABI of libsemx for
 // semtex's Field::solve (src/field.cpp:509-725) over every plane of a field:
 //
-//   k_ess_gather    essential BC values of every plane   (Field::getEssential)
-//   k_condense[_staged]
-//                   -(M f + H g), interior elimination F_b -= hbi F_i, <h,w>
-//                   (Field::constrain, Element::local2globalSumSC, Natural::sum)
+//   k_ess_gather    essential BC values of PCG planes    (Field::getEssential)
+//   k_lift, k_cond, k_force
+//                   element right-hand sides, interior elimination (semx_elem.hip)
 //   k_assemble      owner-gather of the condensed boundary RHS (buildRHS)
 //   k_band_solve    banded Cholesky triangular solves U^T y = b, U x = y
 //                   (LAPACK dpbtrs): one workgroup per mode, the factor
@@ -14,9 +13,7 @@
 //   k_tree_*        the same systems along the elimination tree (semx_tree.hip),
 //                   the default; the band sweeps above serve their own
 //                   switches and systems a tree does not fit
-//   k_backsub[_staged]
-//                   interior recovery u_i = hii F_i - hbi^T u_b and essential
-//                   re-imposition (Element::global2localSC, Field::setEssential)
+//   k_back          interior recovery and essential re-imposition (semx_elem.hip)
 //   k_pcg           JACPCG, persistent workgroups, one or several per plane
 //                   (FP64, or FP32 / BF16-matrix-core inner PCG with FP64
 //                   refinement)
@@ -39,41 +36,6 @@ using namespace semx;
 
 namespace {
 
-constexpr int ELT_THREADS = 1024;  // element kernels: several elements per block
-
-struct ElemArgs {
-  int np, npnp, next, nint, nel, planeSize, nline, nsolve, nzero, nset;
-  double lambda2, beta;
-  int base;
-  const double* hcon;     // per mode: lambda2 + betak2 (1 with mq)
-  const double* mq;       // cylindrical: per mode and set, the operator's mass
-                          // factors (nmodes*nset*npnp); null: Q4 of the set
-  const double* G;
-  const int* eset;
-  const int* emap;
-  const int* pmap;
-  const int* btog;
-  const int* emask;
-  const double* ops;      // DV DT SDV SDT
-  const int* nat_ptr;
-  const int* nat_b;
-  const int* bside;
-  const double* barea;
-  const double* hbi;
-  const double* hii;
-  const int* plane_of;
-  const int* mode_n;
-  const int* mode_kind;   // per mode: SEMX_DIRECT or SEMX_JACPCG
-  double* Fb;
-  double* Fi;
-  double* g;
-  const double* sol;
-  int solstride;
-  const double* f;
-  const double* bc;
-  double* u;
-};
-
 __global__ void k_ess_gather(const double* __restrict__ bc, const int* __restrict__ ess_src,
                              const int* __restrict__ plane_of, double* __restrict__ g,
                              int nzero, int nline) {
@@ -84,263 +46,11 @@ __global__ void k_ess_gather(const double* __restrict__ bc, const int* __restric
   g[(size_t)p * nzero + m] = bc[(size_t)k * nline + ess_src[m]];
 }
 
-// Elements of one plane per block: CE = blockDim / (np*np) elements, thread
-// t works on element t / npnp, node t % npnp.
-// One chunk of ce elements [e0, min(e0 + ce, e_end)) of plane-list entry p.
-// sHbiT: the mode's hbi staged transposed in LDS ([c][b]), or null to read
-// hbi per element from global memory.  Called uniformly by the block.
-__device__ inline void condense_chunk(const ElemArgs& a, int p, int e0, int e_end,
-                                      const double* sHbiT, double* esh) {
-  const int t = threadIdx.x;
-  const int k = a.plane_of[p];
-  const int np = a.np, npnp = a.npnp, next = a.next, nint = a.nint;
-  const int ce = ELT_THREADS / npnp;
-  const int el = t / npnp, pt = t - el * npnp;
-  const int e = e0 + el;
-  const bool act = el < ce && e < e_end;
-  const int m = k >> 1;
-  const double hcon = a.hcon[m];
-  const bool svv = a.lambda2 > EPSDP;
-  double* sD = esh;                       // npnp
-  double* sT = sD + npnp;                 // npnp
-  double* sU = sT + npnp;                 // ce*npnp
-  double* sR = sU + ce * npnp;
-  double* sS = sR + ce * npnp;
-  double* sF = sS + ce * npnp;
-  __syncthreads();   // the previous chunk's reads of the buffers are done
-  if (t < npnp) {
-    sD[t] = a.ops[(svv ? 2 : 0) * npnp + t];
-    sT[t] = a.ops[(svv ? 3 : 1) * npnp + t];
-  }
-  const int set = act ? a.eset[e] : 0;
-  const double* g = a.G + (size_t)set * G_N * npnp;
-  double F = 0.0;
-  if (act) F = g[G_Q4 * npnp + pt] * a.f[(size_t)k * a.planeSize + (size_t)e * npnp + pt];
-  const int em = act ? a.emask[e] : 0;
-  // -(M f + H g): the lifting H g only on elements with essential nodes
-  if (__syncthreads_or(em)) {
-    const int base = el * npnp;
-    if (act) sU[base + pt] = 0.0;
-    __syncthreads();
-    if (act && em && pt < next) {
-      const int gid = a.btog[e * next + pt];
-      sU[base + a.emap[pt]] =
-          (gid >= a.nsolve) ? a.g[(size_t)p * a.nzero + (gid - a.nsolve)] : 0.0;
-    }
-    __syncthreads();
-    const int i = pt / np, j = pt - (pt / np) * np;
-    if (act) {
-      double r = 0.0, s2 = 0.0;
-      for (int q = 0; q < np; ++q) {
-        r += sU[base + i * np + q] * sT[q * np + j];
-        s2 += sD[i * np + q] * sU[base + q * np + j];
-      }
-      const double q1 = g[G_Q1 * npnp + pt], q2 = g[G_Q2 * npnp + pt], q3 = g[G_Q3 * npnp + pt];
-      sR[base + pt] = q1 * r + q3 * s2;
-      sS[base + pt] = q2 * s2 + q3 * r;
-    }
-    __syncthreads();
-    if (act && em) {
-      const double* q4 = a.mq ? a.mq + ((size_t)m * a.nset + set) * npnp : g + G_Q4 * npnp;
-      double T = q4[pt] * sU[base + pt] * hcon;
-      double s1 = 0.0, s3 = 0.0;
-      for (int q = 0; q < np; ++q) {
-        s1 += sT[i * np + q] * sS[base + q * np + j];
-        s3 += sR[base + i * np + q] * sD[q * np + j];
-      }
-      T += s1;
-      T += s3;
-      F += T;
-    }
-  }
-  // element values in emap order: boundary first, then interior
-  if (act) sF[el * npnp + a.pmap[pt]] = -F;
-  __syncthreads();
-  // interior part out; boundary part condensed: F_b - hbi F_i, plus <h,w>
-  for (int idx = t; idx < ce * npnp; idx += ELT_THREADS) {
-    const int le = idx / npnp, q = idx - le * npnp;
-    const int ee = e0 + le;
-    if (ee >= e_end) continue;
-    const size_t pe = (size_t)p * a.nel + ee;
-    const double* Fe = sF + le * npnp;
-    if (q >= next) {
-      a.Fi[pe * nint + (q - next)] = Fe[q];
-    } else {
-      const int b = q;
-      const double* Fi = Fe + next;
-      double s0 = 0.0, s1 = 0.0;
-      if (a.mode_kind[m] == SEMX_DIRECT) {  // PCG modes keep the raw F_b
-        if (sHbiT) {
-          int c = 0;
-          for (; c + 1 < nint; c += 2) {
-            s0 += sHbiT[c * next + b] * Fi[c];
-            s1 += sHbiT[(c + 1) * next + b] * Fi[c + 1];
-          }
-          if (c < nint) s0 += sHbiT[c * next + b] * Fi[c];
-        } else {
-          const double* hbi = a.hbi + ((size_t)m * a.nset + a.eset[ee]) * next * nint;
-          int c = 0;
-          for (; c + 1 < nint; c += 2) {
-            s0 += hbi[b * nint + c] * Fi[c];
-            s1 += hbi[b * nint + c + 1] * Fi[c + 1];
-          }
-          if (c < nint) s0 += hbi[b * nint + c] * Fi[c];
-        }
-      }
-      double fb = Fe[b] - (s0 + s1);
-      const int nm = np - 1;
-      for (int cc = a.nat_ptr[ee]; cc < a.nat_ptr[ee + 1]; ++cc) {
-        const int bb = a.nat_b[cc];
-        const int side = a.bside[bb];
-        const int ii = (b - side * nm + next) % next;
-        if (ii <= nm) fb += a.bc[(size_t)k * a.nline + bb * np + ii] * a.barea[bb * np + ii];
-      }
-      a.Fb[pe * next + b] = fb;
-    }
-  }
-}
-
-// Elements of one plane per block: ce = blockDim / (np*np) elements, thread
-// t works on element t / npnp, node t % npnp.
-__global__ __launch_bounds__(ELT_THREADS) void k_condense(ElemArgs a) {
-  extern __shared__ double esh[];
-  const int ce = ELT_THREADS / a.npnp;
-  condense_chunk(a, blockIdx.y, blockIdx.x * ce, a.nel, nullptr, esh);
-}
-
 // Synchronisation of one wavefront's LDS traffic.
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Meshes with one geometric set: one block per (mode, group of ge
-// elements), the mode's hbi staged transposed in LDS.  Each wavefront forms
-// the forcing of one (element, plane) at a time in emap order -- mass term,
-// and on elements with essential nodes the lifting -H g by the tensor-
-// product operator in a private LDS slice with wavefront synchronisation
-// only -- and after one block barrier all threads condense the block's
-// elements, both planes: interior part out, F_b - hbi F_i plus the natural
-// boundary terms.
-constexpr int CND_WAVES = ELT_THREADS / 64;
-
-__global__ __launch_bounds__(ELT_THREADS, 8) void k_condense_staged(ElemArgs a,
-                                                                 const int* __restrict__ mode_plane,
-                                                                 int ge) {
-  extern __shared__ double esh[];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int np = a.np, next = a.next, nint = a.nint, npnp = a.npnp;
-  const int m = blockIdx.y;
-  const bool direct = a.mode_kind[m] == SEMX_DIRECT;
-  const double hcon = a.hcon[m];
-  const bool svv = a.lambda2 > EPSDP;
-  double* sHbiT = esh;                          // nint*next, [c][b]
-  double* sD = sHbiT + (size_t)next * nint;     // npnp
-  double* sT = sD + npnp;                       // npnp
-  double* sF = sT + npnp;                       // 2*ge*npnp, [plane][element], emap order
-  double* sW = sF + 2 * (size_t)ge * npnp;      // per wave 3*npnp: U, R, S
-  if (direct) {
-    const double* hbi = a.hbi + (size_t)m * next * nint;
-    for (int i = t; i < next * nint; i += ELT_THREADS) {
-      const int b = i / nint, c = i - (i / nint) * nint;
-      sHbiT[c * next + b] = hbi[i];
-    }
-  }
-  for (int i = t; i < npnp; i += ELT_THREADS) {
-    sD[i] = a.ops[(svv ? 2 : 0) * npnp + i];
-    sT[i] = a.ops[(svv ? 3 : 1) * npnp + i];
-  }
-  __syncthreads();
-  const int e_begin = blockIdx.x * ge, e_end = min(a.nel, e_begin + ge);
-  const int ne = e_end - e_begin;
-  const int p0 = mode_plane[2 * m], p1 = mode_plane[2 * m + 1];
-  const int npl = p1 >= 0 ? 2 : 1;
-  const double* g = a.G;                        // the one geometric set
-  double* sU = sW + (size_t)wave * 3 * npnp;
-  double* sR = sU + npnp;
-  double* sS = sR + npnp;
-  for (int item = wave; item < ne * npl; item += CND_WAVES) {
-    const int pl = item / ne, le = item - pl * ne;
-    const int ee = e_begin + le;
-    const int p = pl ? p1 : p0;
-    const int k = a.plane_of[p];
-    double* Fe = sF + (size_t)(pl * ge + le) * npnp;
-    const bool em = a.emask[ee] != 0;           // uniform over the wavefront
-    if (em) {
-      for (int pt = lane; pt < npnp; pt += 64) sU[pt] = 0.0;
-      wave_sync();
-      for (int pt = lane; pt < next; pt += 64) {
-        const int gid = a.btog[ee * next + pt];
-        sU[a.emap[pt]] = (gid >= a.nsolve) ? a.g[(size_t)p * a.nzero + (gid - a.nsolve)] : 0.0;
-      }
-      wave_sync();
-      for (int pt = lane; pt < npnp; pt += 64) {
-        const int i = pt / np, j = pt - (pt / np) * np;
-        double r = 0.0, s2 = 0.0;
-        for (int q = 0; q < np; ++q) {
-          r += sU[i * np + q] * sT[q * np + j];
-          s2 += sD[i * np + q] * sU[q * np + j];
-        }
-        const double q1 = g[G_Q1 * npnp + pt], q2 = g[G_Q2 * npnp + pt], q3 = g[G_Q3 * npnp + pt];
-        sR[pt] = q1 * r + q3 * s2;
-        sS[pt] = q2 * s2 + q3 * r;
-      }
-      wave_sync();
-    }
-    for (int pt = lane; pt < npnp; pt += 64) {
-      double F = g[G_Q4 * npnp + pt] * a.f[(size_t)k * a.planeSize + (size_t)ee * npnp + pt];
-      if (em) {
-        const int i = pt / np, j = pt - (pt / np) * np;
-        const double* q4 = a.mq ? a.mq + (size_t)m * npnp : g + G_Q4 * npnp;
-        double T = q4[pt] * sU[pt] * hcon;
-        double s1 = 0.0, s3 = 0.0;
-        for (int q = 0; q < np; ++q) {
-          s1 += sT[i * np + q] * sS[q * np + j];
-          s3 += sR[i * np + q] * sD[q * np + j];
-        }
-        T += s1;
-        T += s3;
-        F += T;
-      }
-      Fe[a.pmap[pt]] = -F;
-    }
-    wave_sync();   // this wavefront's slice is free for its next item
-  }
-  __syncthreads();
-  const int nm = np - 1;
-  for (int idx = t; idx < npl * ne * npnp; idx += ELT_THREADS) {
-    const int it = idx / npnp, q = idx - it * npnp;
-    const int pl = it / ne, le = it - pl * ne;
-    const int ee = e_begin + le;
-    const int p = pl ? p1 : p0;
-    const int k = a.plane_of[p];
-    const size_t pe = (size_t)p * a.nel + ee;
-    const double* Fe = sF + (size_t)(pl * ge + le) * npnp;
-    if (q >= next) {
-      a.Fi[pe * nint + (q - next)] = Fe[q];
-    } else {
-      const int b = q;
-      const double* Fi = Fe + next;
-      double s0 = 0.0, s1 = 0.0;
-      if (direct) {   // PCG modes keep the raw F_b
-        int c = 0;
-        for (; c + 1 < nint; c += 2) {
-          s0 += sHbiT[c * next + b] * Fi[c];
-          s1 += sHbiT[(c + 1) * next + b] * Fi[c + 1];
-        }
-        if (c < nint) s0 += sHbiT[c * next + b] * Fi[c];
-      }
-      double fb = Fe[b] - (s0 + s1);
-      for (int cc = a.nat_ptr[ee]; cc < a.nat_ptr[ee + 1]; ++cc) {
-        const int bb = a.nat_b[cc];
-        const int side = a.bside[bb];
-        const int ii = (b - side * nm + next) % next;
-        if (ii <= nm) fb += a.bc[(size_t)k * a.nline + bb * np + ii] * a.barea[bb * np + ii];
-      }
-      a.Fb[pe * next + b] = fb;
-    }
-  }
 }
 
 struct BandArgs {
@@ -1693,137 +1403,6 @@ __global__ __launch_bounds__((coop_bt<NB, NR>())) void k_band_xcoop(CoopArgs a) 
   }
 }
 
-__global__ __launch_bounds__(ELT_THREADS) void k_backsub(ElemArgs a) {
-  extern __shared__ double esh[];
-  const int t = threadIdx.x, p = blockIdx.y;
-  const int k = a.plane_of[p];
-  const int next = a.next, nint = a.nint, npnp = a.npnp;
-  const int ce = ELT_THREADS / npnp;
-  const int m = k >> 1;
-  if (a.mode_kind[m] != SEMX_DIRECT) return;
-  const int n = a.mode_n[m];
-  double* sub = esh;                 // ce*next
-  double* sFi = sub + ce * next;     // ce*nint
-  for (int idx = t; idx < ce * npnp; idx += ELT_THREADS) {
-    const int le = idx / npnp, q = idx - le * npnp;
-    const int ee = blockIdx.x * ce + le;
-    if (ee >= a.nel) continue;
-    const size_t pe = (size_t)p * a.nel + ee;
-    if (q < next) {
-      const int gid = a.btog[ee * next + q];
-      const double ub = (gid < n) ? a.sol[(size_t)p * a.solstride + gid] : 0.0;
-      sub[le * next + q] = ub;
-      a.u[(size_t)k * a.planeSize + (size_t)ee * npnp + a.emap[q]] =
-          (gid < n) ? ub : (gid >= a.nsolve ? a.g[(size_t)p * a.nzero + (gid - a.nsolve)] : 0.0);
-    } else {
-      sFi[le * nint + (q - next)] = a.Fi[pe * nint + (q - next)];
-    }
-  }
-  __syncthreads();
-  for (int idx = t; idx < ce * nint; idx += ELT_THREADS) {
-    const int le = idx / nint, q = idx - le * nint;
-    const int ee = blockIdx.x * ce + le;
-    if (ee >= a.nel) continue;
-    const int set = a.eset[ee];
-    const double* hii = a.hii + ((size_t)m * a.nset + set) * nint * nint;
-    const double* hbi = a.hbi + ((size_t)m * a.nset + set) * next * nint;
-    const double* fi = sFi + le * nint;
-    const double* ub = sub + le * next;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int c = 0;
-    for (; c + 1 < nint; c += 2) {
-      s0 += hii[q * nint + c] * fi[c];
-      s1 += hii[q * nint + c + 1] * fi[c + 1];
-    }
-    if (c < nint) s0 += hii[q * nint + c] * fi[c];
-    for (int b = 0; b + 1 < next; b += 2) {
-      s2 += hbi[b * nint + q] * ub[b];
-      s3 += hbi[(b + 1) * nint + q] * ub[b + 1];
-    }
-    a.u[(size_t)k * a.planeSize + (size_t)ee * npnp + a.emap[next + q]] = (s0 + s1) - (s2 + s3);
-  }
-}
-
-// The same for meshes whose elements share one geometric-factor set: one
-// block per (direct mode, group of ge elements) with the mode's hii (stored
-// transposed) and hbi staged in LDS once.  All of the block's element
-// values, both planes, are gathered in one phase (one round of memory
-// latency), then each thread forms one interior row of one element for
-// both planes, each staged coefficient read serving the two.
-__global__ __launch_bounds__(ELT_THREADS) void k_backsub_staged(ElemArgs a,
-                                                                const int* __restrict__ dmode,
-                                                                const int* __restrict__ mode_plane,
-                                                                int ge) {
-  extern __shared__ double esh[];
-  const int t = threadIdx.x;
-  const int next = a.next, nint = a.nint, npnp = a.npnp;
-  const int m = dmode[blockIdx.y];
-  const int n = a.mode_n[m];
-  double* sHiiT = esh;                  // nint*nint, [c][q] = hii[q][c]
-  double* sHbi = sHiiT + nint * nint;   // next*nint
-  double* sub = sHbi + next * nint;     // 2*ge*next, [plane][element][b]
-  double* sFi = sub + 2 * ge * next;    // 2*ge*nint, [plane][element][c]
-  {
-    const double* hii = a.hii + (size_t)m * nint * nint;
-    const double* hbi = a.hbi + (size_t)m * next * nint;
-    for (int i = t; i < nint * nint; i += ELT_THREADS) {
-      const int q = i / nint, c = i - (i / nint) * nint;
-      sHiiT[c * nint + q] = hii[i];
-    }
-    for (int i = t; i < next * nint; i += ELT_THREADS) sHbi[i] = hbi[i];
-  }
-  const int e_begin = blockIdx.x * ge, e_end = min(a.nel, e_begin + ge);
-  const int ne = e_end - e_begin;
-  const int p0 = mode_plane[2 * m], p1 = mode_plane[2 * m + 1];
-  const int npl = p1 >= 0 ? 2 : 1;
-  for (int idx = t; idx < ne * npnp; idx += ELT_THREADS) {
-    const int le = idx / npnp, q = idx - le * npnp;
-    const int ee = e_begin + le;
-    if (q < next) {
-      const int gid = a.btog[ee * next + q];
-      for (int pl = 0; pl < npl; ++pl) {
-        const int p = pl ? p1 : p0;
-        const int k = a.plane_of[p];
-        const double ub = (gid < n) ? a.sol[(size_t)p * a.solstride + gid] : 0.0;
-        sub[(pl * ge + le) * next + q] = ub;
-        a.u[(size_t)k * a.planeSize + (size_t)ee * npnp + a.emap[q]] =
-            (gid < n) ? ub
-                      : (gid >= a.nsolve ? a.g[(size_t)p * a.nzero + (gid - a.nsolve)] : 0.0);
-      }
-    } else {
-      for (int pl = 0; pl < npl; ++pl) {
-        const int p = pl ? p1 : p0;
-        sFi[(pl * ge + le) * nint + (q - next)] =
-            a.Fi[((size_t)p * a.nel + ee) * nint + (q - next)];
-      }
-    }
-  }
-  __syncthreads();
-  const int k0 = a.plane_of[p0], k1 = npl > 1 ? a.plane_of[p1] : k0;
-  for (int idx = t; idx < ne * nint; idx += ELT_THREADS) {
-    const int le = idx / nint, q = idx - le * nint;
-    const int ee = e_begin + le;
-    const double* fi0 = sFi + le * nint;
-    const double* fi1 = sFi + (ge + le) * nint;
-    const double* ub0 = sub + le * next;
-    const double* ub1 = sub + (ge + le) * next;
-    double s0 = 0.0, s1 = 0.0, t0 = 0.0, t1 = 0.0;
-    for (int c = 0; c < nint; ++c) {
-      const double h = sHiiT[c * nint + q];
-      s0 += h * fi0[c];
-      s1 += h * fi1[c];
-    }
-    for (int b = 0; b < next; ++b) {
-      const double h = sHbi[b * nint + q];
-      t0 += h * ub0[b];
-      t1 += h * ub1[b];
-    }
-    const size_t off = (size_t)ee * npnp + a.emap[next + q];
-    a.u[(size_t)k0 * a.planeSize + off] = s0 - t0;
-    if (npl > 1) a.u[(size_t)k1 * a.planeSize + off] = s1 - t1;
-  }
-}
-
 // ===========================================================================
 // Jacobi-preconditioned CG, persistent workgroups (one per plane, or W
 // sharing a plane, below): semtex's JACPCG branch of Field::solve (src/field.cpp:627-720) with the global
@@ -2956,8 +2535,6 @@ int helm_upload(Helm& H) {
   }
   if ((st = dev_upload(&H.d.hcon, hc.data(), hc.size()))) return st;
   if (!H.mq.empty() && (st = dev_upload(&H.d.mq, H.mq.data(), H.mq.size()))) return st;
-  if ((st = dev_upload(&H.d.hbi, H.hbi.data(), H.hbi.size()))) return st;
-  if ((st = dev_upload(&H.d.hii, H.hii.data(), H.hii.size()))) return st;
   if ((st = dev_upload(&H.d.Pf, H.Pf.data(), H.Pf.size()))) return st;
   if ((st = dev_upload(&H.d.Pb, H.Pb.data(), H.Pb.size()))) return st;
   if ((st = dev_upload(&H.d.dmode, H.dmode.data(), H.dmode.size()))) return st;
@@ -2978,6 +2555,7 @@ int helm_upload(Helm& H) {
     if ((st = dev_upload(&H.d.pcg_plane, H.pcg_plane.data(), H.pcg_plane.size()))) return st;
   }
   if ((st = dev_upload(&H.d.plane_of, H.plane_of.data(), H.plane_of.size()))) return st;
+  if ((st = elem_upload(H))) return st;
   if ((st = tree_upload(H))) return st;
   if ((st = coop_setup(H))) return st;
   if (H.npart > 1) {
@@ -3003,7 +2581,7 @@ int helm_upload(Helm& H) {
 }
 
 void helm_release(Helm& H) {
-  dev_free(H.d.hbi); dev_free(H.d.hii); dev_free(H.d.Pf); dev_free(H.d.Pb);
+  dev_free(H.d.Pf); dev_free(H.d.Pb);
   dev_free(H.d.dmode); dev_free(H.d.mode_plane);
   dev_free(H.d.Linv); dev_free(H.d.LinvT); dev_free(H.d.xrows); dev_free(H.d.mode_n); dev_free(H.d.mode_offH);
   dev_free(H.d.mode_offL); dev_free(H.d.pc); dev_free(H.d.Fb); dev_free(H.d.Fi);
@@ -3015,6 +2593,7 @@ void helm_release(Helm& H) {
   dev_free(H.d.err);
   dev_free(H.d.spk); dev_free(H.d.spk_off); dev_free(H.d.prow); dev_free(H.d.pslot);
   dev_free(H.d.pctr); dev_free(H.d.pslot2); dev_free(H.d.pwmap);
+  elem_release(H);
   tree_release(H);
   if (ChipDev* C = H.d.chip) {
     chip_release(C->plan);
@@ -3031,13 +2610,12 @@ void helm_release(Helm& H) {
 }
 
 int helm_scratch(Helm& H, int nf, hipStream_t s) {
-  if (H.tree.on) {
-    if (nf > H.nf_cap) HIPCHK(hipStreamSynchronize(s));
+  if (nf > H.nf_cap) HIPCHK(hipStreamSynchronize(s));
+  if (H.tree.on)
     if (const int st = tree_scratch(H, nf)) return st;
-  }
+  if (const int st = elem_scratch(H, nf)) return st;
   if (nf <= H.nf_cap) return SEMX_OK;
   Mesh& M = *H.M;
-  HIPCHK(hipStreamSynchronize(s));
   dev_free(H.d.Fb); dev_free(H.d.Fi); dev_free(H.d.g); dev_free(H.d.sol);
   dev_free(H.d.work); dev_free(H.d.iters);
   H.nf_cap = 0;
@@ -3045,8 +2623,10 @@ int helm_scratch(Helm& H, int nf, hipStream_t s) {
   const int nzero = M.nglobal - M.nsolve;
   int st;
   if ((st = dev_upload<double>(&H.d.Fb, nullptr, np_ * M.nel * M.next))) return st;
-  if ((st = dev_upload<double>(&H.d.Fi, nullptr, np_ * M.nel * (M.nint ? M.nint : 1)))) return st;
-  if ((st = dev_upload<double>(&H.d.g, nullptr, np_ * (nzero ? nzero : 1)))) return st;
+  if (!H.pcg_plane.empty()) {
+    if ((st = dev_upload<double>(&H.d.Fi, nullptr, np_ * M.nel * (M.nint ? M.nint : 1)))) return st;
+    if ((st = dev_upload<double>(&H.d.g, nullptr, np_ * (nzero ? nzero : 1)))) return st;
+  }
   if ((st = dev_upload<double>(&H.d.sol, nullptr, np_ * H.solstride))) return st;
   if (!H.pcg_plane.empty()) {
     const size_t npcg = H.pcg_plane.size() * nf;
@@ -3240,7 +2820,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
   const size_t pg = (size_t)H.nplanes * (nzero ? nzero : 1);
   const size_t psol = (size_t)H.nplanes * H.solstride;
   hipEvent_t ev;
-  if (nzero > 0) {
+  if (nzero > 0 && !H.pcg_plane.empty()) {
     dim3 grid((nzero + 255) / 256, H.nplanes);
     for (int i = 0; i < nf; ++i) {
       prof_begin(s, &ev);
@@ -3249,58 +2829,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       prof_end(s, "k_ess_gather", ev);
     }
   }
-  ElemArgs ea;
-  ea.np = M.np; ea.npnp = M.npnp; ea.next = M.next; ea.nint = M.nint; ea.nel = M.nel;
-  ea.planeSize = M.planeSize; ea.nline = nline; ea.nsolve = M.nsolve; ea.nzero = nzero;
-  ea.nset = M.nset; ea.lambda2 = H.lambda2; ea.beta = H.beta; ea.base = H.base;
-  ea.hcon = H.d.hcon;
-  ea.mq = H.d.mq;
-  ea.G = M.d.G; ea.eset = M.d.eset; ea.emap = M.d.emap; ea.pmap = M.d.pmap; ea.btog = M.d.btog;
-  ea.emask = M.d.emask; ea.ops = M.d.ops; ea.nat_ptr = M.d.nat_ptr; ea.nat_b = M.d.nat_b;
-  ea.bside = M.d.bside; ea.barea = M.d.barea; ea.hbi = H.d.hbi; ea.hii = H.d.hii;
-  ea.plane_of = H.d.plane_of; ea.mode_n = H.d.mode_n; ea.mode_kind = H.d.mode_kind;
-  ea.Fb = H.d.Fb; ea.Fi = H.d.Fi;
-  ea.g = H.d.g; ea.sol = H.d.sol; ea.solstride = H.solstride;
-  ea.f = nullptr; ea.bc = nullptr; ea.u = nullptr;
-  // per-field arguments of the element kernels
-  auto field_args = [&](int i) {
-    ElemArgs e = ea;
-    e.f = fs[i]; e.bc = bcs ? bcs[i] : nullptr; e.u = us[i];
-    e.Fb = H.d.Fb + i * pFb; e.Fi = H.d.Fi + i * pFi; e.g = H.d.g + i * pg;
-    e.sol = H.d.sol + i * psol;
-    return e;
-  };
-  const int ce = ELT_THREADS / M.npnp;
-  dim3 eg((M.nel + ce - 1) / ce, H.nplanes);
-  const size_t lds_c = (2 * (size_t)M.npnp + 4 * (size_t)ce * M.npnp) * sizeof(double);
-  const size_t lds_b = (size_t)ce * (M.next + M.nint) * sizeof(double);
-  if (lds_c > 64 * 1024 || lds_b > 64 * 1024) {
-    HIPCHK(hipFuncSetAttribute((const void*)k_condense,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_c));
-    HIPCHK(hipFuncSetAttribute((const void*)k_backsub,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_b));
-  }
-  // staged hbi when every element shares one geometric set; elements per
-  // block: enough blocks for two per CU, at most 2 ce
-  int cge = (M.nel * H.nmodes + 511) / 512;
-  cge = std::max(1, std::min(2 * ce, cge));
-  const size_t lds_cs = ((size_t)M.next * M.nint + 2 * (size_t)M.npnp +
-                         2 * (size_t)cge * M.npnp + 3 * (size_t)CND_WAVES * M.npnp) *
-                        sizeof(double);
-  const bool cstaged = M.nset == 1 && lds_cs <= 160 * 1024;
-  if (cstaged && lds_cs > 64 * 1024)
-    HIPCHK(hipFuncSetAttribute((const void*)k_condense_staged,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_cs));
-  for (int i = 0; i < nf; ++i) {
-    ElemArgs e = field_args(i);
-    prof_begin(s, &ev);
-    if (cstaged)
-      hipLaunchKernelGGL(k_condense_staged, dim3((M.nel + cge - 1) / cge, H.nmodes),
-                         dim3(ELT_THREADS), lds_cs, s, e, H.d.mode_plane, cge);
-    else
-      hipLaunchKernelGGL(k_condense, eg, dim3(ELT_THREADS), lds_c, s, e);
-    prof_end(s, "k_condense", ev);
-  }
+  if ((st = elem_condense(H, nf, fs, bcs, us, pFb, pFi, psol, s))) return st;
   if (!H.dmode.empty() && H.tree.on) {
     if ((st = tree_solve(H, nf, pFb, psol, s))) return st;
     H.band_pick[nf] = 9;
@@ -3617,28 +3146,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       prof_end(s, "k_band_solve", ev);
     }
   }
-  if (!H.dmode.empty()) {
-    // staged operators when every element shares one geometric set
-    // elements per block: enough blocks for two per CU, at most 2 ce
-    int ge = (int)((M.nel * H.dmode.size() + 511) / 512);
-    ge = std::max(1, std::min(2 * ce, ge));
-    const size_t lds_s = ((size_t)M.nint * M.nint + (size_t)M.next * M.nint +
-                          2 * (size_t)ge * (M.next + M.nint)) * sizeof(double);
-    const bool staged = M.nset == 1 && lds_s <= 160 * 1024;
-    if (staged && lds_s > 64 * 1024)
-      HIPCHK(hipFuncSetAttribute((const void*)k_backsub_staged,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_s));
-    for (int i = 0; i < nf; ++i) {
-      ElemArgs e = field_args(i);
-      prof_begin(s, &ev);
-      if (staged)
-        hipLaunchKernelGGL(k_backsub_staged, dim3((M.nel + ge - 1) / ge, H.dmode.size()),
-                           dim3(ELT_THREADS), lds_s, s, e, H.d.dmode, H.d.mode_plane, ge);
-      else
-        hipLaunchKernelGGL(k_backsub, eg, dim3(ELT_THREADS), lds_b, s, e);
-      prof_end(s, "k_backsub", ev);
-    }
-  }
+  if (!H.dmode.empty() && (st = elem_backsub(H, nf, fs, bcs, us, pFb, pFi, psol, s))) return st;
   bool chip = !H.pcg_plane.empty() && H.pcg_prec != SEMX_PCG_BF16_REFINED &&
               !getenv("SEMX_PCG_WG") && !getenv("SEMX_PCG_OP") &&
               !(getenv("SEMX_PCG_CHIP") && atoi(getenv("SEMX_PCG_CHIP")) == 0);
