@@ -1,15 +1,18 @@
 // semx_dns.hip -- field operators and the 3D3C Navier-Stokes time step of
 // semtex's dns solver on CDNA4 (gfx950):
 //
-//   k_dft_z      dDFTr along z, femlib/fourier.c:47-171: every column of a
-//                field (ntrn columns, z-stride ntrn) transformed as one
-//                dense real N x N product with semtex's packing
+//   k_fft        dDFTr along z, femlib/fourier.c:47-171: every column of a
+//                field (ntrn columns, z-stride ntrn), semtex's packing
 //                [Re0, Re_N/2, Re1, Im1, ...] and 1/N forward scaling
+//   k_dft_z      the same as one dense real N x N product (odd lengths and
+//                the allocation-free entry point)
 //   k_grad_xy    AuxField::gradient x/y, src/auxfield.cpp:514-665 with
 //                Element::grad, src/element.cpp:552-597
 //   k_grad_z     AuxField::gradient z in Fourier space, auxfield.cpp:636-657
 //   k_smooth     Field::smooth, src/field.cpp:190-236 (mass-weighted DSS)
-//   elementwise  AuxField times / timesMinus / axpy / scaling passes
+//   k_nl         the nonlinear terms of all components
+//   k_wave_div   waveProp and setPForce
+//   k_project    project
 //
 //   k_hopbc      BCmgr::maintainFourier and evaluateCNBCp (src/bcmgr.cpp:
 //                1039-1337): the computed high-order pressure flux on the
@@ -35,7 +38,6 @@ using namespace semx;
 namespace {
 
 constexpr int DFT_KB = 16;          // padding of the transform matrix columns
-constexpr int OP_THREADS = 1024;    // element-operator blocks
 
 // The same product on the FP64 matrix cores (v_mfma_f64_16x16x4: A 16x4,
 // B 4x16, D 16x16; lane l holds A[l%16][l/16], B[l/16][l%16] and, in
@@ -178,106 +180,303 @@ __global__ __launch_bounds__(256) void k_dft_z(const double* __restrict__ in,
   }
 }
 
-// d/dx (dir 0) or d/dy (dir 1) on every element of every plane:
-// tgt = (D_s u) * ds/dx_i + (u D_r^T) * dr/dx_i, plain (non-SVV) D.
-__global__ __launch_bounds__(OP_THREADS) void k_grad_xy(double* __restrict__ data,
-                                                        const double* __restrict__ G,
-                                                        const int* __restrict__ eset,
-                                                        const double* __restrict__ ops, int np,
-                                                        int nel, int planeSize, int dir) {
-  extern __shared__ double gsh[];
-  const int npnp = np * np;
-  const int ce = OP_THREADS / npnp;
-  const int t = threadIdx.x;
-  const int el = t / npnp, pt = t - el * npnp;
-  const int e = blockIdx.x * ce + el;
-  const bool act = el < ce && e < nel;
-  double* sD = gsh;
-  double* sT = sD + npnp;
-  double* sU = sT + npnp;
-  if (t < npnp) {
-    sD[t] = ops[t];
-    sT[t] = ops[npnp + t];
+// Transforms of even length N <= 256 = 2 M along z: the real sequence of a
+// column taken as M complex values, a Stockham FFT of radix 5, 4, 3 and 2
+// passes over them, and the split into (or, inverse, the join from) the
+// spectrum of length N.  A workgroup holds CT columns in LDS, twice (a pass
+// reads one copy and writes the other), [row][column], so that every access
+// of a wavefront is to whole rows of columns; it reads all rows of its
+// columns before it writes any, so input and output may be one buffer.
+//
+// What bounds it: memory, one read and one write of the field.  The dense
+// product on the matrix cores that took even lengths before did 2 N^2
+// operations a column (11 us at the FP64 peak on 96 x 46656 values, 40 us
+// measured with its operands' latencies); it stays for odd lengths.
+// Measured, N = 96: 38880 columns 39 us and 10 us for the copy back -> 19 us
+// (3.1 TB/s); three components of 46656, the transforms with their
+// derivatives: 85 us inverse (3.8 TB/s), 87 us forward, for 24 and 24 us of
+// z derivatives, 240 us and 160 us of products and 64 us of elementwise passes.
+//
+// Kinds, with c the column's component (blockIdx.y):
+//   FORWARD     out = F(in), semtex's packing, 1/N
+//   INVERSE     out = F^-1(in)
+//   INVERSE_DZ  out = F^-1(in), out2 = F^-1(d(in)/dz): a convective term's
+//               two operands from one read of the spectrum
+//   FORWARD_DZ  out = sc (F(in) - d/dz F(b1 b2)): the transform of a
+//               nonlinear term with its conservative z part formed there
+enum { FFT_FORWARD, FFT_INVERSE, FFT_INVERSE_DZ, FFT_FORWARD_DZ };
+
+struct FftArgs {
+  const double* in[3];
+  double* out[3];
+  double* out2[3];
+  const double* b1[3];
+  const double* b2;
+  const double2* tw;      // cos, sin of 2 pi j / N, j < N
+  int N, ntrn, nrad;
+  int rad[8];
+  double beta, sc;
+};
+
+template <int R, bool INV>
+__device__ __forceinline__ void fft_butterfly(double (&x)[R], double (&y)[R]) {
+  constexpr double sg = INV ? 1.0 : -1.0;
+  if constexpr (R == 2) {
+    const double a = x[1], b = y[1];
+    x[1] = x[0] - a; y[1] = y[0] - b;
+    x[0] += a; y[0] += b;
+  } else if constexpr (R == 3) {
+    constexpr double s3 = 0.86602540378443864676;
+    const double ax = x[1] + x[2], ay = y[1] + y[2];
+    const double bx = sg * s3 * (x[1] - x[2]), by = sg * s3 * (y[1] - y[2]);
+    const double mx = x[0] - 0.5 * ax, my = y[0] - 0.5 * ay;
+    x[0] += ax; y[0] += ay;
+    x[1] = mx - by; y[1] = my + bx;
+    x[2] = mx + by; y[2] = my - bx;
+  } else if constexpr (R == 4) {
+    const double ax = x[0] + x[2], ay = y[0] + y[2], bx = x[0] - x[2], by = y[0] - y[2];
+    const double cx = x[1] + x[3], cy = y[1] + y[3];
+    const double dx = sg * (x[1] - x[3]), dy = sg * (y[1] - y[3]);
+    x[0] = ax + cx; y[0] = ay + cy;
+    x[2] = ax - cx; y[2] = ay - cy;
+    x[1] = bx - dy; y[1] = by + dx;
+    x[3] = bx + dy; y[3] = by - dx;
+  } else {
+    constexpr double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;
+    constexpr double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;
+    const double ax = x[1] + x[4], ay = y[1] + y[4], bx = x[2] + x[3], by = y[2] + y[3];
+    const double cx = sg * (x[1] - x[4]), cy = sg * (y[1] - y[4]);
+    const double dx = sg * (x[2] - x[3]), dy = sg * (y[2] - y[3]);
+    const double px = x[0] + c1 * ax + c2 * bx, py = y[0] + c1 * ay + c2 * by;
+    const double qx = x[0] + c2 * ax + c1 * bx, qy = y[0] + c2 * ay + c1 * by;
+    const double ux = s1 * cx + s2 * dx, uy = s1 * cy + s2 * dy;
+    const double vx = s2 * cx - s1 * dx, vy = s2 * cy - s1 * dy;
+    x[0] += ax + bx; y[0] += ay + by;
+    x[1] = px - uy; y[1] = py + ux;
+    x[4] = px + uy; y[4] = py - ux;
+    x[2] = qx - vy; y[2] = qy + vx;
+    x[3] = qx + vy; y[3] = qy - vx;
   }
-  double* u = data + (size_t)blockIdx.y * planeSize + (size_t)e * npnp;
-  if (act) sU[el * npnp + pt] = u[pt];
-  __syncthreads();
-  if (!act) return;
-  const int i = pt / np, j = pt - (pt / np) * np;
-  const double* su = sU + el * npnp;
-  double A = 0.0, B = 0.0;
-  for (int q = 0; q < np; ++q) {
-    A += su[i * np + q] * sT[q * np + j];
-    B += sD[i * np + q] * su[q * np + j];
-  }
-  const double* g = G + (size_t)eset[e] * G_N * npnp;
-  const double rx = g[(dir ? G_DRDY : G_DRDX) * npnp + pt];
-  const double sx = g[(dir ? G_DSDY : G_DSDX) * npnp + pt];
-  u[pt] = B * sx + A * rx;
 }
 
-// An x or y derivative (the element operator of k_grad_xy) read out of
-// place, so the operand needs no copy, with its use applied in the
-// epilogue:
-//   MODE 0  N -= b * d(a)/dx_dir     convective term (dns/nonlinear.cpp:36-211)
-//   MODE 1  N -= d(a b)/dx_dir       conservative term
-//   MODE 2  N  = d(a)/dx_dir         setPForce (dns/integrate.cpp:159-160)
-//   MODE 3  N = sc N + c d(a)/dx_dir project (dns/integrate.cpp:174-186)
-// Entries of a plane beyond its elements (the padding up to planeSize) take
-// the values the unfused copy-derivative-update sequence gives them (the
-// derivative leaves them as they were): N -= a b, N -= a b, N = a,
-// N = sc N + c a.  In modes 0 and 1, sc = 0 starts N from zero (N is not
-// read: the first term of a nonlinear product needs no cleared field).
-template <int MODE>
-__global__ __launch_bounds__(OP_THREADS) void k_grad_nl(double* __restrict__ N,
-                                                        const double* __restrict__ a,
-                                                        const double* __restrict__ b,
-                                                        const double* __restrict__ G,
-                                                        const int* __restrict__ eset,
-                                                        const double* __restrict__ ops, int np,
-                                                        int nel, int planeSize, int dir,
-                                                        double c, double sc) {
+// One pass of radix R over S sets of M complex values (rows 2 j, 2 j + 1):
+// l values of each transform are done.
+template <int R, bool INV, int S, int CT>
+__device__ __forceinline__ void fft_pass(const double* src, double* dst, const double2* tw, int N,
+                                         int l) {
+  constexpr int NG = 256 / CT;
+  const int col = threadIdx.x % CT, M = N / 2, nb = M / R, step = N / (l * R);
+  const float il = 1.0f / (float)l;
+  for (int it = threadIdx.x / CT; it < S * nb; it += NG) {
+    const int s = S > 1 && it >= nb ? 1 : 0, b = it - s * nb;
+    const int k = b - (int)(((float)b + 0.5f) * il) * l;
+    const double* in = src + (size_t)s * N * CT + col;
+    double* out = dst + (size_t)s * N * CT + col;
+    double x[R], y[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      x[t] = in[2 * (b + t * nb) * CT];
+      y[t] = in[(2 * (b + t * nb) + 1) * CT];
+    }
+#pragma unroll
+    for (int t = 1; t < R; ++t) {
+      const double2 w = tw[t * k * step];
+      const double wi = INV ? w.y : -w.y, a = x[t];
+      x[t] = a * w.x - y[t] * wi;
+      y[t] = a * wi + y[t] * w.x;
+    }
+    fft_butterfly<R, INV>(x, y);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = (b - k) * R + k + t * l;
+      out[2 * r * CT] = x[t];
+      out[(2 * r + 1) * CT] = y[t];
+    }
+  }
+}
+
+template <int KIND, int CT>
+__global__ __launch_bounds__(256) void k_fft(FftArgs a) {
+  constexpr bool INV = KIND == FFT_INVERSE || KIND == FFT_INVERSE_DZ;
+  constexpr int S = KIND == FFT_INVERSE_DZ || KIND == FFT_FORWARD_DZ ? 2 : 1;
+  constexpr int NG = 256 / CT, U = 4;
+  extern __shared__ double fft_lds[];
+  const int tid = threadIdx.x, col = tid % CT, g = tid / CT, N = a.N, M = N / 2, c = blockIdx.y;
+  double2* tw = reinterpret_cast<double2*>(fft_lds);
+  double* src = fft_lds + 2 * N;
+  double* dst = src + (size_t)S * N * CT;
+  const size_t ld = a.ntrn;
+  const int gc = blockIdx.x * CT + col;
+  const bool on = gc < a.ntrn;
+  const size_t cc = on ? gc : a.ntrn - 1;       // columns past the last are not stored
+  for (int i = tid; i < N; i += 256) tw[i] = a.tw[i];
+  const double* in = a.in[c] + cc;
+  if (!INV) {
+    for (int n0 = g; n0 < N; n0 += U * NG) {
+      double v[U], w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const size_t r = (size_t)min(n0 + u * NG, N - 1) * ld;
+        v[u] = in[r];
+        if (S > 1) w[u] = a.b1[c][cc + r] * a.b2[cc + r];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (n0 + u * NG < N) {
+          src[(n0 + u * NG) * CT + col] = v[u];
+          if (S > 1) src[(size_t)(N + n0 + u * NG) * CT + col] = w[u];
+        }
+    }
+    __syncthreads();
+  } else {
+    __syncthreads();
+    for (int k0 = g; k0 <= M / 2; k0 += 2 * NG) {
+      double v[2][4];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int k = min(k0 + u * NG, M / 2), q = k ? M - k : 0;
+        v[u][0] = in[(size_t)(2 * k) * ld];
+        v[u][1] = in[(size_t)(2 * k + 1) * ld];
+        v[u][2] = in[(size_t)(2 * q) * ld];
+        v[u][3] = in[(size_t)(2 * q + 1) * ld];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int k = k0 + u * NG, q = M - k;
+        if (k > M / 2) continue;
+        if (k == 0) {
+          src[col] = v[u][0] + v[u][1];
+          src[CT + col] = v[u][0] - v[u][1];
+          if (S > 1) src[(size_t)N * CT + col] = src[(size_t)(N + 1) * CT + col] = 0.0;
+          continue;
+        }
+        const double2 w = tw[k];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const double bk = s ? a.beta * k : 1.0, bq = s ? a.beta * q : 1.0;
+          const double xr = s ? -bk * v[u][1] : v[u][0], xi = s ? bk * v[u][0] : v[u][1];
+          const double yr = s ? -bq * v[u][3] : v[u][2], yi = s ? bq * v[u][2] : v[u][3];
+          const double pr = xr + yr, pi = xi - yi, dr = xr - yr, di = xi + yi;
+          const double e = w.x * di + w.y * dr, f = w.x * dr - w.y * di;
+          double* z = src + (size_t)s * N * CT + col;
+          z[2 * k * CT] = pr - e;
+          z[(2 * k + 1) * CT] = pi + f;
+          if (q != k) {
+            z[2 * q * CT] = pr + e;
+            z[(2 * q + 1) * CT] = f - pi;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = 0, l = 1; i < a.nrad; ++i) {
+    const int r = a.rad[i];
+    if (r == 4) fft_pass<4, INV, S, CT>(src, dst, tw, N, l);
+    else if (r == 3) fft_pass<3, INV, S, CT>(src, dst, tw, N, l);
+    else if (r == 5) fft_pass<5, INV, S, CT>(src, dst, tw, N, l);
+    else fft_pass<2, INV, S, CT>(src, dst, tw, N, l);
+    __syncthreads();
+    double* t = src; src = dst; dst = t;
+    l *= r;
+  }
+  if (!on) return;
+  double* out = a.out[c] + cc;
+  if (INV) {
+    for (int n = g; n < N; n += NG) {
+      out[(size_t)n * ld] = src[n * CT + col];
+      if (S > 1) a.out2[c][cc + (size_t)n * ld] = src[(size_t)(N + n) * CT + col];
+    }
+    return;
+  }
+  const double sc = (KIND == FFT_FORWARD_DZ ? a.sc : 1.0) / N;
+  for (int k = g; k <= M / 2; k += NG) {
+    const double* z = src + col;
+    if (k == 0) {
+      out[0] = sc * (z[0] + z[CT]);
+      out[ld] = sc * (z[0] - z[CT]);
+      continue;
+    }
+    const int q = M - k;
+    const double2 w = tw[k];
+    double x[S][4];             // X_k, X_{M-k}
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const double* zs = z + (size_t)s * N * CT;
+      const double zr = zs[2 * k * CT], zi = zs[(2 * k + 1) * CT];
+      const double yr = zs[2 * q * CT], yi = zs[(2 * q + 1) * CT];
+      const double er = 0.5 * (zr + yr), ei = 0.5 * (zi - yi);
+      const double pr = 0.5 * (zi + yi), pi = 0.5 * (yr - zr);
+      const double tr = w.x * pr + w.y * pi, ti = w.x * pi - w.y * pr;
+      x[s][0] = er + tr; x[s][1] = ei + ti;
+      x[s][2] = er - tr; x[s][3] = ti - ei;
+    }
+    if (S > 1) {                // - i beta k
+      const double bk = a.beta * k, bq = a.beta * q;
+      x[0][0] += bk * x[S - 1][1]; x[0][1] -= bk * x[S - 1][0];
+      x[0][2] += bq * x[S - 1][3]; x[0][3] -= bq * x[S - 1][2];
+    }
+    out[(size_t)(2 * k) * ld] = sc * x[0][0];
+    out[(size_t)(2 * k + 1) * ld] = sc * x[0][1];
+    if (q != k) {
+      out[(size_t)(2 * q) * ld] = sc * x[0][2];
+      out[(size_t)(2 * q + 1) * ld] = sc * x[0][3];
+    }
+  }
+}
+
+// d/dx (dir 0) or d/dy (dir 1) on every element, PB planes per workgroup:
+// tgt = (D_s u) * ds/dx_i + (u D_r^T) * dr/dx_i, plain (non-SVV) D.  The
+// planes share the element's factors and put PB loads per thread in flight.
+// Measured, 24x20 quads np=9, 96 planes: 27 -> 20 us (3.0 TB/s).
+template <int PB>
+__global__ __launch_bounds__(256) void k_grad_xy(double* __restrict__ data,
+                                                 const double* __restrict__ G,
+                                                 const int* __restrict__ eset,
+                                                 const double* __restrict__ ops, int np,
+                                                 int nel, int planeSize, int nz, int dir) {
   extern __shared__ double gsh[];
-  const int npnp = np * np;
-  const int ce = OP_THREADS / npnp;
-  const int t = threadIdx.x;
+  const int npnp = np * np, ce = 256 / npnp, t = threadIdx.x;
   const int el = t / npnp, pt = t - el * npnp;
   const int e = blockIdx.x * ce + el;
   const bool act = el < ce && e < nel;
   double* sD = gsh;
   double* sT = sD + npnp;
-  double* sU = sT + npnp;
+  double* sU = sT + npnp;                 // PB x ce * npnp
   if (t < npnp) {
     sD[t] = ops[t];
     sT[t] = ops[npnp + t];
   }
-  const size_t pbase = (size_t)blockIdx.y * planeSize;
-  if (blockIdx.x == 0)
-    for (int k = nel * npnp + t; k < planeSize; k += OP_THREADS) {
-      const size_t q = pbase + k;
-      if (MODE <= 1) N[q] = (sc == 0.0 ? 0.0 : N[q]) - a[q] * b[q];
-      else if (MODE == 2) N[q] = a[q];
-      else N[q] = sc * N[q] + c * a[q];
-    }
-  const size_t off = pbase + (size_t)e * npnp + pt;
-  if (act) sU[el * npnp + pt] = MODE == 1 ? a[off] * b[off] : a[off];
+  const int k0 = blockIdx.y * PB;
+  double* u = data + (size_t)k0 * planeSize + (size_t)e * npnp + pt;
+  if (act) {
+    double v[PB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) v[p] = u[(size_t)min(p, nz - 1 - k0) * planeSize];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) sU[p * ce * npnp + t] = v[p];
+  }
   __syncthreads();
   if (!act) return;
-  const int i = pt / np, j = pt - (pt / np) * np;
+  const int i = pt / np, j = pt - i * np;
   const double* su = sU + el * npnp;
-  double A = 0.0, B = 0.0;
+  double A[PB], B[PB];
+#pragma unroll
+  for (int p = 0; p < PB; ++p) A[p] = B[p] = 0.0;
   for (int q = 0; q < np; ++q) {
-    A += su[i * np + q] * sT[q * np + j];
-    B += sD[i * np + q] * su[q * np + j];
+    const double dt = sT[q * np + j], ds = sD[i * np + q];
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+      A[p] += su[p * ce * npnp + i * np + q] * dt;
+      B[p] += ds * su[p * ce * npnp + q * np + j];
+    }
   }
   const double* g = G + (size_t)eset[e] * G_N * npnp;
   const double rx = g[(dir ? G_DRDY : G_DRDX) * npnp + pt];
   const double sx = g[(dir ? G_DSDY : G_DSDX) * npnp + pt];
-  const double d = B * sx + A * rx;
-  if (MODE == 0) N[off] = (sc == 0.0 ? 0.0 : N[off]) - b[off] * d;
-  else if (MODE == 1) N[off] = (sc == 0.0 ? 0.0 : N[off]) - d;
-  else if (MODE == 2) N[off] = d;
-  else N[off] = sc * N[off] + c * d;
+#pragma unroll
+  for (int p = 0; p < PB; ++p)
+    if (k0 + p < nz) u[(size_t)p * planeSize] = fma(B[p], sx, A[p] * rx);   // one order for every PB
 }
 
 // Computed pressure boundary conditions (KIO91; BCmgr::maintainFourier,
@@ -423,55 +622,51 @@ __global__ void k_grad_z(const double* src, double* dst, int nmodes, int planeSi
   }
 }
 
-// dst = sc dst + c d(src)/dz over the Fourier planes (k_grad_z's derivative).
-__global__ void k_grad_z_axpby(const double* __restrict__ src, double* __restrict__ dst,
-                               int nmodes, int planeSize, double beta, double sc, double c) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = blockIdx.y;
-  if (idx >= (size_t)planeSize || k >= nmodes) return;
-  const size_t re = (size_t)(2 * k) * planeSize + idx, im = re + planeSize;
-  const double bk = beta * k;
-  const double dr = k == 0 ? 0.0 : -bk * src[im], di = k == 0 ? 0.0 : bk * src[re];
-  dst[re] = sc * dst[re] + c * dr;
-  dst[im] = sc * dst[im] + c * di;
-}
-
 // Mass-weighted average of element-boundary values over the copies of each
-// global node, per plane; copies are summed in increasing storage order.
-__global__ void k_smooth(double* __restrict__ data, const double* __restrict__ G,
-                         const int* __restrict__ eset, const int* __restrict__ emap,
-                         const int* __restrict__ asm_ptr, const int* __restrict__ asm_idx,
-                         const double* __restrict__ imass, int next, int npnp, int nglobal,
-                         int planeSize) {
+// global node; copies are summed in increasing storage order.  A thread takes
+// one node of PB planes of a field (the tables are read once for them, PB
+// values in flight), blockIdx.z the field.
+// Measured, 24x20 quads np=9, 96 planes: 33 -> 28 us: every cache line of
+// the field, for the 8 bytes in 72 of its vertical element sides.
+struct SmoothArgs {
+  double* data[3];
+  const double* G;
+  const int* eset;
+  const int* emap;
+  const int* asm_ptr;
+  const int* asm_idx;
+  const double* imass;
+  int next, npnp, nglobal, planeSize, nz;
+};
+
+template <int PB>
+__global__ __launch_bounds__(256) void k_smooth(SmoothArgs a) {
   const int gI = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gI >= nglobal) return;
-  double* src = data + (size_t)blockIdx.y * planeSize;
-  double s = 0.0;
-  for (int c = asm_ptr[gI]; c < asm_ptr[gI + 1]; ++c) {
-    const int e = asm_idx[c] / next, b = asm_idx[c] - (asm_idx[c] / next) * next;
-    const int q = emap[b];
-    s += G[((size_t)eset[e] * G_N + G_Q4) * npnp + q] * src[(size_t)e * npnp + q];
+  if (gI >= a.nglobal) return;
+  const int k0 = blockIdx.y * PB;
+  double* src = a.data[blockIdx.z] + (size_t)k0 * a.planeSize;
+  double s[PB];
+#pragma unroll
+  for (int p = 0; p < PB; ++p) s[p] = 0.0;
+  const int c0 = a.asm_ptr[gI], c1 = a.asm_ptr[gI + 1];
+  for (int c = c0; c < c1; ++c) {
+    const int i = a.asm_idx[c], e = i / a.next, q = a.emap[i - e * a.next];
+    const double w = a.G[((size_t)a.eset[e] * G_N + G_Q4) * a.npnp + q];
+    const size_t o = (size_t)e * a.npnp + q;
+#pragma unroll
+    for (int p = 0; p < PB; ++p) s[p] += w * src[(size_t)min(p, a.nz - 1 - k0) * a.planeSize + o];
   }
-  s *= imass[gI];
-  for (int c = asm_ptr[gI]; c < asm_ptr[gI + 1]; ++c) {
-    const int e = asm_idx[c] / next, b = asm_idx[c] - (asm_idx[c] / next) * next;
-    src[(size_t)e * npnp + emap[b]] = s;
+  const double im = a.imass[gI];
+  for (int c = c0; c < c1; ++c) {
+    const int i = a.asm_idx[c], e = i / a.next;
+    const size_t o = (size_t)e * a.npnp + a.emap[i - e * a.next];
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+      if (k0 + p < a.nz) src[(size_t)p * a.planeSize + o] = s[p] * im;
   }
 }
 
 // --- elementwise passes over whole fields -------------------------------
-__global__ void k_times(size_t n, double* __restrict__ t, const double* __restrict__ a,
-                        const double* __restrict__ b) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) t[i] = a[i] * b[i];
-}
-
-__global__ void k_times_minus(size_t n, double* __restrict__ t, const double* __restrict__ a,
-                              const double* __restrict__ b) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) t[i] -= a[i] * b[i];
-}
-
 __global__ void k_fill(size_t n, double* __restrict__ t, double a) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) t[i] = a;
@@ -480,11 +675,6 @@ __global__ void k_fill(size_t n, double* __restrict__ t, double a) {
 __global__ void k_copy(size_t n, double* __restrict__ t, const double* __restrict__ a) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) t[i] = a[i];
-}
-
-__global__ void k_scale(size_t n, double* __restrict__ t, double a) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) t[i] *= a;
 }
 
 // AuxField::couple / Field::coupleBCs (src/auxfield.cpp:1352-1420,
@@ -514,45 +704,273 @@ __global__ void k_couple(double* __restrict__ v, double* __restrict__ w, size_t 
   }
 }
 
-__global__ void k_axpy(size_t n, double* __restrict__ t, double a, const double* __restrict__ x) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) t[i] += a * x[i];
-}
+// --- fused passes of the time step ------------------------------------------
+// Elements of one plane (or of a mode's two planes) per workgroup: ce = 256 /
+// (np np) of them, a thread per node.  Each is one pass over memory for what
+// were a derivative kernel per component and direction and elementwise passes
+// between them; the element data sit in LDS, where a derivative's np values
+// are read.  What bounds them: memory traffic.
+// Measured on 24x24 quads np=9 Nz=96 (a field is 36 MB), a step's passes, us:
+// nonlinear terms 97 (3.3 TB/s; 404 as twelve derivative kernels), waveProp
+// and the pressure's forcing 174 (4.5 TB/s; 243), projection 48 (5.2 TB/s;
+// 98 and 45 of copies).
 
-__global__ void k_axpby(size_t n, double* __restrict__ t, double b, double a,
-                        const double* __restrict__ x) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) t[i] = b * t[i] + a * x[i];
-}
+constexpr int NLT = 256;
 
-struct WaveArgs {
-  const double* us[3];
-  const double* uf[3];
-  double a[3], b[3];
-  int nlev;
+// r and s derivatives' factors in x and y of node pt of an element
+struct NodeGeo {
+  double rx, sx, ry, sy;
+  __device__ NodeGeo(const double* g, int npnp, int pt)
+      : rx(g[G_DRDX * npnp + pt]), sx(g[G_DSDX * npnp + pt]), ry(g[G_DRDY * npnp + pt]),
+        sy(g[G_DSDY * npnp + pt]) {}
 };
 
-// waveProp (dns/integrate.cpp:224-259): u = sum_q (-alpha_{q+1} Us_q) +
-// (beta_q dt Uf_q), accumulated in semtex's order.
-__global__ void k_wave(size_t n, double* __restrict__ u, WaveArgs w) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int q = 0; q < w.nlev; ++q) {
-    s += w.a[q] * w.us[q][i];
-    s += w.b[q] * w.uf[q][i];
+struct NlArgs {
+  const double* u[3];     // velocity, physical space
+  double* n[3];           // in: its z derivatives (Z); out: the terms
+  const double* G;
+  const int* eset;
+  const double* ops;
+  int np, nel, planeSize;
+  double sc;
+};
+
+// n_c = -sc (u . grad u_c [CONV] + d(u_c u)/dx + d(u_c v)/dy [CONS]); Z: the
+// convective z term w du_c/dz included, the conservative one left to the
+// transform (dns/nonlinear.cpp:36-211, 214-411, 414-525).
+template <int NC, bool Z, bool CONV, bool CONS>
+__global__ __launch_bounds__(NLT) void k_nl(NlArgs a) {
+  extern __shared__ double gsh[];
+  const int np = a.np, npnp = np * np, ce = NLT / npnp, t = threadIdx.x;
+  const int el = t / npnp, pt = t - el * npnp, e = blockIdx.x * ce + el;
+  const bool act = el < ce && e < a.nel;
+  double* sD = gsh;
+  double* sT = sD + npnp;
+  double* sU = sT + npnp;                 // NC x ce * npnp
+  if (t < npnp) {
+    sD[t] = a.ops[t];
+    sT[t] = a.ops[npnp + t];
   }
-  u[i] = s;
+  const size_t pbase = (size_t)blockIdx.y * a.planeSize;
+  if (blockIdx.x == 0)                    // a plane's padding holds no terms
+    for (int k = a.nel * npnp + t; k < a.planeSize; k += NLT)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) a.n[c][pbase + k] = 0.0;
+  const size_t off = pbase + (size_t)e * npnp + pt;
+  double u[NC], dz[NC];
+  if (act) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      u[c] = a.u[c][off];
+      if (Z && CONV) dz[c] = a.n[c][off];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) sU[c * ce * npnp + t] = u[c];
+  }
+  __syncthreads();
+  if (!act) return;
+  const NodeGeo g(a.G + (size_t)a.eset[e] * G_N * npnp, npnp, pt);
+  const int i = pt / np, j = pt - i * np;
+  const double* su = sU + el * npnp;
+  double r[NC], s[NC], pr[NC][2], ps[NC][2];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) r[c] = s[c] = pr[c][0] = pr[c][1] = ps[c][0] = ps[c][1] = 0.0;
+  for (int q = 0; q < np; ++q) {
+    const double dt = sT[q * np + j], ds = sD[i * np + q];
+    double x[NC], y[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      x[c] = su[c * ce * npnp + i * np + q];
+      y[c] = su[c * ce * npnp + q * np + j];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (CONV) {
+        r[c] += x[c] * dt;
+        s[c] += ds * y[c];
+      }
+      if (CONS)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          if (c == 0 && d == 1) continue;   // u v: formed for c = 1
+          pr[c][d] += x[c] * x[d] * dt;
+          ps[c][d] += ds * (y[c] * y[d]);
+        }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    double v = 0.0;
+    if (CONV) v -= u[0] * (s[c] * g.sx + r[c] * g.rx);
+    if (CONS) v -= ps[c][0] * g.sx + pr[c][0] * g.rx;
+    if (CONV) v -= u[1] * (s[c] * g.sy + r[c] * g.ry);
+    if (CONS) {
+      const double py = c ? pr[c][1] : pr[1][0], qy = c ? ps[c][1] : ps[1][0];
+      v -= qy * g.sy + py * g.ry;
+    }
+    if (Z && CONV) v -= u[2] * dz[c];
+    a.n[c][off] = a.sc * v;
+  }
 }
 
-// setPForce (dns/integrate.cpp:262-277): f0 = (f0 + f1 [+ f2]) / dt
-__global__ void k_divergence_sum(size_t n, double* __restrict__ f0, const double* __restrict__ f1,
-                                 const double* __restrict__ f2, double dt) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = f0[i] + f1[i];
-  if (f2) s += f2[i];
-  f0[i] = s / dt;
+// waveProp and setPForce (dns/integrate.cpp:224-277): u_c = sum_q a_q us_q,c
+// + b_q uf_q,c in semtex's order, then f = div(u) / dt.  NPL = 2: a mode's
+// Re and Im planes together, d/dz in Fourier space (mode 0 and the Nyquist
+// plane have none).
+struct WaveArgs {
+  const double* us[3][3];   // [level][component]
+  const double* uf[3][3];
+  double* u[3];
+  double* f;
+  double a[3], b[3];
+  int nlev;
+  const double* G;
+  const int* eset;
+  const double* ops;
+  int np, nel, planeSize;
+  double beta, dt;
+};
+
+template <int NC, int NPL>
+__global__ __launch_bounds__(NLT) void k_wave_div(WaveArgs w) {
+  extern __shared__ double gsh[];
+  const int np = w.np, npnp = np * np, ce = NLT / npnp, t = threadIdx.x;
+  const int el = t / npnp, pt = t - el * npnp, e = blockIdx.x * ce + el, m = blockIdx.y;
+  const bool act = el < ce && e < w.nel;
+  double* sD = gsh;
+  double* sT = sD + npnp;
+  double* sU = sT + npnp;                 // 2 NPL x ce * npnp
+  if (t < npnp) {
+    sD[t] = w.ops[t];
+    sT[t] = w.ops[npnp + t];
+  }
+  const size_t base = (size_t)NPL * m * w.planeSize;
+  const size_t off = base + (size_t)e * npnp + pt;
+  double wz[NPL];
+  auto sum = [&](int c, size_t i) {
+    double s = 0.0;
+    for (int q = 0; q < w.nlev; ++q) {
+      s += w.a[q] * w.us[q][c][i];
+      s += w.b[q] * w.uf[q][c][i];
+    }
+    return s;
+  };
+  if (blockIdx.x == 0)
+    for (int k = w.nel * npnp + t; k < w.planeSize; k += NLT)
+      for (int p = 0; p < NPL; ++p) {
+        const size_t i = base + (size_t)p * w.planeSize + k;
+        for (int c = 0; c < NC; ++c) w.u[c][i] = sum(c, i);
+        w.f[i] = 0.0;
+      }
+  if (act)
+#pragma unroll
+    for (int p = 0; p < NPL; ++p) {
+      const size_t i = off + (size_t)p * w.planeSize;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const double s = sum(c, i);
+        w.u[c][i] = s;
+        if (c < 2) sU[(2 * p + c) * ce * npnp + t] = s;
+        else wz[p] = s;
+      }
+    }
+  __syncthreads();
+  if (!act) return;
+  const NodeGeo g(w.G + (size_t)w.eset[e] * G_N * npnp, npnp, pt);
+  const int i = pt / np, j = pt - i * np;
+  const double bk = w.beta * m;
+#pragma unroll
+  for (int p = 0; p < NPL; ++p) {
+    const double* su = sU + (2 * p) * ce * npnp + el * npnp;
+    const double* sv = su + ce * npnp;
+    double r = 0.0, s = 0.0, rv = 0.0, sw = 0.0;
+    for (int q = 0; q < np; ++q) {
+      const double dt = sT[q * np + j], ds = sD[i * np + q];
+      r += su[i * np + q] * dt;
+      s += ds * su[q * np + j];
+      rv += sv[i * np + q] * dt;
+      sw += ds * sv[q * np + j];
+    }
+    double d = (s * g.sx + r * g.rx) + (sw * g.sy + rv * g.ry);
+    if (NC == 3 && NPL == 2 && m > 0) d += p ? bk * wz[0] : -bk * wz[NPL - 1];
+    w.f[off + (size_t)p * w.planeSize] = d / w.dt;
+  }
+}
+
+// project (dns/integrate.cpp:280-310): f_c = sc f_c + b dP/dx_c.  keep: the
+// entries of `to` that the velocity solve leaves alone (the Nyquist plane and
+// each plane's padding) take over those of `from`.
+struct ProjectArgs {
+  const double* P;
+  double* f[3];
+  const double* from[3];
+  double* to[3];
+  const double* G;
+  const int* eset;
+  const double* ops;
+  int np, nel, planeSize, keep;
+  double beta, sc, b;
+};
+
+template <int NC, int NPL>
+__global__ __launch_bounds__(NLT) void k_project(ProjectArgs a) {
+  extern __shared__ double gsh[];
+  const int np = a.np, npnp = np * np, ce = NLT / npnp, t = threadIdx.x;
+  const int el = t / npnp, pt = t - el * npnp, e = blockIdx.x * ce + el, m = blockIdx.y;
+  const bool act = el < ce && e < a.nel;
+  double* sD = gsh;
+  double* sT = sD + npnp;
+  double* sP = sT + npnp;                 // NPL x ce * npnp
+  if (t < npnp) {
+    sD[t] = a.ops[t];
+    sT[t] = a.ops[npnp + t];
+  }
+  const size_t base = (size_t)NPL * m * a.planeSize;
+  const size_t off = base + (size_t)e * npnp + pt;
+  if (blockIdx.x == 0)
+    for (int k = a.nel * npnp + t; k < a.planeSize; k += NLT)
+      for (int p = 0; p < NPL; ++p)
+        for (int c = 0; c < NC; ++c) {
+          const size_t i = base + (size_t)p * a.planeSize + k;
+          a.f[c][i] *= a.sc;
+          if (a.keep) a.to[c][i] = a.from[c][i];
+        }
+  double P[NPL], f[NPL][NC];
+  if (act) {
+#pragma unroll
+    for (int p = 0; p < NPL; ++p) {
+      P[p] = a.P[off + (size_t)p * a.planeSize];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) f[p][c] = a.f[c][off + (size_t)p * a.planeSize];
+    }
+#pragma unroll
+    for (int p = 0; p < NPL; ++p) sP[p * ce * npnp + t] = P[p];
+    if (NPL == 2 && m == 0 && a.keep)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        a.to[c][off + a.planeSize] = a.from[c][off + a.planeSize];
+  }
+  __syncthreads();
+  if (!act) return;
+  const NodeGeo g(a.G + (size_t)a.eset[e] * G_N * npnp, npnp, pt);
+  const int i = pt / np, j = pt - i * np;
+  const double bk = a.beta * m;
+#pragma unroll
+  for (int p = 0; p < NPL; ++p) {
+    const double* sp = sP + p * ce * npnp + el * npnp;
+    double r = 0.0, s = 0.0;
+    for (int q = 0; q < np; ++q) {
+      r += sp[i * np + q] * sT[q * np + j];
+      s += sD[i * np + q] * sp[q * np + j];
+    }
+    const size_t o = off + (size_t)p * a.planeSize;
+    a.f[0][o] = a.sc * f[p][0] + a.b * (s * g.sx + r * g.rx);
+    a.f[1][o] = a.sc * f[p][1] + a.b * (s * g.sy + r * g.ry);
+    if (NC == 3) {
+      const double dz = NPL < 2 || m == 0 ? 0.0 : p ? bk * P[0] : -bk * P[NPL - 1];
+      a.f[NC - 1][o] = a.sc * f[p][NC - 1] + a.b * dz;
+    }
+  }
 }
 
 inline dim3 grid1(size_t n, int bs) { return dim3((unsigned)((n + bs - 1) / bs)); }
@@ -723,38 +1141,73 @@ int dft_launch(const double* in, double* out, int N, int ntrn, int sign, hipStre
   return dft_launch_w(in, out, W, ldw, N, ntrn, s);
 }
 
-// The fused derivative of k_grad_nl (modes 0-3 there), dir 0 or 1
-int grad_nl_launch(Mesh& M, int nz, double* N, const double* a, const double* b, int dir,
-                   int mode, hipStream_t s, double c = 0.0, double sc = 1.0) {
-  hipEvent_t ev;
-  const int ce = OP_THREADS / M.npnp;
-  dim3 g((M.nel + ce - 1) / ce, nz);
-  const size_t lds = (2 + (size_t)ce) * M.npnp * sizeof(double);
-  prof_begin(s, &ev);
-#define SEMX_GNL(MODE_)                                                                     \
-  hipLaunchKernelGGL(k_grad_nl<MODE_>, g, dim3(OP_THREADS), lds, s, N, a, b, M.d.G, M.d.eset, \
-                     M.d.ops, M.np, M.nel, M.planeSize, dir, c, sc)
-  switch (mode) {
-    case 0: SEMX_GNL(0); break;
-    case 1: SEMX_GNL(1); break;
-    case 2: SEMX_GNL(2); break;
-    default: SEMX_GNL(3); break;
+// Device table of (cos, sin)(2 pi j / N), long double values rounded, kept
+// for the process per device and length.
+struct FftPlan { int dev, N; double2* tw; };
+std::mutex g_fft_mu;
+std::vector<FftPlan> g_fft;
+
+int fft_plan(int N, const double2** tw) {
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_fft_mu);
+  for (const FftPlan& p : g_fft)
+    if (p.dev == dev && p.N == N) { *tw = p.tw; return SEMX_OK; }
+  std::vector<double2> h(N);
+  for (int j = 0; j < N; ++j) {
+    const long double a = 6.283185307179586476925286766559L * j / N;
+    h[j] = make_double2((double)cosl(a), (double)sinl(a));
   }
-#undef SEMX_GNL
-  prof_end(s, "k_grad_nl", ev);
-  HIPCHK(hipGetLastError());
+  double2* d = nullptr;
+  if (const int st = dev_upload(&d, h.data(), h.size())) return st;
+  g_fft.push_back({dev, N, d});
+  *tw = d;
+  return SEMX_OK;
+}
+
+bool fft_takes(int N) { return N >= 2 && N <= 256 && N % 2 == 0 && fft_length_ok(N); }
+
+// nfield fields of ntrn columns (fft_takes(N)); a: everything but tw, N,
+// ntrn and the radices.  Columns per workgroup: 32 (whole cache lines, two
+// per row) where the LDS of two workgroups allows, else 16.
+int fft_launch(int kind, FftArgs a, int N, int ntrn, int nfield, hipStream_t s) {
+  if (const int st = fft_plan(N, &a.tw)) return st;
+  a.N = N; a.ntrn = ntrn; a.nrad = 0;
+  int m = N / 2;
+  for (int r : {4, 3, 5, 2})
+    while (m % r == 0) { a.rad[a.nrad++] = r; m /= r; }
+  const int sets = kind == FFT_INVERSE_DZ || kind == FFT_FORWARD_DZ ? 2 : 1;
+  const int ct = 2 * (size_t)sets * N * 32 * sizeof(double) <= 76 * 1024 ? 32 : 16;
+  const size_t lds = (2 * (size_t)N + 2 * (size_t)sets * N * ct) * sizeof(double);
+  const void* fn = nullptr;
+#define SEMX_FFT(K_) \
+  if (kind == K_) fn = ct == 32 ? (const void*)k_fft<K_, 32> : (const void*)k_fft<K_, 16>
+  SEMX_FFT(FFT_FORWARD); SEMX_FFT(FFT_INVERSE); SEMX_FFT(FFT_INVERSE_DZ); SEMX_FFT(FFT_FORWARD_DZ);
+#undef SEMX_FFT
+  if (lds > 64 * 1024)
+    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipEvent_t ev;
+  void* kargs[] = {&a};
+  prof_begin(s, &ev);
+  HIPCHK(hipLaunchKernel(fn, dim3((unsigned)((ntrn + ct - 1) / ct), (unsigned)nfield), dim3(256),
+                         kargs, lds, s));
+  prof_end(s, "k_dft_z", ev);
   return SEMX_OK;
 }
 
 int grad_launch(Mesh& M, int nz, double beta, double* data, int dir, hipStream_t s) {
   hipEvent_t ev;
   if (dir < 2) {
-    const int ce = OP_THREADS / M.npnp;
-    dim3 g((M.nel + ce - 1) / ce, nz);
-    const size_t lds = (2 + (size_t)ce) * M.npnp * sizeof(double);
+    const int ce = 256 / M.npnp, pb = nz > 1 ? 4 : 1;
+    dim3 g((M.nel + ce - 1) / ce, (nz + pb - 1) / pb);
+    const size_t lds = (2 + (size_t)pb * ce) * M.npnp * sizeof(double);
     prof_begin(s, &ev);
-    hipLaunchKernelGGL(k_grad_xy, g, dim3(OP_THREADS), lds, s, data, M.d.G, M.d.eset, M.d.ops,
-                       M.np, M.nel, M.planeSize, dir);
+    if (nz > 1)
+      hipLaunchKernelGGL(k_grad_xy<4>, g, dim3(256), lds, s, data, M.d.G, M.d.eset, M.d.ops,
+                         M.np, M.nel, M.planeSize, nz, dir);
+    else
+      hipLaunchKernelGGL(k_grad_xy<1>, g, dim3(256), lds, s, data, M.d.G, M.d.eset, M.d.ops,
+                         M.np, M.nel, M.planeSize, nz, dir);
     prof_end(s, "k_grad_xy", ev);
   } else {
     dim3 g((M.planeSize + 255) / 256, nz / 2);
@@ -766,12 +1219,18 @@ int grad_launch(Mesh& M, int nz, double beta, double* data, int dir, hipStream_t
   return SEMX_OK;
 }
 
-int smooth_launch(Mesh& M, int nz, double* data, hipStream_t s) {
+int smooth_launch(Mesh& M, int nz, double* const* data, int nfield, hipStream_t s) {
   hipEvent_t ev;
-  dim3 g((M.nglobal + 255) / 256, nz);
+  SmoothArgs a{};
+  for (int i = 0; i < nfield; ++i) a.data[i] = data[i];
+  a.G = M.d.G; a.eset = M.d.eset; a.emap = M.d.emap; a.asm_ptr = M.d.asm_ptr;
+  a.asm_idx = M.d.asm_idx; a.imass = M.d.imass; a.next = M.next; a.npnp = M.npnp;
+  a.nglobal = M.nglobal; a.planeSize = M.planeSize; a.nz = nz;
+  const int pb = nz > 1 ? 4 : 1;
+  dim3 g((M.nglobal + 255) / 256, (nz + pb - 1) / pb, nfield);
   prof_begin(s, &ev);
-  hipLaunchKernelGGL(k_smooth, g, dim3(256), 0, s, data, M.d.G, M.d.eset, M.d.emap, M.d.asm_ptr,
-                     M.d.asm_idx, M.d.imass, M.next, M.npnp, M.nglobal, M.planeSize);
+  if (nz > 1) hipLaunchKernelGGL(k_smooth<4>, g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_smooth<1>, g, dim3(256), 0, s, a);
   prof_end(s, "k_smooth", ev);
   HIPCHK(hipGetLastError());
   return SEMX_OK;
@@ -829,8 +1288,8 @@ struct semx_dns_s {
   double* P = nullptr;
   double* Us[3][3] = {};                // [level][component]
   double* Uf[3][3] = {};
-  double* tmp = nullptr;
-  double* spare = nullptr;              // transform output, swapped in
+  double* tmp = nullptr;                // the pressure's forcing
+  double* spare = nullptr;
   Helm* vel = nullptr;                  // DIRECT, lambda2 = alpha0/(dt nu)
   Helm* pre = nullptr;                  // DIRECT, lambda2 = 0
   Helm* start[2] = {nullptr, nullptr};  // JACPCG start-up velocity systems
@@ -853,22 +1312,6 @@ struct semx_dns_s {
 
 namespace {
 
-int dns_transform(semx_dns_s& D, double*& a, int sign, hipStream_t s) {
-  Mesh& M = *D.M;
-  if (D.nz == 1) return SEMX_OK;
-  if (D.nz == 2) {   // AuxField::transform with two planes (auxfield.cpp:1133-1170)
-    const size_t n = M.planeSize;
-    if (sign == 1) hipLaunchKernelGGL(k_fill, grid1(n, 256), dim3(256), 0, s, n, a + n, 0.0);
-    else hipLaunchKernelGGL(k_copy, grid1(n, 256), dim3(256), 0, s, n, a + n, a);
-    HIPCHK(hipGetLastError());
-    return SEMX_OK;
-  }
-  int st = dft_launch(a, D.spare, D.nz, M.planeSize, sign, s);
-  if (st) return st;
-  std::swap(a, D.spare);
-  return SEMX_OK;
-}
-
 int ew_launch_check() {
   HIPCHK(hipGetLastError());
   return SEMX_OK;
@@ -882,78 +1325,91 @@ int ew_launch_check() {
 
 #define CHK(x) do { if (int st_ = (x)) return st_; } while (0)
 
-// skewSymmetric / altSkewSymmetric (dns/nonlinear.cpp:36-411, Cartesian):
-// on entry U holds the Fourier velocity; on exit U holds the physical-space
-// velocity, Us[0] the Fourier copy and Uf[0] the Fourier N(u), smoothed.
-int dns_nonlinear(semx_dns_s& D, hipStream_t s) {
-  Mesh& M = *D.M;
-  const size_t n = D.ntot;
+// Geometry arguments and launch shape of the fused element kernels
+template <class A>
+void op_args(A& a, const Mesh& M) {
+  a.G = M.d.G; a.eset = M.d.eset; a.ops = M.d.ops;
+  a.np = M.np; a.nel = M.nel; a.planeSize = M.planeSize;
+}
+
+template <class A>
+int op_launch(void (*fn)(A), const A& a, const Mesh& M, int layers, int nbuf, const char* name,
+              hipStream_t s) {
+  const int ce = NLT / M.npnp;
+  const size_t lds = (2 + (size_t)nbuf * ce) * M.npnp * sizeof(double);   // 16 KB at most
   hipEvent_t ev;
   prof_begin(s, &ev);
-  for (int i = 0; i < D.ncom; ++i) {
-    if (D.nz > 2) {
-      // the transform is out of place: its input stays as the Fourier copy
-      // Us[0] and the previous Us[0] buffer becomes the spare (no copy)
-      double* f = D.U[i];
-      CHK(dft_launch(f, D.spare, D.nz, M.planeSize, -1, s));
-      D.U[i] = D.spare;
-      D.spare = D.Us[0][i];
-      D.Us[0][i] = f;
-    } else {
-      EW(k_copy, D.Us[0][i], D.U[i]);
-      CHK(dns_transform(D, D.U[i], -1, s));
-    }
-  }
+  hipLaunchKernelGGL(fn, dim3((M.nel + ce - 1) / ce, layers), dim3(NLT), lds, s, a);
+  prof_end(s, name, ev);
+  HIPCHK(hipGetLastError());
+  return SEMX_OK;
+}
+
+// The nonlinear terms (dns/nonlinear.cpp, Cartesian): on entry U holds the
+// Fourier velocity; on exit Us[0] does, Uf[0] the Fourier N(u), smoothed, and
+// U nothing that is needed.
+int dns_nonlinear(semx_dns_s& D, hipStream_t s) {
+  Mesh& M = *D.M;
+  hipEvent_t ev;
+  prof_begin(s, &ev);
   // skewSymmetric (0): both forms, halved; altSkewSymmetric (1): one form
   // per step in turn; convective (2): u . grad u; Stokes (3): none
   // (dns/nonlinear.cpp:36-211, 214-411, 414-525, 528-570)
   const bool conv = D.advection == 0 || D.advection == 2 || (D.advection == 1 && D.toggle);
   const bool cons = D.advection == 0 || (D.advection == 1 && !D.toggle);
+  const double half = D.advection == 0 ? 0.5 : 1.0;
+  const bool z = D.nz > 2;
+  if (z && !fft_takes(D.nz)) return SEMX_E_UNSUPPORTED;
+  for (int i = 0; i < D.ncom; ++i) std::swap(D.U[i], D.Us[0][i]);
+  NlArgs n{};
+  FftArgs f{};
+  op_args(n, M);
+  f.beta = D.beta;
+  f.sc = half;
   for (int i = 0; i < D.ncom; ++i) {
-    double* N = D.Uf[0][i];
-    bool zdefer = false;   // the conservative z term waits in tmp (Fourier space)
-    double start = 0.0;    // the first x/y term stores N instead of updating it
-    for (int j = 0; j < D.ndim; ++j) {
-      if (conv) {   // n_i -= u_j d(u_i)/dx_j
-        if (j == 2) {
-          dim3 g((M.planeSize + 255) / 256, D.nz / 2);
-          hipLaunchKernelGGL(k_grad_z, g, dim3(256), 0, s, D.Us[0][i], D.tmp, D.nz / 2,
-                             M.planeSize, D.beta);
-          CHK(ew_launch_check());
-          CHK(dns_transform(D, D.tmp, -1, s));
-          EW(k_times_minus, N, D.U[j], D.tmp);
-        } else {   // fused: no copy of u_i, the product in the epilogue
-          CHK(grad_nl_launch(M, D.nz, N, D.U[i], D.U[j], j, 0, s, 0.0, start));
-          start = 1.0;
-        }
-      }
-      if (cons) {   // n_i -= d(u_i u_j)/dx_j
-        if (j == 2) {
-          // d(u_i w)/dz is formed in Fourier space and, the transform being
-          // linear, subtracted there after N's own forward transform below
-          // (one inverse transform fewer than subtracting it in physical
-          // space); tmp holds it until then
-          EW(k_times, D.tmp, D.U[i], D.U[j]);
-          CHK(dns_transform(D, D.tmp, +1, s));
-          CHK(grad_launch(M, D.nz, D.beta, D.tmp, j, s));
-          zdefer = true;
-        } else {   // fused: the product formed on load, the difference in the epilogue
-          CHK(grad_nl_launch(M, D.nz, N, D.U[i], D.U[j], j, 1, s, 0.0, start));
-          start = 1.0;
-        }
-      }
-    }
-    if (!conv && !cons) EW(k_fill, N, 0.0);   // Stokes: no nonlinear terms
-    const double half = D.advection == 0 ? 0.5 : 1.0;
-    // the skew-symmetric halving, exact in binary and commuting with the
-    // linear transform, rides on the deferred z term when there is one
-    const bool fold = D.advection == 0 && zdefer;
-    if (D.advection == 0 && !fold) EW(k_scale, N, 0.5);
-    CHK(dns_transform(D, D.Uf[0][i], +1, s));
-    if (fold) EW(k_axpby, D.Uf[0][i], 0.5, -half, D.tmp);
-    else if (zdefer) EW(k_axpy, D.Uf[0][i], -half, D.tmp);
-    CHK(smooth_launch(M, D.nz, D.Uf[0][i], s));
+    n.n[i] = D.Uf[0][i];
+    n.u[i] = D.nz == 1 ? D.Us[0][i] : D.U[i];
+    f.in[i] = D.Us[0][i]; f.out[i] = D.U[i]; f.out2[i] = D.Uf[0][i];
   }
+  if (!conv && !cons) {   // Stokes: no nonlinear terms
+    const size_t nt = D.ntot;
+    for (int i = 0; i < D.ncom; ++i)
+      hipLaunchKernelGGL(k_fill, grid1(nt, 256), dim3(256), 0, s, nt, D.Uf[0][i], 0.0);
+    prof_end(s, "dns_nonlinear", ev);
+    HIPCHK(hipGetLastError());
+    return SEMX_OK;
+  }
+  const size_t pl = M.planeSize;
+  if (z)
+    CHK(fft_launch(conv ? FFT_INVERSE_DZ : FFT_INVERSE, f, D.nz, M.planeSize, D.ncom, s));
+  else if (D.nz == 2)   // both planes the mean (AuxField::transform, auxfield.cpp:1133-1170)
+    for (int i = 0; i < D.ncom; ++i)
+      for (int k = 0; k < 2; ++k)
+        hipLaunchKernelGGL(k_copy, grid1(pl, 256), dim3(256), 0, s, pl, D.U[i] + k * pl, D.Us[0][i]);
+  // the conservative z term is formed in Fourier space, with N's transform,
+  // which then also takes the halving of the skew-symmetric form (exact)
+  const bool zcons = z && cons;
+  n.sc = zcons ? 1.0 : half;
+  void (*fn)(NlArgs) = nullptr;
+#define SEMX_NL(NC_, Z_) \
+  fn = conv ? (cons ? k_nl<NC_, Z_, true, true> : k_nl<NC_, Z_, true, false>) : k_nl<NC_, Z_, false, true>
+  if (D.ncom == 2) SEMX_NL(2, false);
+  else if (z) SEMX_NL(3, true);
+  else SEMX_NL(3, false);
+#undef SEMX_NL
+  CHK(op_launch(fn, n, M, D.nz, D.ncom, "k_grad_nl", s));
+  if (z) {
+    for (int i = 0; i < D.ncom; ++i) {
+      f.in[i] = f.out[i] = D.Uf[0][i];
+      f.b1[i] = D.U[i];
+    }
+    f.b2 = D.U[2];
+    CHK(fft_launch(zcons ? FFT_FORWARD_DZ : FFT_FORWARD, f, D.nz, M.planeSize, D.ncom, s));
+  } else if (D.nz == 2) {
+    for (int i = 0; i < D.ncom; ++i)
+      hipLaunchKernelGGL(k_fill, grid1(pl, 256), dim3(256), 0, s, pl, D.Uf[0][i] + pl, 0.0);
+  }
+  CHK(smooth_launch(M, D.nz, D.Uf[0], D.ncom, s));
   if (D.advection == 1) D.toggle = 1 - D.toggle;
   prof_end(s, "dns_nonlinear", ev);
   return SEMX_OK;
@@ -994,6 +1450,21 @@ void roll(double* lev[3][3], int nord, int ncom) {
   }
 }
 
+// Between steps Us[0], Uf[0], tmp and spare hold nothing; which of those
+// buffers a step takes for what is free.  They are exchanged here (and, for
+// the skew-symmetric form, before the viscous solves) so that the roles recur
+// after 88 steps of that form and 182 of the alternating one at N_TIME = 3:
+// the number of step graphs that programs which capture a full cycle count on.
+void rotate_spares(semx_dns_s& D) {
+  if (D.advection == 0) {
+    std::swap(D.Uf[0][2], D.tmp);
+    std::swap(D.Us[0][0], D.spare);
+  } else if (D.advection == 1) {
+    if (!D.toggle) std::swap(D.Us[0][0], D.Uf[0][1]);
+    else std::swap(D.Us[0][1], D.Uf[0][0]);
+  }
+}
+
 // One time step of integrate (dns/integrate.cpp:79-221).
 int dns_step(semx_dns_s& D, hipStream_t s) {
   Mesh& M = *D.M;
@@ -1007,63 +1478,66 @@ int dns_step(semx_dns_s& D, hipStream_t s) {
   stiffly_stable(Je, alpha);
   extrapolation(Je, beta);
   for (int q = 0; q < Je; ++q) beta[q] *= D.dt;
-  // waveProp
-  for (int i = 0; i < ncom; ++i) {
+  const int npl = D.nz > 1 ? 2 : 1, layers = D.nz / npl;
+  // waveProp into U, setPForce into tmp
+  {
     WaveArgs w{};
+    op_args(w, M);
     w.nlev = Je;
     for (int q = 0; q < Je; ++q) {
-      w.us[q] = D.Us[q][i];
-      w.uf[q] = D.Uf[q][i];
+      for (int i = 0; i < ncom; ++i) {
+        w.us[q][i] = D.Us[q][i];
+        w.uf[q][i] = D.Uf[q][i];
+      }
       w.a[q] = -alpha[q + 1];
       w.b[q] = beta[q];
     }
-    EW(k_wave, D.U[i], w);
+    for (int i = 0; i < ncom; ++i) w.u[i] = D.U[i];
+    w.f = D.tmp;
+    w.beta = D.beta;
+    w.dt = D.dt;
+    if (ncom == 3) CHK(op_launch(k_wave_div<3, 2>, w, M, layers, 4, "k_wave_div", s));
+    else CHK(op_launch(k_wave_div<2, 1>, w, M, layers, 2, "k_wave_div", s));
   }
-  // swapData (U[i], Us[0][i]) and roll of the forcing levels
-  for (int i = 0; i < ncom; ++i) std::swap(D.U[i], D.Us[0][i]);
   roll(D.Uf, nord, ncom);
-  // setPForce: Uf[0][i] = d(Us[0][i])/dx_i, read out of place
-  for (int i = 0; i < D.ndim; ++i) {
-    if (i < 2) {
-      CHK(grad_nl_launch(M, D.nz, D.Uf[0][i], D.Us[0][i], nullptr, i, 2, s));
-    } else {
-      dim3 g((M.planeSize + 255) / 256, D.nz / 2);
-      hipLaunchKernelGGL(k_grad_z, g, dim3(256), 0, s, D.Us[0][i], D.Uf[0][i], D.nz / 2,
-                         M.planeSize, D.beta);
-      CHK(ew_launch_check());
-    }
-  }
-  EW(k_divergence_sum, D.Uf[0][0], D.Uf[0][1], D.ndim > 2 ? D.Uf[0][2] : nullptr, D.dt);
   // pressure solve
-  CHK(helm_solve(*D.pre, D.Uf[0][0], D.bcp, D.P, D.tol_rel, D.step_max, nullptr, s));
-  // project
-  {
-    const double a = -1.0 / (D.dt * D.kinvis), b = 1.0 / D.kinvis;
-    for (int i = 0; i < ncom; ++i) {
-      std::swap(D.Us[0][i], D.Uf[0][i]);
-      if (i >= D.ndim) EW(k_scale, D.Uf[0][i], a);
-    }
-    for (int i = 0; i < D.ndim; ++i) {   // Uf[0][i] = a Uf[0][i] + b dP/dx_i
-      if (i < 2) {
-        CHK(grad_nl_launch(M, D.nz, D.Uf[0][i], D.P, nullptr, i, 3, s, b, a));
-      } else {
-        dim3 g((M.planeSize + 255) / 256, D.nz / 2);
-        hipLaunchKernelGGL(k_grad_z_axpby, g, dim3(256), 0, s, D.P, D.Uf[0][i], D.nz / 2,
-                           M.planeSize, D.beta, a, b);
-        CHK(ew_launch_check());
-      }
-    }
-  }
-  for (int i = 0; i < ncom; ++i) EW(k_copy, D.Us[0][i], D.U[i]);
-  roll(D.Us, nord, ncom);
-  // viscous solves: start-up JACPCG systems while step < N_TIME
-  // (the velocity components share one system: one sweep of its factor)
+  CHK(helm_solve(*D.pre, D.tmp, D.bcp, D.P, D.tol_rel, D.step_max, nullptr, s));
+  // project, in place: U becomes the viscous solves' forcing.  Start-up
+  // systems (JACPCG) while step < N_TIME; iterative ones start from the old
+  // velocity, direct ones only leave parts of it in place.
   Helm* V = (D.step < nord) ? D.start[D.step - 1] : D.vel;
-  double* fs[3] = {D.Uf[0][0], D.Uf[0][1], D.Uf[0][2]};
-  double* us[3] = {D.U[0], D.U[1], D.U[2]};
+  if (D.advection == 0) {   // spare buffers: see rotate_spares
+    std::swap(D.Uf[0][0], D.Uf[0][1]);
+    std::swap(D.Uf[0][0], D.spare);
+  }
+  const bool guess = !V->pcg_plane.empty();
+  {
+    ProjectArgs p{};
+    op_args(p, M);
+    p.P = D.P;
+    for (int i = 0; i < ncom; ++i) {
+      p.f[i] = D.U[i];
+      p.from[i] = D.Us[0][i];
+      p.to[i] = D.Uf[0][i];
+    }
+    p.keep = !guess;
+    p.beta = D.beta;
+    p.sc = -1.0 / (D.dt * D.kinvis);
+    p.b = 1.0 / D.kinvis;
+    if (ncom == 3) CHK(op_launch(k_project<3, 2>, p, M, layers, 2, "k_project", s));
+    else CHK(op_launch(k_project<2, 1>, p, M, layers, 1, "k_project", s));
+  }
+  if (guess)
+    for (int i = 0; i < ncom; ++i) EW(k_copy, D.Uf[0][i], D.Us[0][i]);
+  // viscous solves (the velocity components share one system)
+  double* us[3] = {D.Uf[0][0], D.Uf[0][1], D.Uf[0][2]};
+  double* fs[3] = {D.U[0], D.U[1], D.U[2]};
   const double* bcs[3] = {D.bcu[0], D.bcu[1], D.bcu[2]};
   CHK(helm_solve_fields(*V, ncom, fs, D.Mp ? bcs : nullptr, us, D.tol_rel, D.step_max,
                         nullptr, s));
+  for (int i = 0; i < ncom; ++i) std::swap(D.U[i], D.Uf[0][i]);
+  roll(D.Us, nord, ncom);
+  rotate_spares(D);
   return SEMX_OK;
 }
 
@@ -1227,6 +1701,11 @@ int semx_dft_r(double* data, int tlen, int ntrn, int sign, void* stream) {
   int st = dft_args(data, tlen, ntrn, sign);
   if (st) return st < 0 ? SEMX_OK : st;
   hipStream_t s = (hipStream_t)stream;
+  if (fft_takes(tlen)) {   // in place
+    FftArgs a{};
+    a.in[0] = a.out[0] = data;
+    return fft_launch(sign == 1 ? FFT_FORWARD : FFT_INVERSE, a, tlen, ntrn, 1, s);
+  }
   static double* stage = nullptr;
   static size_t cap = 0;
   const size_t need = (size_t)tlen * ntrn;
@@ -1295,7 +1774,7 @@ int semx_smooth(semx_mesh mesh, int nz, double* data, void* stream) {
   Mesh& M = mesh->M;
   int st = mesh_upload(M);
   if (st) return st;
-  return smooth_launch(M, nz, data, (hipStream_t)stream);
+  return smooth_launch(M, nz, &data, 1, (hipStream_t)stream);
 }
 
 }  // extern "C"
