@@ -16,6 +16,13 @@
 // kernel it stands in for (k_pcg) reads and writes every vector in global
 // memory each iteration and meets at four grid barriers whose fences write
 // back the L2.
+//
+// Eight wavefronts of 256 registers, not twelve of 168: the iteration of
+// np = 11 in FP64 then spills 23 registers in place of 291, whose traffic was
+// most of its time.  With that and sums by row shifts in place of shuffles
+// (us a solve, before -> after): 32x32 np=11 Nz=128 MIXED 72200 -> 41100; 512
+// mixed 2D problems FP32 refined 25900 -> 15700; 9x6 np=7 one distorted plane
+// 2480 -> 1750; 16x16 np=9 Nz=64 FP32 refined 633 -> 614.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,9 +36,9 @@ namespace semx {
 
 namespace {
 
-constexpr int CT = 768;                 // threads: 12 wavefronts, 170 registers each
+constexpr int CT = 512;                 // threads: 8 wavefronts, 256 registers each
 constexpr int CWV = CT / 64;
-constexpr int CHIP_WMAX = 32;           // workgroups of one problem at most
+constexpr int CHIP_WMAX = 48;           // workgroups of one problem at most
 constexpr int CHIP_NPMIN = 4, CHIP_NPMAX = 12;
 constexpr long CHIP_SPIN = 1L << 22;    // polls before a wait gives up
 constexpr unsigned long long CHIP_SENT = 0x7FF4DEADBEEF0001ull;   // signalling NaN
@@ -101,11 +108,26 @@ struct Wg {
   int* err;
 };
 
-// Sum over the wavefront, then the wavefronts in order.
+// Sum over the wavefront by row shifts and broadcasts (the data-parallel
+// paths: a step costs two moves and an add, where a shuffle through LDS costs
+// its latency), the same bits in all lanes.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
 __device__ inline double wave_add(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off /= 2) v += __shfl_xor(v, off);
-  return v;
+  v = dpp_add<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
 // Sums of (u, v) over every thread of the problem's workgroups, the same
@@ -739,10 +761,13 @@ int chip_plan(Mesh& M, ChipPlan& P, const ChipMesh** dev) {
     int s4[4] = {-1, -1, -1, -1};
     for (int c = c0; c < c1; ++c) {
       s4[c - c0] = M.asm_idx[c];
-      if (shared) pos[M.asm_idx[c]] = nif++;
+      if (shared) pos[M.asm_idx[c]] = 0;
     }
     for (int c = c0; c < c1; ++c) gsrc[M.asm_idx[c]] = make_int4(s4[0], s4[1], s4[2], s4[3]);
   }
+  // in slot order: what a workgroup sends lies together (whole cache lines)
+  for (int& q : pos)
+    if (q == 0) q = nif++;
   std::vector<ushort4> tab((size_t)nel * next);
   std::vector<int2> pub;
   size_t lds = 0;
