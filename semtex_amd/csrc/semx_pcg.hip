@@ -42,7 +42,7 @@ constexpr int CHIP_WMAX = 48;           // workgroups of one problem at most
 constexpr int CHIP_NPMIN = 4, CHIP_NPMAX = 12;
 constexpr long CHIP_SPIN = 1L << 22;    // polls before a wait gives up
 constexpr unsigned long long CHIP_SENT = 0x7FF4DEADBEEF0001ull;   // signalling NaN
-constexpr int CHIP_RED = 4 * CWV + CWV + 8;   // LDS doubles of the sums
+constexpr int CHIP_RED = 4 * CWV + CWV + 8 + CHIP_WMAX;   // LDS doubles of the sums
 
 constexpr int chip_epw(int np) { return 64 / np; }
 constexpr int chip_ldr(int np) { return np | 1; }
@@ -99,8 +99,8 @@ struct Wg {
   double* exch;                // ring of 4 x nif
   double* red;                 // ring of 4 x 3 W
   int nif;
-  const int* rem;
-  const int2* pub;
+  const int* rem;              // LDS
+  const int2* pub;             // LDS
   double* lb;                  // LDS: boundary results (T), received ones, a zero
   double* lb2;                 // LDS: their sums (T)
   const ushort4* tab;          // LDS
@@ -182,6 +182,7 @@ __device__ inline double plane_assemble(Wg& G, double pq) {
   pq = wave_add(pq);
   double* rb = G.rd + 4 * CWV;
   if (lane == 0) rb[wave] = pq;
+  if (tid == 0) lb[G.nslot + G.nrem] = 0;
   ch_barrier_mem();
   double t = 0.0;
 #pragma unroll
@@ -189,33 +190,45 @@ __device__ inline double plane_assemble(Wg& G, double pq) {
   if (G.W > 1) {
     double* ex = G.exch + (size_t)(G.kA & 3) * G.nif;
     double* zx = G.exch + (size_t)((G.kA + 2) & 3) * G.nif;
-    double* out = G.rd + 5 * CWV + 4;
+    double* xs = G.rd + 5 * CWV + 8;
     double* s = G.red + (size_t)(G.kA & 3) * 3 * G.W;
-    if (tid == 0) {
-      ch_st(s + 3 * G.w, t);
-      ch_reset(G.red + (size_t)((G.kA + 2) & 3) * 3 * G.W + 3 * G.w);
-    }
     for (int i = tid; i < G.npub; i += CT) {
       const int2 p = G.pub[i];
       ch_st(ex + p.y, (double)lb[p.x]);
       ch_reset(zx + p.y);
     }
-    for (int i = tid; i < G.nrem; i += CT) lb[G.nslot + i] = (T)ch_take(ex + G.rem[i], G.dead);
-    if (wave == 0) {
-      double a = lane < G.W ? ch_take(s + 3 * lane, G.dead) : 0.0;
-      a = wave_add(a);
-      if (lane == 0) out[0] = a;
+    if (tid == CT - 1) {
+      ch_st(s + 3 * G.w, t);
+      ch_reset(G.red + (size_t)((G.kA + 2) & 3) * 3 * G.W + 3 * G.w);
+    }
+    // received results and the workgroups' partial sums, two per thread asked
+    // for before either is waited for
+    const int n = G.nrem + G.W;
+    for (int i = tid; i < n; i += 2 * CT) {
+      const int k = min(i + CT, n - 1);
+      const double* p = i < G.nrem ? ex + G.rem[i] : s + 3 * (i - G.nrem);
+      const double* q = k < G.nrem ? ex + G.rem[k] : s + 3 * (k - G.nrem);
+      double u = ch_ld(p), v = ch_ld(q);
+      if ((unsigned long long)__double_as_longlong(u) == CHIP_SENT) u = ch_take(p, G.dead);
+      if ((unsigned long long)__double_as_longlong(v) == CHIP_SENT) v = ch_take(q, G.dead);
+      if (i < G.nrem) lb[G.nslot + i] = (T)u;
+      else xs[i - G.nrem] = u;
+      if (k < G.nrem) lb[G.nslot + k] = (T)v;
+      else xs[k - G.nrem] = v;
     }
     __syncthreads();
-    t = out[0];
+    t = wave_add(lane < G.W ? xs[lane] : 0.0);
   }
-  for (int i = tid; i < G.nslot; i += CT) {
-    const ushort4 q = G.tab[i];
-    T v = lb[q.x];
-    if (q.y != 0xFFFF) v += lb[q.y];
-    if (q.z != 0xFFFF) v += lb[q.z];
-    if (q.w != 0xFFFF) v += lb[q.w];
-    lb2[i] = v;
+  // two slots at a time and without conditions, so that their reads are in
+  // flight together: absent terms read the zero, threads past the last slot
+  // sum zeros into the spare one
+  for (int i = tid; i < G.nslot; i += 2 * CT) {
+    const int k = min(i + CT, G.nslot);
+    const ushort4 a = G.tab[i], b = G.tab[k];
+    const T u = lb[a.x], v = lb[b.x], u1 = lb[a.y], v1 = lb[b.y], u2 = lb[a.z], v2 = lb[b.z],
+            u3 = lb[a.w], v3 = lb[b.w];
+    lb2[i] = ((u + u1) + u2) + u3;
+    lb2[k] = ((v + v1) + v2) + v3;
   }
   __syncthreads();
   ++G.kA;
@@ -396,29 +409,36 @@ __device__ inline unsigned fresh(unsigned v) {
 }
 
 // The column's element-boundary entries into / out of their LDS slots: the
-// first and last row of every column, the others of the first and last.
+// first and last row of every column, the others of the first and last.  The
+// slots of the last column ascend and those of the first descend; each has
+// its own branch with constant offsets (a common one with a step of +-1 kept
+// an address register per row, spilled and reloaded one after the other).
 template <typename T, int NP>
 __device__ inline void to_boundary(T* lb, const Place& P, const T (&q)[NP]) {
   constexpr int nm = NP - 1;
-  lb[P.slot0 + P.j] = q[0];
-  lb[P.slot0 + 3 * nm - P.j] = q[nm];
-  if (P.j == 0 || P.j == nm) {
-    T* s = lb + P.slot0 + (P.j ? nm : 4 * nm);
-    const int d = P.j ? 1 : -1;
+  T* s = lb + fresh((unsigned)P.slot0);
+  s[P.j] = q[0];
+  s[3 * nm - P.j] = q[nm];
+  if (P.j == nm) {
 #pragma unroll
-    for (int i = 1; i < nm; ++i) s[d * i] = q[i];
+    for (int i = 1; i < nm; ++i) s[nm + i] = q[i];
+  } else if (P.j == 0) {
+#pragma unroll
+    for (int i = 1; i < nm; ++i) s[4 * nm - i] = q[i];
   }
 }
 template <typename T, int NP>
 __device__ inline void from_boundary(const T* lb, const Place& P, T (&q)[NP]) {
   constexpr int nm = NP - 1;
-  q[0] = lb[P.slot0 + P.j];
-  q[nm] = lb[P.slot0 + 3 * nm - P.j];
-  if (P.j == 0 || P.j == nm) {
-    const T* s = lb + P.slot0 + (P.j ? nm : 4 * nm);
-    const int d = P.j ? 1 : -1;
+  const T* s = lb + fresh((unsigned)P.slot0);
+  q[0] = s[P.j];
+  q[nm] = s[3 * nm - P.j];
+  if (P.j == nm) {
 #pragma unroll
-    for (int i = 1; i < nm; ++i) q[i] = s[d * i];
+    for (int i = 1; i < nm; ++i) q[i] = s[nm + i];
+  } else if (P.j == 0) {
+#pragma unroll
+    for (int i = 1; i < nm; ++i) q[i] = s[4 * nm - i];
   }
 }
 
@@ -693,18 +713,28 @@ __global__ __launch_bounds__(CT) void k_pcg_chip(ChipArgs a) {
   G.nif = M.nif;
   G.exch = a.exch + fld * a.exchF + I.exch;
   G.red = a.red + fld * a.redF + I.red;
-  G.rem = M.rem + pt.rem0;
-  G.pub = M.pub + pt.pub0;
   G.err = a.err;
   const int np = M.np, ldr = chip_ldr(np), epw = chip_epw(np);
   const int ecap = (pt.ne + epw - 1) / epw * epw;
   G.rd = lds;
   double* buf = lds + CHIP_RED;
   G.lb = buf + (size_t)(ecap + 1) * np * ldr;
-  G.lb2 = G.lb + G.nslot + G.nrem;
-  ushort4* tab = reinterpret_cast<ushort4*>(G.lb2 + G.nslot);
+  G.lb2 = G.lb + G.nslot + G.nrem + 1;          // the zero behind
+  ushort4* tab = reinterpret_cast<ushort4*>(G.lb2 + G.nslot + 1);
   G.tab = tab;
-  for (int i = threadIdx.x; i < G.nslot; i += CT) tab[i] = M.tab[(size_t)pt.elo * M.next + i];
+  int2* pub = reinterpret_cast<int2*>(tab + G.nslot + 1);
+  int* rem = reinterpret_cast<int*>(pub + G.npub);
+  G.pub = pub;
+  G.rem = rem;
+  for (int i = threadIdx.x; i < G.npub; i += CT) pub[i] = M.pub[pt.pub0 + i];
+  for (int i = threadIdx.x; i < G.nrem; i += CT) rem[i] = M.rem[pt.rem0 + i];
+  const unsigned short zero = (unsigned short)(G.nslot + G.nrem);
+  for (int i = threadIdx.x; i <= G.nslot; i += CT) {
+    ushort4 q = ushort4{zero, zero, zero, zero};
+    if (i < G.nslot) q = M.tab[(size_t)pt.elo * M.next + i];
+    tab[i] = ushort4{q.x, q.y == 0xFFFF ? zero : q.y, q.z == 0xFFFF ? zero : q.z,
+                     q.w == 0xFFFF ? zero : q.w};
+  }
   __syncthreads();
   switch (np) {
 #define CHIP_CASE(N) case N: chip_solve<REFINE, N>(a, I, M, fld, pid, pt, G, buf); break;
@@ -800,7 +830,8 @@ int chip_plan(Mesh& M, ChipPlan& P, const ChipMesh** dev) {
     p.nrem = (int)rem.size() - p.rem0;
     p.npub = (int)pub.size() - p.pub0;
     const size_t ecap = (size_t)(p.ne + epw - 1) / epw * epw;
-    lds = std::max(lds, (CHIP_RED + (ecap + 1) * M.np * ldr + (size_t)ns + p.nrem + ns + ns) * sizeof(double));
+    lds = std::max(lds, (CHIP_RED + (ecap + 1) * M.np * ldr + (size_t)(ns + 1) * 3 + p.nrem + p.npub +
+                         (p.nrem + 1) / 2) * sizeof(double));
   }
   if (lds > 160 * 1024 - 1024) return SEMX_OK;
   // parallelograms: factors proportional to the products of the weights
