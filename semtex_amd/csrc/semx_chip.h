@@ -105,7 +105,8 @@ int chip_workgroups(const Mesh& M);
 // Builds the tables (M on the device); mesh descriptor included in `store`.
 int chip_plan(Mesh& M, ChipPlan& P, const ChipMesh** dev);
 void chip_release(ChipPlan& P);
-int chip_launch(const ChipArgs& a, bool refine, int groups, size_t lds, long long nexch,
+// np: that of every problem, or 0 where they differ (a batch)
+int chip_launch(const ChipArgs& a, int np, bool refine, int groups, size_t lds, long long nexch,
                 long long nred, hipStream_t s);
 
 }  // namespace semx

@@ -17,12 +17,14 @@
 // memory each iteration and meets at four grid barriers whose fences write
 // back the L2.
 //
-// Eight wavefronts of 256 registers, not twelve of 168: the iteration of
-// np = 11 in FP64 then spills 23 registers in place of 291, whose traffic was
-// most of its time.  With that and sums by row shifts in place of shuffles
-// (us a solve, before -> after): 32x32 np=11 Nz=128 MIXED 72200 -> 41100; 512
-// mixed 2D problems FP32 refined 25900 -> 15700; 9x6 np=7 one distorted plane
-// 2480 -> 1750; 16x16 np=9 Nz=64 FP32 refined 633 -> 614.
+// Eight wavefronts of 256 registers, not twelve of 168: those spilled up to
+// 291 registers (np = 11, FP64) inside the iteration, whose traffic was most
+// of its time.  us a solve, twelve wavefronts with shuffle sums -> eight with
+// row shifts -> boundary slots at constant offsets, awaited values two at a
+// time, general factors and preconditioner in registers up to np = 7, one
+// kernel per np: 32x32 np=11 Nz=128 MIXED 72200 -> 40500 -> 32700; 512 mixed
+// 2D problems FP32 refined 25900 -> 15700 -> 12900; 9x6 np=7 one distorted
+// plane 2480 -> 1754 -> 1343; 16x16 np=9 Nz=64 FP32 refined 633 -> 621 -> 550.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,6 +42,7 @@ constexpr int CT = 512;                 // threads: 8 wavefronts, 256 registers 
 constexpr int CWV = CT / 64;
 constexpr int CHIP_WMAX = 48;           // workgroups of one problem at most
 constexpr int CHIP_NPMIN = 4, CHIP_NPMAX = 12;
+constexpr int CHIP_NPREG = 7;         // at 8 they spill
 constexpr long CHIP_SPIN = 1L << 22;    // polls before a wait gives up
 constexpr unsigned long long CHIP_SENT = 0x7FF4DEADBEEF0001ull;   // signalling NaN
 constexpr int CHIP_RED = 4 * CWV + CWV + 8 + CHIP_WMAX;   // LDS doubles of the sums
@@ -255,13 +258,16 @@ __device__ inline int bnode(int b) {   // node i * NP + j of boundary position b
 }
 
 // What a thread needs for its column of one element's operator.
-template <typename T>
+template <typename TT, int NP, bool GREG>
 struct ElemFac {
+  typedef TT T;
+  static constexpr bool greg = GREG;
   bool aff;
   T f1, f2, f3, f4;              // parallelograms: Q1..Q4 = f (this column) x weight (row)
   typename ConstPtr<T>::type w;
   const double* g;               // else the set's factors, and the mass factors
   const double* m;
+  T q[4][GREG ? NP : 1];         // GREG: these in registers, the last times hcon
   T hcon;
   typename ConstPtr<T>::type D, DT;
 };
@@ -304,8 +310,8 @@ __device__ inline void scalar_rows(typename ConstPtr<T>::type A, F fn) {
 // src/element.cpp:1621-1650), columns in registers.  The row products go
 // through the element's LDS tile; the operator matrices come as scalars,
 // one load serving the row and the column product of a step.
-template <typename T, int NP>
-__device__ inline void elem_apply(const ElemFac<T>& F, const T (&p)[NP], T (&out)[NP], T* buf, int j) {
+template <typename T, int NP, class Fac>
+__device__ inline void elem_apply(const Fac& F, const T (&p)[NP], T (&out)[NP], T* buf, int j) {
   constexpr int LD = chip_ldr(NP), NN = NP * NP;
 #pragma unroll
   for (int i = 0; i < NP; ++i) buf[i * LD + j] = p[i];
@@ -334,6 +340,14 @@ __device__ inline void elem_apply(const ElemFac<T>& F, const T (&p)[NP], T (&out
       R[i] = wi * (F.f1 * r + F.f3 * s);
       S[i] = wi * (F.f2 * s + F.f3 * r);
       out[i] = wi * F.f4 * p[i];
+    }
+  } else if constexpr (Fac::greg) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const T r = R[i], s = S[i];
+      R[i] = F.q[0][i] * r + F.q[2][i] * s;
+      S[i] = F.q[1][i] * s + F.q[2][i] * r;
+      out[i] = F.q[3][i] * p[i];
     }
   } else {
     const double *g = F.g + j, *m = F.m + j;
@@ -372,10 +386,10 @@ __device__ inline void elem_apply(const ElemFac<T>& F, const T (&p)[NP], T (&out
 // (the first copy of a node).
 struct Place { int e, el, j, slot0; bool act; unsigned bnd, msk, own; };
 
-template <typename T, int NP>
-__device__ inline ElemFac<T> elem_fac(const ChipMesh& M, const ChipInst& I, const Place& P) {
+template <typename T, int NP, bool GREG>
+__device__ inline ElemFac<T, NP, GREG> elem_fac(const ChipMesh& M, const ChipInst& I, const Place& P) {
   constexpr int NN = NP * NP;
-  ElemFac<T> F;
+  ElemFac<T, NP, GREG> F;
   const int set = M.nset == 1 ? 0 : M.eset[P.e];
   F.g = M.G + (size_t)set * G_N * NN;
   F.m = I.mq ? I.mq + (size_t)set * NN : F.g + G_Q4 * NN;
@@ -387,6 +401,14 @@ __device__ inline ElemFac<T> elem_fac(const ChipMesh& M, const ChipInst& I, cons
     const double wj = M.wq[P.j];
     F.f1 = (T)(c[0] * wj); F.f2 = (T)(c[1] * wj); F.f3 = (T)(c[2] * wj);
     F.f4 = (T)(c[3] * wj * I.hcon);
+  }
+  if constexpr (GREG) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int n = i * NP + P.j;
+      for (int k = 0; k < 3; ++k) F.q[k][i] = (T)F.g[(G_Q1 + k) * NN + n];
+      F.q[3][i] = (T)F.m[n] * F.hcon;
+    }
   }
   const int o = I.svv ? 2 * NN : 0;
   if constexpr (sizeof(T) == 8) {
@@ -445,8 +467,8 @@ __device__ inline void from_boundary(const T* lb, const Place& P, T (&q)[NP]) {
 // q = A p for the thread's column, summed over elements, rows not solved
 // zero; returns p . q over the problem (each element's own part of it, which
 // counts a shared node once).
-template <typename T, int NP>
-__device__ inline double plane_apply(Wg& G, const Place& P, const ElemFac<T>& F, const T (&p)[NP],
+template <typename T, int NP, class Fac>
+__device__ inline double plane_apply(Wg& G, const Place& P, const Fac& F, const T (&p)[NP],
                                      T (&q)[NP], T* buf) {
   elem_apply<T, NP>(F, p, q, buf, P.j);
   double pq = 0.0;
@@ -467,8 +489,8 @@ __device__ inline double plane_apply(Wg& G, const Place& P, const ElemFac<T>& F,
 // PCG iterations on A d = r from d = x, semtex's loop (src/field.cpp:
 // 665-712): pc holds the preconditioner's column in registers, or (null
 // pcr) the thread reads its entries from element-ordered memory.
-template <typename T, int NP, bool PCREG>
-__device__ inline int chip_core(Wg& G, const Place& P, const ElemFac<T>& F, T (&x)[NP], T (&r)[NP],
+template <typename T, int NP, bool PCREG, class Fac>
+__device__ inline int chip_core(Wg& G, const Place& P, const Fac& F, T (&x)[NP], T (&r)[NP],
                                 const T (&pcr)[NP], const double* pcm, double epsb2, int step_max,
                                 T* buf) {
   T p[NP], q[NP];
@@ -518,7 +540,7 @@ __device__ inline int chip_core(Wg& G, const Place& P, const ElemFac<T>& F, T (&
 }
 
 template <bool REFINE, int NP>
-__device__ inline void chip_solve(const ChipArgs& a, const ChipInst& I, const ChipMesh& M, int fld,
+__device__ __forceinline__ void chip_solve(const ChipArgs& a, const ChipInst& I, const ChipMesh& M, int fld,
                                   int pid, const ChipPart& pt, Wg& G, double* bufd) {
   constexpr int NN = NP * NP, NX = 4 * (NP - 1), NI = (NP - 2) * (NP - 2);
   constexpr int EPW = chip_epw(NP), LD = chip_ldr(NP);
@@ -549,7 +571,10 @@ __device__ inline void chip_solve(const ChipArgs& a, const ChipInst& I, const Ch
   // inactive lanes share one more tile, which nobody else reads
   const int ecap = (pt.ne + EPW - 1) / EPW * EPW;
   double* tile = bufd + (size_t)(P.act ? P.el : ecap) * NP * LD;
-  const ElemFac<double> F = elem_fac<double, NP>(M, I, P);
+  // FP64 iterations, small np: general factors and the preconditioner fit in
+  // the registers beside the vectors
+  constexpr bool REGS = !REFINE && NP <= CHIP_NPREG;
+  const auto F = elem_fac<double, NP, REGS>(M, I, P);
   double x[NP], r[NP], q[NP];
   const double* bc = a.bbc ? a.bbc[pid] : nullptr;
   // right-hand side of the element: -(M f + H g) + <h,w>
@@ -635,9 +660,16 @@ __device__ inline void chip_solve(const ChipArgs& a, const ChipInst& I, const Ch
                      : b >= 0 ? I.pc[M.btog[P.e * NX + b]]
                               : I.pc[M.nglobal + P.e * NI + (i - 1) * (NP - 2) + P.j - 1];
       }
-    its = chip_core<double, NP, false>(G, P, F, x, r, q, wk, epsb2, a.step_max, tile);
+    if constexpr (REGS) {
+      double pc[NP];
+#pragma unroll
+      for (int i = 0; i < NP; ++i) pc[i] = P.act ? wk[i * NP] : 0.0;
+      its = chip_core<double, NP, true>(G, P, F, x, r, pc, wk, epsb2, a.step_max, tile);
+    } else {
+      its = chip_core<double, NP, false>(G, P, F, x, r, q, wk, epsb2, a.step_max, tile);
+    }
   } else {
-    const ElemFac<float> Ff = elem_fac<float, NP>(M, I, P);
+    const auto Ff = elem_fac<float, NP, false>(M, I, P);
     float pc[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -692,7 +724,9 @@ __device__ inline void chip_solve(const ChipArgs& a, const ChipInst& I, const Ch
 // makes the order of taking the order of starting, so the problem taken
 // first among the unfinished ones always has all its workgroups running,
 // or the next free ones: the grid drains whatever the dispatch order.
-template <bool REFINE>
+// SNP: the np of every problem (planes of one system: the compiler then
+// allocates the registers for that np alone), or 0 (a batch of any).
+template <bool REFINE, int SNP>
 __global__ __launch_bounds__(CT) void k_pcg_chip(ChipArgs a) {
   extern __shared__ double lds[];
   __shared__ int s_t;
@@ -736,7 +770,10 @@ __global__ __launch_bounds__(CT) void k_pcg_chip(ChipArgs a) {
                      q.w == 0xFFFF ? zero : q.w};
   }
   __syncthreads();
-  switch (np) {
+  if constexpr (SNP > 0) {
+    chip_solve<REFINE, SNP>(a, I, M, fld, pid, pt, G, buf);
+    return;
+  } else switch (np) {
 #define CHIP_CASE(N) case N: chip_solve<REFINE, N>(a, I, M, fld, pid, pt, G, buf); break;
     CHIP_CASE(4) CHIP_CASE(5) CHIP_CASE(6) CHIP_CASE(7) CHIP_CASE(8) CHIP_CASE(9)
     CHIP_CASE(10) CHIP_CASE(11) CHIP_CASE(12)
@@ -907,9 +944,19 @@ void chip_release(ChipPlan& P) {
   P = ChipPlan();
 }
 
-int chip_launch(const ChipArgs& a, bool refine, int groups, size_t lds, long long nexch,
+int chip_launch(const ChipArgs& a, int np, bool refine, int groups, size_t lds, long long nexch,
                 long long nred, hipStream_t s) {
-  const void* fn = refine ? (const void*)k_pcg_chip<true> : (const void*)k_pcg_chip<false>;
+  const void* fn = nullptr;
+  switch (np) {
+#define CHIP_FN(N)                                                                      \
+  case N:                                                                               \
+    fn = refine ? (const void*)k_pcg_chip<true, N> : (const void*)k_pcg_chip<false, N>; \
+    break;
+    CHIP_FN(0) CHIP_FN(4) CHIP_FN(5) CHIP_FN(6) CHIP_FN(7) CHIP_FN(8) CHIP_FN(9) CHIP_FN(10)
+    CHIP_FN(11) CHIP_FN(12)
+#undef CHIP_FN
+    default: return SEMX_E_UNSUPPORTED;
+  }
   HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const long long n = std::max(std::max(nexch, nred), 1LL);
   hipLaunchKernelGGL(k_chip_reset, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.exch,

@@ -3169,7 +3169,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
     ca.Fb = H.d.Fb; ca.Fi = H.d.Fi; ca.g = H.d.g;
     ca.FbF = (long long)pFb; ca.FiF = (long long)pFi; ca.gF = (long long)pg;
     for (int i = 0; i < nf; ++i) ca.u[i] = us[i];
-    if ((st = chip_launch(ca, H.pcg_prec != SEMX_PCG_FP64, npcg * nf * W, C.plan.lds64,
+    if ((st = chip_launch(ca, M.np, H.pcg_prec != SEMX_PCG_FP64, npcg * nf * W, C.plan.lds64,
                           W > 1 ? (long long)npcg * nf * 4 * C.plan.nif : 0,
                           W > 1 ? (long long)npcg * nf * 12 * W : 0, s)))
       return st;
@@ -4014,7 +4014,7 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
     ca.count = b.count; ca.tol = tol_rel; ca.inner_tol = b.inner_tol;
     ca.step_max = step_max; ca.max_outer = b.max_outer;
     ca.bf = b.ptrs; ca.bbc = b.ptrs + b.count; ca.bu = (double* const*)(b.ptrs + 2 * b.count);
-    if (const int st = chip_launch(ca, b.prec != SEMX_PCG_FP64, b.nwg, b.lds, b.nexch, b.nred, s))
+    if (const int st = chip_launch(ca, 0, b.prec != SEMX_PCG_FP64, b.nwg, b.lds, b.nexch, b.nred, s))
       return st;
   }
   PcgBatchArgs a;
