@@ -375,7 +375,8 @@ void tree_plan(Helm& H) {
 
 // ---------------------------------------------------------------------------
 // Dense kernels of the factorisation, row-major, blocked so that the inner
-// loops run along rows (cloned for AVX-512 and AVX2 hosts).
+// loops run along rows (cloned by feature for AVX-512 and FMA hosts: a clone by processor name
+// left every other model on the baseline code).
 // ---------------------------------------------------------------------------
 
 namespace {
@@ -385,7 +386,7 @@ constexpr int FB = 48;    // block size of the triangular steps
 typedef double v8d __attribute__((vector_size(64)));
 
 // C (m x n) -= A (m x k) B (k x n)
-__attribute__((target_clones("arch=skylake-avx512", "arch=haswell", "default")))
+__attribute__((target_clones("avx512f", "fma", "default")))
 void gemm_sub(int m, int n, int k, const double* __restrict__ A, int lda,
               const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc) {
   int i = 0;
@@ -434,7 +435,7 @@ void pack_t(const double* A, int lda, int rows, int cols, double* out) {
 }
 
 // Rows of T (n x w, row stride w) <- L^-1 T, L the n x n lower triangle at A.
-__attribute__((target_clones("arch=skylake-avx512", "arch=haswell", "default")))
+__attribute__((target_clones("avx512f", "fma", "default")))
 void panel_forward(int n, int w, const double* A, int ld, double* T) {
   for (int c0 = 0; c0 < w; c0 += 128) {
     const int m = std::min(128, w - c0);
@@ -489,7 +490,7 @@ int chol_lower(int n, double* A, int ld, std::vector<double>& tmp) {
 constexpr int FC = 64;    // columns per chunk of the triangular solves
 
 // Column chunk T (rows i0..ni of n columns, row stride FC) <- L^-1 T.
-__attribute__((target_clones("arch=skylake-avx512", "arch=haswell", "default")))
+__attribute__((target_clones("avx512f", "fma", "default")))
 void chunk_forward(int ni, int i0, const double* A, int ld, double* T) {
   for (int b0 = i0 / FB * FB; b0 < ni; b0 += FB) {
     const int s = std::max(b0, i0), e = std::min(b0 + FB, ni);
@@ -510,7 +511,7 @@ void chunk_forward(int ni, int i0, const double* A, int ld, double* T) {
 
 // Rows i0..ni of the chunk T <- (L^-T T), rows from the last up; LT: L
 // transposed (row-major, upper triangle).
-__attribute__((target_clones("arch=skylake-avx512", "arch=haswell", "default")))
+__attribute__((target_clones("avx512f", "fma", "default")))
 void chunk_backward(int ni, int i0, const double* LT, double* T) {
   for (int b0 = (ni - 1) / FB * FB; b0 + FB > i0; b0 -= FB) {
     const int s = std::max(b0, i0), e = std::min(b0 + FB, ni);
