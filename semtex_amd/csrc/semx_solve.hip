@@ -2707,6 +2707,16 @@ int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, si
   return SEMX_OK;
 }
 
+// The workgroups of nf fields' planes in the order of C.rank.
+std::vector<int2> chip_order(const ChipDev& C, int npcg, int nf) {
+  std::vector<int2> o;
+  o.reserve((size_t)npcg * nf * C.plan.W);
+  for (int p : C.rank)
+    for (int f = 0; f < nf; ++f)
+      for (int w = 0; w < C.plan.W; ++w) o.push_back(make_int2(f * npcg + p, w));
+  return o;
+}
+
 // The on-chip PCG of a system's planes for nf fields: tables on first use,
 // slots for the largest field count met, and the order the planes are taken
 // in: as listed (low modes, which take the most iterations, first), or by
@@ -2714,9 +2724,8 @@ int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, si
 // stays null where the on-chip iteration does not take the system; its own
 // switches (SEMX_PCG_WG, SEMX_PCG_OP, SEMX_PCG_CHIP=0) and BF16 refinement
 // select k_pcg.
-int chip_prepare(Helm& H, int nfields) {
+int chip_prepare(Helm& H, int nf) {
   Mesh& M = *H.M;
-  int nf = nfields;
   const int npcg = (int)H.pcg_plane.size();
   int st;
   if (!H.d.chip_tried) {
@@ -2761,16 +2770,15 @@ int chip_prepare(Helm& H, int nfields) {
       I.red = (long long)i * 12 * W;
     }
     if ((st = dev_upload(&C->inst, inst.data(), inst.size()))) return st;
+    // the orders of every field count up to this one: a solve of fewer fields
+    // may be captured into a graph without a call of its own before it
+    for (int f = 1; f <= nf; ++f)
+      if (!C->order[f]) {
+        const std::vector<int2> o = chip_order(*C, npcg, f);
+        if ((st = dev_upload(&C->order[f], o.data(), o.size()))) return st;
+      }
     C->nf_cap = nf;
     C->work = H.d.work;
-  }
-  nf = nfields;
-  if (!C->order[nf]) {
-    std::vector<int2> o;
-    for (int p : C->rank)
-      for (int f = 0; f < nf; ++f)
-        for (int w = 0; w < W; ++w) o.push_back(make_int2(f * npcg + p, w));
-    if ((st = dev_upload(&C->order[nf], o.data(), o.size()))) return st;
   }
   int cus = 256, dev = 0;
   if (hipGetDevice(&dev) == hipSuccess)
@@ -2779,10 +2787,12 @@ int chip_prepare(Helm& H, int nfields) {
   return SEMX_OK;
 }
 
-// the planes in decreasing order of their measured iteration counts
-void chip_rank(Helm& H, const std::vector<int>& it, int nf) {
+// The planes in decreasing order of their measured iteration counts, written
+// over the orders in place: the next solve may be captured into a graph, which
+// allows no allocation.  The stream that read the counts back is idle.
+int chip_rank(Helm& H, const std::vector<int>& it, int nf) {
   ChipDev* C = H.d.chip;
-  if (H.pcg_frozen || !C) return;
+  if (H.pcg_frozen || !C) return SEMX_OK;
   const int npcg = (int)H.pcg_plane.size();
   std::vector<int> cnt(npcg, 0), rank(npcg);
   for (int f = 0; f < nf; ++f)
@@ -2791,9 +2801,14 @@ void chip_rank(Helm& H, const std::vector<int>& it, int nf) {
   for (int p = 0; p < npcg; ++p) rank[p] = p;
   std::stable_sort(rank.begin(), rank.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
   C->ranked = true;
-  if (rank == C->rank) return;
+  if (rank == C->rank) return SEMX_OK;
   C->rank = rank;
-  for (int2*& o : C->order) dev_free(o);
+  for (int f = 1; f <= SEMX_MAX_FIELDS; ++f)
+    if (C->order[f]) {
+      const std::vector<int2> o = chip_order(*C, npcg, f);
+      HIPCHK(hipMemcpy(C->order[f], o.data(), o.size() * sizeof(int2), hipMemcpyHostToDevice));
+    }
+  return SEMX_OK;
 }
 
 int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* bcs,
@@ -3186,7 +3201,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
         const int st2 = helm_check(H, s);
         return st2 ? st2 : SEMX_E_MAXITER;
       }
-      chip_rank(H, it, nf);
+      if ((st = chip_rank(H, it, nf))) return st;
     }
   } else if (!H.pcg_plane.empty()) {
     PcgArgs pa;
@@ -3677,6 +3692,7 @@ struct semx_batch_s {
   double* red = nullptr;
   unsigned* ticket = nullptr;
   int2* order = nullptr;
+  std::vector<int> horder;         // the problems in that order
   long long nexch = 0, nred = 0;
 };
 
@@ -3766,9 +3782,16 @@ static int batch_chip_order(semx_batch_s* b, const std::vector<double>& its) {
   std::vector<int2> o;
   for (int i : ord)
     for (int w = 0; w < b->plans[b->helms[i]->H.M].W; ++w) o.push_back(make_int2(i, w));
-  dev_free(b->order);
-  b->nwg = (int)o.size();
-  return dev_upload(&b->order, o.data(), o.size());
+  b->nwg = (int)o.size();               // the same for every order
+  if (!b->order) {
+    b->horder = ord;
+    return dev_upload(&b->order, o.data(), o.size());
+  }
+  if (ord == b->horder) return SEMX_OK;
+  b->horder = ord;
+  // in place: the next solve may be captured into a graph
+  HIPCHK(hipMemcpy(b->order, o.data(), o.size() * sizeof(int2), hipMemcpyHostToDevice));
+  return SEMX_OK;
 }
 
 // Tables of the on-chip iteration for every problem of a batch; b->chip

@@ -1,0 +1,93 @@
+"""Solves captured into a HIP graph right after a solve that changed how the
+next one is launched: a call under capture allocates nothing, so whatever it
+launches from has to be in place by then.  Three replays with eager work
+between them equal the eager solve bit for bit.
+"""
+import numpy as np
+import pytest
+
+import semtex_amd as sx
+from semtex_amd.mesh import rect_mesh
+from semtex_amd.workloads import helmholtz_batch
+
+pytestmark = pytest.mark.gpu
+
+SWITCHES = ("SEMX_AUTOTUNE", "SEMX_BAND_COOP", "SEMX_BAND_XCOOP", "SEMX_BAND_PARTS", "SEMX_TREE",
+            "SEMX_PCG_WG", "SEMX_PCG_OP", "SEMX_PCG_CHIP")
+
+
+@pytest.fixture(autouse=True)
+def default_switches(monkeypatch):
+    for v in SWITCHES:
+        monkeypatch.delenv(v, raising=False)
+
+
+def _case(kx, ky, np_, nz, seeds, quiet=0):
+    """Mesh and per-seed device (f, bc); the first `quiet` planes of f and bc
+    are zero, so that their planes take no iterations."""
+    import torch
+    P = sx.Mesh(np_, rect_mesh(kx, ky, 0, 0.5 * kx, 0, 0.5 * ky, distort=0.1))
+    ins = []
+    for seed in seeds:
+        f, b, _ = helmholtz_batch(P, nz, 2.0, 1.2, seed=seed)
+        f[:quiet], b[:quiet] = 0.0, 0.0
+        ins.append([torch.from_numpy(a.ravel().copy()).to("cuda:0") for a in (f, b)])
+    return P, ins
+
+
+def _capture_and_replay(torch, call, ref):
+    """call(us) captured on its own output buffers, replayed three times."""
+    us = [torch.zeros_like(r) for r in ref]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for u in us:
+            u.zero_()
+        call(us)
+    for _ in range(3):
+        for u in us:
+            u.fill_(1.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(u, r) for u, r in zip(us, ref))
+        vs = [torch.zeros_like(r) for r in ref]
+        call(vs)
+        torch.cuda.synchronize()
+        assert all(torch.equal(v, r) for v, r in zip(vs, ref))
+
+
+@pytest.mark.parametrize("kx,ky", [(4, 3), (17, 9)], ids=["one-workgroup", "several"])
+def test_pcg_captured_after_reranking(cuda, kx, ky):
+    """Iteration counts read back reverse the order the planes are taken in
+    (the low modes, listed first, take none); the next solve is captured."""
+    import torch
+    print(f"[capture] reranked {kx}x{ky}", flush=True)
+    P, [(f, b)] = _case(kx, ky, 6, 16, [1], quiet=8)
+    S = sx.ModalMatrixSys(P, 2.0, 1.2, 0, 8, 16, sx.JACPCG)
+    ref = torch.zeros_like(f)
+    sx.solve(S, f, b, ref)                      # counts read back
+    it = S.plane_iters()
+    assert it[:8].max() == 0 and it[8:].min() > 0
+    _capture_and_replay(torch, lambda u: sx.solve(S, f, b, u[0], iters=False), [ref])
+
+
+def test_batch_reranked_solves_repeat(cuda):
+    """A batch whose measured counts change the order its problems are taken
+    in gives the same bits in every order."""
+    import torch
+    sizes = [(3, 3, 5), (9, 8, 6), (2, 2, 9), (17, 9, 6), (5, 4, 7)]
+    hs, fs, bs, keep = [], [], [], []
+    for i, (kx, ky, np_) in enumerate(sizes):
+        # the largest problems take no iterations
+        P, [(f, b)] = _case(kx, ky, np_, 1, [i], quiet=int(kx > 6))
+        keep.append(P)
+        hs.append(sx.ModalMatrixSys(P, 2.0, 1.2, 0, 1, 1, sx.JACPCG))
+        fs.append(f)
+        bs.append(b)
+    B = sx.Batch(hs)
+    ref = None
+    for r in range(4):
+        us = [torch.zeros_like(f) for f in fs]
+        B.solve(fs, bs, us, iters=r != 2)
+        torch.cuda.synchronize()
+        ref = ref or us
+        assert all(torch.equal(u, v) for u, v in zip(us, ref)), r
