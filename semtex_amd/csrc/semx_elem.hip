@@ -550,21 +550,11 @@ static int end_ld(const Mesh& M) {
   return std::max(M.next + (M.nint + 7) / 8 * 8, (M.npnp + 7) / 8 * 8) | 1;
 }
 
-// Boundary-term scratch for nf fields and the element groups of that field
-// count: two column tiles (32 columns) per workgroup, or one where two would
-// leave fewer than 512 workgroups (two per CU).
-int elem_scratch(Helm& H, int nf) {
-  ElemDev* D = H.d.elem;
-  Mesh& M = *H.M;
-  int st;
-  if (nf > D->nf_cap) {
-    dev_free(D->L);
-    D->nf_cap = 0;
-    if ((st = dev_upload<double>(&D->L, nullptr, (size_t)H.nplanes * nf * D->nbe * M.npnp))) return st;
-    D->nf_cap = nf;
-  }
-  ElemList& l = D->list[nf];
-  if (l.grp || H.dmode.empty()) return SEMX_OK;
+// The element groups of nf fields: two column tiles (32 columns) per
+// workgroup, or one where two would leave fewer than 512 workgroups (two per
+// CU).
+static int elem_list(Helm& H, int nf, ElemList& l) {
+  const Mesh& M = *H.M;
   int npl = 1;
   for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) npl = 2;
   const int nrhs = npl * nf;
@@ -592,8 +582,22 @@ int elem_scratch(Helm& H, int nf) {
   int nmax = 1;
   for (const int4& q : g) nmax = std::max(nmax, q.y * nrhs);
   l.ncol = nmax;                        // np <= 16: at most 32 x 4 KB
-  if ((st = dev_upload(&l.grp, g.data(), g.size()))) return st;
   l.ngrp = (int)g.size();
+  return dev_upload(&l.grp, g.data(), g.size());
+}
+
+// Boundary-term scratch for nf fields and the element groups of every field
+// count up to that (see tree_scratch).
+int elem_scratch(Helm& H, int nf) {
+  ElemDev* D = H.d.elem;
+  int st;
+  if (nf <= D->nf_cap) return SEMX_OK;
+  dev_free(D->L);
+  D->nf_cap = 0;
+  if ((st = dev_upload<double>(&D->L, nullptr, (size_t)H.nplanes * nf * D->nbe * H.M->npnp))) return st;
+  for (int f = 1; f <= nf; ++f)
+    if (!D->list[f].grp && !H.dmode.empty() && (st = elem_list(H, f, D->list[f]))) return st;
+  D->nf_cap = nf;
   return SEMX_OK;
 }
 

@@ -2610,15 +2610,15 @@ void helm_release(Helm& H) {
 }
 
 int helm_scratch(Helm& H, int nf, hipStream_t s) {
-  if (nf > H.nf_cap) HIPCHK(hipStreamSynchronize(s));
+  if (nf <= H.nf_cap) return SEMX_OK;
+  Mesh& M = *H.M;
+  HIPCHK(hipStreamSynchronize(s));
+  H.nf_cap = 0;
   if (H.tree.on)
     if (const int st = tree_scratch(H, nf)) return st;
   if (const int st = elem_scratch(H, nf)) return st;
-  if (nf <= H.nf_cap) return SEMX_OK;
-  Mesh& M = *H.M;
   dev_free(H.d.Fb); dev_free(H.d.Fi); dev_free(H.d.g); dev_free(H.d.sol);
   dev_free(H.d.work); dev_free(H.d.iters);
-  H.nf_cap = 0;
   const size_t np_ = (size_t)H.nplanes * nf;
   const int nzero = M.nglobal - M.nsolve;
   int st;

@@ -30,8 +30,8 @@ typedef double tree_d4 __attribute__((ext_vector_type(4)));
 struct TreeTypeDev { int ni, nb; long long off_f, off_b; };
 struct TreeTask { int node, count, mt, pad; };   // regions of one type, first row tile
 
-struct TreeList {               // launch lists of one direction and stage
-  TreeTask* task = nullptr;
+struct TreeList {               // launch list of one direction and stage
+  size_t first = 0;             // of its tasks
   int ntask = 0, wk = 1, ct = 1, ldn = 16;
   size_t lds = 0;
 };
@@ -48,6 +48,7 @@ struct TreeDev {
   int nf_cap = 0;
   // launch lists per field count: forward stages, then backward stages
   std::vector<TreeList> list[SEMX_MAX_FIELDS + 1];
+  TreeTask* task[SEMX_MAX_FIELDS + 1] = {nullptr};
 };
 
 namespace {
@@ -271,26 +272,11 @@ int tree_upload(Helm& H) {
   return SEMX_OK;
 }
 
-// Contribution scratch for nf fields and the launch lists of that field
-// count: up to TREE_GROUP regions of one type per workgroup, as many as the
-// right-hand-side tile's LDS holds.
-int tree_scratch(Helm& H, int nf) {
-  Tree& T = H.tree;
-  TreeDev* D = H.d.tree;
-  int st;
-  if (nf > D->nf_cap) {
-    dev_free(D->C); dev_free(D->Y);
-    D->nf_cap = 0;
-    const size_t np = (size_t)H.nplanes * nf;
-    if ((st = dev_upload<double>(&D->C, nullptr, np * T.nslot_c))) return st;
-    if ((st = dev_upload<double>(&D->Y, nullptr, np * T.nslot_y))) return st;
-    D->nf_cap = nf;
-  }
-  if (!D->list[nf].empty()) return SEMX_OK;
-  int npl = 1;
-  for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) npl = 2;
-  const int nrhs = npl * nf;
-  std::vector<TreeList> out;
+// Launch lists of nf fields, without their device addresses: up to TREE_GROUP
+// regions of one type per workgroup, as many as the right-hand-side tile's
+// LDS holds.
+static int tree_lists(const Tree& T, int nrhs, std::vector<TreeList>& out,
+                      std::vector<TreeTask>& tasks) {
   for (int dir = 0; dir < 2; ++dir)
     for (int s = 0; s < T.nstage; ++s) {
       TreeList L;
@@ -301,7 +287,7 @@ int tree_scratch(Helm& H, int nf) {
       }
       L.wk = share(Kmax);
       const int wm = TW / L.wk;
-      std::vector<TreeTask> task;
+      const size_t first = tasks.size();
       int nmax = 1, kl = 0;
       for (int i = T.stage_ptr[s]; i < T.stage_ptr[s + 1];) {
         const TreeType& t = T.type[T.node[i].type];
@@ -314,7 +300,7 @@ int tree_scratch(Helm& H, int nf) {
         g = (run + (run + g - 1) / g - 1) / ((run + g - 1) / g);
         for (int j = 0; j < run; j += g)
           for (int mt = 0; mt < tree_mt(rows) || (mt == 0 && rows == 0); mt += wm)
-            task.push_back({i + j, std::min(g, run - j), mt, 0});
+            tasks.push_back({i + j, std::min(g, run - j), mt, 0});
         nmax = std::max(nmax, g * nrhs);
         kl = std::max(kl, (K + 7) / 8 * 8);
         i += run;
@@ -323,20 +309,46 @@ int tree_scratch(Helm& H, int nf) {
       L.ldn = 16;
       if (L.ct == 1) { L.ldn = 1; while (L.ldn < nmax) L.ldn *= 2; }
       size_t v = 0;
-      for (const TreeTask& k : task) {
-        const TreeType& t = T.type[T.node[k.node].type];
+      for (size_t k = first; k < tasks.size(); ++k) {
+        const TreeType& t = T.type[T.node[tasks[k].node].type];
         const size_t Kr = ((dir ? t.ni + t.nb : t.ni) + 7) / 8 * 8;
-        v = std::max(v, Kr * (L.ct == 1 ? (size_t)L.ldn : (size_t)(k.count * nrhs + 15) / 16 * 16));
+        v = std::max(v, Kr * (L.ct == 1 ? (size_t)L.ldn : (size_t)(tasks[k].count * nrhs + 15) / 16 * 16));
       }
       // the product reads every column tile of its width
       if (L.ct > 1) v = std::max(v, (size_t)kl * 16 * L.ct);
       L.lds = std::max(v, (size_t)TW * 16 * L.ct * 17) * sizeof(double);
       if (L.ct > 3 || L.lds > 160 * 1024) return SEMX_E_UNSUPPORTED;
-      L.ntask = (int)task.size();
-      if ((st = dev_upload(&L.task, task.data(), task.size()))) return st;
+      L.first = first;
+      L.ntask = (int)(tasks.size() - first);
       out.push_back(L);
     }
-  D->list[nf] = out;
+  return SEMX_OK;
+}
+
+// Contribution scratch for nf fields and the launch lists of every field
+// count up to that (one allocation each): a solve of fewer fields may be
+// captured into a graph without a call of its own before it.
+int tree_scratch(Helm& H, int nf) {
+  Tree& T = H.tree;
+  TreeDev* D = H.d.tree;
+  int st;
+  if (nf <= D->nf_cap) return SEMX_OK;
+  dev_free(D->C); dev_free(D->Y);
+  D->nf_cap = 0;
+  const size_t np = (size_t)H.nplanes * nf;
+  if ((st = dev_upload<double>(&D->C, nullptr, np * T.nslot_c))) return st;
+  if ((st = dev_upload<double>(&D->Y, nullptr, np * T.nslot_y))) return st;
+  int npl = 1;
+  for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) npl = 2;
+  for (int f = 1; f <= nf; ++f) {
+    if (D->task[f]) continue;
+    std::vector<TreeTask> tasks;
+    std::vector<TreeList> list;
+    if ((st = tree_lists(T, npl * f, list, tasks))) return st;
+    if ((st = dev_upload(&D->task[f], tasks.data(), tasks.size()))) return st;
+    D->list[f] = list;
+  }
+  D->nf_cap = nf;
   return SEMX_OK;
 }
 
@@ -345,7 +357,7 @@ void tree_release(Helm& H) {
   if (!D) return;
   dev_free(D->mat); dev_free(D->type); dev_free(D->node); dev_free(D->gid);
   dev_free(D->rowptr); dev_free(D->src); dev_free(D->C); dev_free(D->Y);
-  for (auto& v : D->list) for (TreeList& L : v) dev_free(L.task);
+  for (TreeTask*& t : D->task) dev_free(t);
   delete D;
   H.d.tree = nullptr;
 }
@@ -383,7 +395,7 @@ int tree_solve(Helm& H, int nf, size_t pFb, size_t psol, hipStream_t s) {
     else
       fn = l.ct == 1 ? (const void*)k_tree_down<1, false>
                      : l.ct == 2 ? (const void*)k_tree_down<2, false> : (const void*)k_tree_down<3, false>;
-    a.task = l.task; a.wk = l.wk; a.ldn = l.ldn;
+    a.task = D->task[nf] + l.first; a.wk = l.wk; a.ldn = l.ldn;
     if (l.lds > 64 * 1024)
       HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
     void* kargs[] = {&a, &nleaf};

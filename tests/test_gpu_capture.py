@@ -91,3 +91,20 @@ def test_batch_reranked_solves_repeat(cuda):
         torch.cuda.synchronize()
         ref = ref or us
         assert all(torch.equal(u, v) for u, v in zip(us, ref)), r
+
+
+@pytest.mark.parametrize("method", [sx.DIRECT, sx.JACPCG, sx.MIXED], ids=["direct", "jacpcg", "mixed"])
+def test_fewer_fields_captured(cuda, method):
+    """A system solved with three fields captures a solve of one and of two
+    without solving that many before."""
+    import torch
+    print(f"[capture] fields, method {method}", flush=True)
+    P, ins = _case(7, 6, 6, 8, [3, 4, 5])
+    S = sx.ModalMatrixSys(P, 2.0, 1.2, 0, 4, 8, method)
+    fs, bs = [i[0] for i in ins], [i[1] for i in ins]
+    ref = [torch.zeros_like(f) for f in fs]
+    sx.solve_fields(S, fs, bs, ref, iters=False)
+    torch.cuda.synchronize()
+    for nf in (1, 2):
+        _capture_and_replay(
+            torch, lambda us: sx.solve_fields(S, fs[:nf], bs[:nf], us, iters=False), ref[:nf])
