@@ -272,9 +272,13 @@ int tree_upload(Helm& H) {
   return SEMX_OK;
 }
 
-// Launch lists of nf fields, without their device addresses: up to TREE_GROUP
-// regions of one type per workgroup, as many as the right-hand-side tile's
-// LDS holds.
+// Launch lists for nrhs right-hand sides a mode, without their device
+// addresses: up to TREE_GROUP regions of one type per workgroup, as many as
+// the right-hand-side tile's LDS holds.  Every workgroup of a stage reads as
+// many column tiles as its widest one, so the stage's longest regions limit
+// the columns of all: a duct's short regions beside a large section's long
+// ones are taken in smaller groups (nrhs <= 6 columns of the at most 2048
+// rows that tree_plan allows always fit).
 static int tree_lists(const Tree& T, int nrhs, std::vector<TreeList>& out,
                       std::vector<TreeTask>& tasks) {
   for (int dir = 0; dir < 2; ++dir)
@@ -283,18 +287,22 @@ static int tree_lists(const Tree& T, int nrhs, std::vector<TreeList>& out,
       int Kmax = 0;
       for (int i = T.stage_ptr[s]; i < T.stage_ptr[s + 1]; ++i) {
         const TreeType& t = T.type[T.node[i].type];
-        Kmax = std::max(Kmax, dir ? t.ni + t.nb : t.ni);
+        Kmax = std::max(Kmax, dir && t.ni ? t.ni + t.nb : t.ni);
       }
       L.wk = share(Kmax);
-      const int wm = TW / L.wk;
+      const int wm = TW / L.wk, kl = (Kmax + 7) / 8 * 8;
+      int cols = 48;            // three column tiles
+      while (cols > 16 && (size_t)kl * cols * 8 > 160 * 1024) cols -= 16;
+      if ((size_t)kl * cols * 8 > 160 * 1024) cols = 8;
       const size_t first = tasks.size();
-      int nmax = 1, kl = 0;
+      int nmax = 1;
       for (int i = T.stage_ptr[s]; i < T.stage_ptr[s + 1];) {
         const TreeType& t = T.type[T.node[i].type];
         const int K = dir ? t.ni + t.nb : t.ni, rows = dir ? t.ni : t.nb;
         int run = 1;
         while (i + run < T.stage_ptr[s + 1] && T.node[i + run].type == T.node[i].type) ++run;
-        int g = std::min(run, TREE_GROUP);
+        if (dir && rows == 0) { i += run; continue; }    // nothing to recover
+        int g = std::min({run, TREE_GROUP, std::max(1, cols / nrhs)});
         while (g > 1 && (size_t)((K + 7) / 8 * 8) * ((g * nrhs + 15) / 16 * 16) * 8 > 64 * 1024) --g;
         // even groups
         g = (run + (run + g - 1) / g - 1) / ((run + g - 1) / g);
@@ -302,7 +310,6 @@ static int tree_lists(const Tree& T, int nrhs, std::vector<TreeList>& out,
           for (int mt = 0; mt < tree_mt(rows) || (mt == 0 && rows == 0); mt += wm)
             tasks.push_back({i + j, std::min(g, run - j), mt, 0});
         nmax = std::max(nmax, g * nrhs);
-        kl = std::max(kl, (K + 7) / 8 * 8);
         i += run;
       }
       L.ct = (nmax + 15) / 16;
@@ -395,6 +402,7 @@ int tree_solve(Helm& H, int nf, size_t pFb, size_t psol, hipStream_t s) {
     else
       fn = l.ct == 1 ? (const void*)k_tree_down<1, false>
                      : l.ct == 2 ? (const void*)k_tree_down<2, false> : (const void*)k_tree_down<3, false>;
+    if (!l.ntask) continue;
     a.task = D->task[nf] + l.first; a.wk = l.wk; a.ldn = l.ldn;
     if (l.lds > 64 * 1024)
       HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
