@@ -224,8 +224,9 @@ int semx_helm_solve (semx_helm helm, double* f, const double* bc, double* u,
                      double tol_rel, int step_max, int* iters, void* stream);
 
 /* Waits for stream and reports whether any solve of this system since the
- * last check had a cooperative band sweep whose bounded hand-off wait
- * expired (SEMX_E_TIMEOUT; its solution is wrong), then clears the mark.
+ * last check had a bounded wait between workgroups that expired -- in a
+ * cooperative or partitioned band sweep, or in the PCG of a plane on several
+ * workgroups (SEMX_E_TIMEOUT; its solution is wrong) -- then clears the mark.
  * No counterpart in semtex, whose solves are synchronous.  A solve called
  * with iters != NULL and semx_dns_run make this check themselves, so a
  * timeout is reported by the first synchronising call after it, never

@@ -228,8 +228,8 @@ def solve(msys, f, bc, u, tol_rel=1e-12, step_max=10000, stream=None, iters=True
 
 def helm_check(msys, stream=None):
     """Wait for the stream and raise SemxError(SEMX_E_TIMEOUT) if any solve
-    of this system since the last check had a cooperative band sweep whose
-    bounded hand-off wait expired (semx_helm_check)."""
+    of this system since the last check had a bounded wait between workgroups
+    (a band sweep's or a PCG's) that expired (semx_helm_check)."""
     check(load().semx_helm_check(msys.h, _stream(stream)), "semx_helm_check")
 
 

@@ -65,6 +65,7 @@ struct ChipArgs {
   int planeSize, nzero;
   double tol, inner_tol;
   int step_max, max_outer;
+  bool no_wait;            // set by chip_launch
   // planes: condensed right-hand sides, essential values, solutions
   const double* Fb;
   const double* Fi;

@@ -1958,15 +1958,17 @@ int semx_dns_run(semx_dns dns, int nstep, double* u, double* v, double* w, doubl
   for (int i = 0; i < D.ncom; ++i)
     HIPCHK(hipMemcpyAsync(D.U[i], ext[i], bytes, hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync(D.P, p, bytes, hipMemcpyDeviceToDevice, s));
+  const bool startup = D.step + 1 < D.nord;
   for (int k = 0; k < nstep; ++k) CHK(dns_step_graph(D, s));
   for (int i = 0; i < D.ncom; ++i)
     HIPCHK(hipMemcpyAsync(ext[i], D.U[i], bytes, hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync(p, D.P, bytes, hipMemcpyDeviceToDevice, s));
   // the solves of the steps ran without host synchronisation: any expired
-  // cooperative hand-off wait among them is reported here
+  // wait between workgroups among them is reported here (every system is
+  // checked, so that none keeps its mark for a later run)
   int st = SEMX_OK;
-  for (Helm* h : {D.vel, D.pre})
-    if (h && !st) st = helm_check(*h, s);
+  for (Helm* h : {D.vel, D.pre, startup ? D.start[0] : nullptr, startup ? D.start[1] : nullptr})
+    if (const int e = h ? helm_check(*h, s) : SEMX_OK) st = e;
   return st;
 }
 

@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <vector>
 
@@ -742,7 +743,7 @@ __global__ __launch_bounds__(CT) void k_pcg_chip(ChipArgs a) {
   Wg G;
   G.W = M.W; G.w = job.y; G.ne = pt.ne; G.nslot = pt.ne * M.next;
   G.nrem = pt.nrem; G.npub = pt.npub;
-  G.dead = false;
+  G.dead = a.no_wait;
   G.kA = G.kB = 0;
   G.nif = M.nif;
   G.exch = a.exch + fld * a.exchF + I.exch;
@@ -961,9 +962,13 @@ int chip_launch(const ChipArgs& a, int np, bool refine, int groups, size_t lds, 
   const long long n = std::max(std::max(nexch, nred), 1LL);
   hipLaunchKernelGGL(k_chip_reset, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.exch,
                      nexch, a.red, nred, a.ticket);
+  // SEMX_PCG_NOWAIT=1, for tests of an expired wait: no value is waited for
+  // (a limit on the polls as an argument of the kernel cost the batch 3%)
+  ChipArgs b = a;
+  b.no_wait = getenv("SEMX_PCG_NOWAIT") && atoi(getenv("SEMX_PCG_NOWAIT")) != 0;
   hipEvent_t ev;
   prof_begin(s, &ev);
-  void* kargs[] = {(void*)&a};
+  void* kargs[] = {&b};
   HIPCHK(hipLaunchKernel(fn, dim3((unsigned)groups), dim3(CT), kargs, lds, s));
   prof_end(s, a.bf ? "k_pcg_batch" : "k_pcg", ev);
   HIPCHK(hipGetLastError());

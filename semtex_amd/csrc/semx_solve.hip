@@ -3384,20 +3384,24 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
   return SEMX_OK;
 }
 
-// The cooperative and partitioned band sweeps set a sticky error word when a bounded
-// hand-off wait expires (their result is then wrong).  Every host
-// synchronisation point of the solve path reads it here, after the stream
-// has drained, and clears it, so a timeout is reported exactly once, by the
-// first check after it happened, whatever the caller passed for iters.
+// The cooperative and partitioned band sweeps and the PCG of planes on several
+// workgroups set a sticky error word when a bounded wait for another workgroup
+// expires (their result is then wrong).  Every host synchronisation point of
+// the solve path reads it here, after the stream has drained, and clears it,
+// so a timeout is reported exactly once, by the first check after it happened,
+// whatever the caller passed for iters.
 int helm_check(Helm& H, hipStream_t s) {
   HIPCHK(hipStreamSynchronize(s));
-  if ((H.coop_w <= 0 && H.npart <= 1 && H.pcg_w <= 1 && !H.d.chip) || !H.d.err) return SEMX_OK;
+  const bool band = H.coop_w > 0 || H.npart > 1;
+  const bool pcg = H.pcg_w > 1 || (H.d.chip && H.d.chip->plan.W > 1);
+  if ((!band && !pcg) || !H.d.err) return SEMX_OK;
   int e = 0;
   HIPCHK(hipMemcpy(&e, H.d.err, sizeof(int), hipMemcpyDeviceToHost));
   if (!e) return SEMX_OK;
   const int zero = 0;
   HIPCHK(hipMemcpy(H.d.err, &zero, sizeof(int), hipMemcpyHostToDevice));
-  fprintf(stderr, "semx: cooperative or partitioned band solve: hand-off wait timed out\n");
+  fprintf(stderr, "semx: %s: a wait for another workgroup timed out\n",
+          band && pcg ? "band sweep or PCG" : band ? "band sweep" : "PCG");
   return SEMX_E_TIMEOUT;
 }
 
