@@ -193,16 +193,26 @@ int semx_helm_destroy (semx_helm helm);
  *           bytes_per_solve_factor(MB*1000, int) singular(mode0); the factor
  *           is the elimination tree's matrices or the band's factor        */
 int semx_helm_info (semx_helm helm, int* info);
-/* How the direct planes' band sweeps run; no counterpart in semtex (whose
- * dpbtrs is one call) -- and how the PCG planes run.  info[6] = partitions
- * per mode of the partitioned sweep (1: not available), the sweep variant
- * the first call picked for 1, 2 and 3 fields (0 before that call; 1-7 one
- * workgroup per mode, field or plane over the whole band, 8 the
- * partitioned sweep, 9 the elimination tree: regions of elements merged
- * level by level, each eliminated with dense matrices; the default, with
- * SEMX_TREE=0 or any of the sweeps' own switches selecting the sweeps), workgroups per mode of the cooperative sweep (0: not
- * used), workgroups per PCG plane in the last solve.                      */
+/* How the direct planes are solved, and how k_pcg lays out the PCG planes;
+ * no counterpart in semtex (whose dpbtrs is one call).  info[6] = partitions
+ * per mode of the partitioned sweep (1: not available); the variant the first
+ * call picked for 1, 2 and 3 fields (0 before that call; 1-7 band sweeps of
+ * one workgroup per mode, field or plane over the whole band, 8 the
+ * partitioned sweep, 9 the elimination tree: regions of elements merged level
+ * by level, each eliminated with dense matrices; the default, with
+ * SEMX_TREE=0 or any of the sweeps' own switches selecting the sweeps);
+ * workgroups per mode of the cooperative sweep (0: not used); workgroups per
+ * PCG plane of the kernel k_pcg: uniform until a solve has read back the
+ * planes' iteration counts, then the most of a plane in the map balanced by
+ * them.  Where the last solve ran on chip instead (semx_helm_pcg_info) the
+ * last figure is what k_pcg would have taken, and takes once the precision or
+ * a switch selects it.                                                     */
 int semx_helm_sweep_info (semx_helm helm, int* info);
+/* Where the last solve's PCG planes ran.  info[2] = 1: with the vectors held
+ * on chip (np 4 to 12 in FP64 and FP32 refined, meshes of at most 48
+ * workgroups a plane; SEMX_PCG_CHIP=0, SEMX_PCG_WG or SEMX_PCG_OP select
+ * k_pcg), 0: in k_pcg; workgroups per plane (k_pcg: the most of one).      */
+int semx_helm_pcg_info (semx_helm helm, int* info);
 /* Host copies of one element's condensed matrices for mode index m
  * (HelmholtzSC, src/element.cpp:131-229): hbb next^2, hbi next*nint,
  * hii nint^2, all row-major in emap order.                                 */

@@ -177,12 +177,19 @@ class ModalMatrixSys:
         return hbb, hbi[:, :M.nint], hii[:M.nint, :M.nint]
 
     def sweep_info(self):
-        """Band-sweep and PCG layout: dict(npart, pick={1: , 2: , 3: },
-        coop_w, pcg_w)."""
+        """How the direct planes are solved and k_pcg's layout: dict(npart,
+        pick={1: , 2: , 3: }, coop_w, pcg_w)."""
         info = np.zeros(6, dtype=np.int32)
         check(load().semx_helm_sweep_info(self.h, _ip(info)), "semx_helm_sweep_info")
         return dict(npart=int(info[0]), pick={f: int(info[f]) for f in (1, 2, 3)},
                     coop_w=int(info[4]), pcg_w=int(info[5]))
+
+    def pcg_info(self):
+        """Where the last solve's PCG planes ran: dict(on_chip, workgroups)
+        (workgroups per plane)."""
+        info = np.zeros(2, dtype=np.int32)
+        check(load().semx_helm_pcg_info(self.h, _ip(info)), "semx_helm_pcg_info")
+        return dict(on_chip=bool(info[0]), workgroups=int(info[1]))
 
     def __del__(self):
         try:

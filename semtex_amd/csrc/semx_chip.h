@@ -96,8 +96,8 @@ struct ChipDev {
   unsigned* ticket = nullptr;
   int nf_cap = 0;                      // fields the slots hold
   const double* work = nullptr;        // the scratch inst points into
-  std::vector<int> rank;               // planes in the order they are taken
-  bool ranked = false;                 // by measured iteration counts
+  std::vector<int> rank;               // planes in the order they are taken:
+                                       // as listed, or by iteration counts
   int2* order[SEMX_MAX_FIELDS + 1] = {nullptr};
 };
 

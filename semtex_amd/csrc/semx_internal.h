@@ -187,7 +187,11 @@ struct Helm {
   std::vector<int> dmode, mode_plane;
   std::vector<int> pcg_plane;         // plane-list indices of JACPCG modes
   int pcg_prec = 0;                   // SEMX_PCG_FP64, _FP32_REFINED or _BF16_REFINED
-  int pcg_w = 1;                      // workgroups per PCG plane (last solve)
+  int pcg_w = 1;                      // workgroups per PCG plane (last k_pcg solve)
+  bool pcg_onchip = false;            // the last solve's PCG planes ran on chip
+  std::vector<double> pcg_counts;     // planes' iteration counts last read back
+  bool pcg_stale = false;             // newer than the balanced map
+  bool pcg_known = false;             // there were any at the last on-chip solve
   size_t pcg_ws = 0;                  // plane-workgroup slots allocated
   int pcg_nwg = 0;                    // workgroups of the balanced map (0: none)
   int pcg_wtop = 1;                   // most workgroups of a plane in that map

@@ -2603,6 +2603,7 @@ void helm_release(Helm& H) {
     H.d.chip = nullptr;
   }
   H.d.chip_tried = false;
+  H.pcg_onchip = false;
   H.pcg_ws = 0;
   H.pcg_nwg = 0;
   H.nf_cap = 0;
@@ -2642,8 +2643,8 @@ bool stream_capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
-// Workgroups per PCG plane from the planes' iteration counts of the last
-// solve (it: npcg per field; the largest over the fields is taken).  An
+// Workgroups per PCG plane of k_pcg from the planes' iteration counts of the
+// last solve that read them back (false: no split).  An
 // iteration of a plane on W workgroups is modelled as taking A + 1/W of its
 // one-workgroup time (A: the share that does not shrink with W; 0.03 was
 // the fastest of 0.35, 0.2, 0.1 and 0.03 on 32x32 quads np=11 Nz=128, in
@@ -2655,8 +2656,7 @@ bool stream_capturing(hipStream_t s) {
 // the model's error (the refined solves' inner iteration counts leave out
 // their outer sweeps).  The planes' workgroups are laid out plane by
 // plane, the most-split planes first.
-int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, size_t lds) {
-  if (H.pcg_frozen) return SEMX_OK;
+bool pcg_split(const Helm& H, const void* kfn, size_t lds, std::vector<int>& Wp) {
   const int npcg = (int)H.pcg_plane.size();
   int cus = 256, dev = 0, per_cu = 0;
   if (hipGetDevice(&dev) == hipSuccess)
@@ -2665,13 +2665,10 @@ int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, si
     per_cu = 0;
   const long budget = (long)per_cu * cus;
   const int wcap = std::max(1, std::min(PCG_WMAX, H.npts / 6144));
-  if (npcg == 0 || budget <= npcg || wcap == 1) return SEMX_OK;
-  std::vector<double> cnt(npcg, 1.0);
-  for (int f = 0; f < nf; ++f)
-    for (int p = 0; p < npcg; ++p)
-      cnt[p] = std::max(cnt[p], (double)std::abs(it[(size_t)f * npcg + p]));
+  if (H.pcg_counts.empty() || npcg == 0 || budget <= npcg || wcap == 1) return false;
+  const std::vector<double>& cnt = H.pcg_counts;
   constexpr double A = 0.03;
-  std::vector<int> Wp(npcg, 1);
+  Wp.assign(npcg, 1);
   long tot = npcg;
   while (tot < budget) {
     int b = -1;
@@ -2682,28 +2679,104 @@ int pcg_balance(Helm& H, const std::vector<int>& it, int nf, const void* kfn, si
     ++Wp[b];
     ++tot;
   }
+  return true;
+}
+
+// The workgroup map of that split.
+int pcg_balance(Helm& H, int nf, const void* kfn, size_t lds) {
+  const int npcg = (int)H.pcg_plane.size();
+  std::vector<int> Wp;
+  H.pcg_stale = false;
+  if (!pcg_split(H, kfn, lds, Wp)) return SEMX_OK;
   std::vector<int> ord(npcg);
   for (int p = 0; p < npcg; ++p) ord[p] = p;
   std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return Wp[x] > Wp[y]; });
   std::vector<int> wm;
-  wm.reserve((size_t)tot * 4);
   for (int p : ord)
     for (int w = 0; w < Wp[p]; ++w) { wm.push_back(p); wm.push_back(w); wm.push_back(Wp[p]); wm.push_back(0); }
   dev_free(H.d.pwmap);
   H.pcg_nwg = 0;
-  if (H.pcg_ws < (size_t)npcg * nf || !H.d.pctr) {
-    dev_free(H.d.pctr);
-    dev_free(H.d.pslot2);
-    int st = dev_upload<unsigned>(&H.d.pctr, nullptr, (size_t)npcg * nf * 16);
-    if (!st) st = dev_upload<double>(&H.d.pslot2, nullptr, (size_t)npcg * nf * 4 * PCG_WMAX);
-    if (!st && !H.d.err) st = dev_upload<int>(&H.d.err, nullptr, 1);
-    if (st) return st;
-    H.pcg_ws = (size_t)npcg * nf;
-  }
   const int st = dev_upload(&H.d.pwmap, wm.data(), wm.size());
   if (st) return st;
-  H.pcg_nwg = (int)tot;
+  H.pcg_nwg = (int)(wm.size() / 4);
   H.pcg_wtop = std::max(2, *std::max_element(Wp.begin(), Wp.end()));
+  return SEMX_OK;
+}
+
+// Iteration counts read back (it: npcg per field), for the next map.
+void pcg_counted(Helm& H, const std::vector<int>& it, int nf) {
+  if (H.pcg_frozen) return;
+  const int npcg = (int)H.pcg_plane.size();
+  H.pcg_counts.assign(npcg, 1.0);
+  for (int f = 0; f < nf; ++f)
+    for (int p = 0; p < npcg; ++p)
+      H.pcg_counts[p] = std::max(H.pcg_counts[p], (double)std::abs(it[(size_t)f * npcg + p]));
+  H.pcg_stale = true;
+}
+
+// k_pcg for the system's precision, and the LDS of every element operator
+// (block-wide, wavefront-level, BF16).
+const void* pcg_fn(const Helm& H, int opk) {
+  if (H.pcg_prec == SEMX_PCG_FP64)
+    return opk == OPK_WAVE ? (const void*)k_pcg<double, false, OPK_WAVE>
+                           : (const void*)k_pcg<double, false, OPK_BLOCK>;
+  if (H.pcg_prec == SEMX_PCG_BF16_REFINED && opk == OPK_MFMA)
+    return (const void*)k_pcg<float, true, OPK_MFMA>;
+  return opk == OPK_WAVE ? (const void*)k_pcg<float, true, OPK_WAVE>
+                         : (const void*)k_pcg<float, true, OPK_BLOCK>;
+}
+
+size_t pcg_lds_bytes(const Helm& H) {
+  const size_t npnp = H.M->npnp, cep = PCG_THREADS / npnp;
+  size_t d = std::max((2 + 3 * cep) * npnp, (2 + 3 * (size_t)PCG_WAVES) * npnp) * sizeof(double);
+  if (H.pcg_prec == SEMX_PCG_BF16_REFINED)
+    d = std::max(d, (size_t)PCG_WAVES * 2 * MF_TILE * sizeof(float));
+  return RED_DOUBLES * sizeof(double) + d;
+}
+
+// Workgroups per plane of k_pcg without a map: enough that the planes of one
+// field fill the chip's CUs (each 1024-thread workgroup holds a CU), at most
+// 8, each with at least 8192 vector rows, and only if the whole grid can be
+// resident (the plane's workgroups wait for each other); SEMX_PCG_WG sets the
+// count (1: one workgroup per plane).
+int pcg_uniform(const Helm& H, const void* fn, size_t lds) {
+  const long npcg = std::max<long>((long)H.pcg_plane.size(), 1);
+  int cus = 256, dev = 0, per_cu = 0;
+  if (hipGetDevice(&dev) == hipSuccess)
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  int W = std::max(1, std::min(8, cus / (int)npcg));
+  W = std::max(1, std::min(W, H.npts / 8192));
+  if (const char* e = getenv("SEMX_PCG_WG")) W = std::max(1, std::min(8, atoi(e)));
+  if (W > 1 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, PCG_THREADS, lds) !=
+                    hipSuccess ||
+                per_cu * (long)cus < npcg * W))
+    W = 1;
+  return W;
+}
+
+// What a k_pcg launch for nf fields needs: its uniform workgroup count W,
+// and, once a solve has read back the planes' iteration counts -- k_pcg's own
+// or the on-chip iteration's --, the balanced map in its place (bal).
+int pcg_shape(Helm& H, int nf, int& W, bool& bal) {
+  const int opk = H.pcg_opk >= 0 ? H.pcg_opk
+                  : H.pcg_prec == SEMX_PCG_BF16_REFINED ? OPK_MFMA : OPK_BLOCK;
+  const void* fn = pcg_fn(H, opk);
+  const size_t lds = pcg_lds_bytes(H), npcg = H.pcg_plane.size();
+  if (lds > 64 * 1024)
+    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  if (H.pcg_stale && !H.pcg_frozen && !getenv("SEMX_PCG_WG"))
+    if (const int st = pcg_balance(H, nf, fn, lds)) return st;
+  W = pcg_uniform(H, fn, lds);
+  bal = H.pcg_nwg > 0 && H.d.pwmap && !getenv("SEMX_PCG_WG");
+  if ((W > 1 || bal) && (H.pcg_ws < npcg * nf || !H.d.pctr)) {
+    dev_free(H.d.pctr);
+    dev_free(H.d.pslot2);
+    int st = dev_upload<unsigned>(&H.d.pctr, nullptr, npcg * nf * 16);
+    if (!st) st = dev_upload<double>(&H.d.pslot2, nullptr, npcg * nf * 4 * PCG_WMAX);
+    if (!st && !H.d.err) st = dev_upload<int>(&H.d.err, nullptr, 1);
+    if (st) return st;
+    H.pcg_ws = npcg * nf;
+  }
   return SEMX_OK;
 }
 
@@ -2780,10 +2853,6 @@ int chip_prepare(Helm& H, int nf) {
     C->nf_cap = nf;
     C->work = H.d.work;
   }
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  H.pcg_w = C->ranked ? W : std::max(1, std::min(W, cus / npcg));
   return SEMX_OK;
 }
 
@@ -2800,7 +2869,6 @@ int chip_rank(Helm& H, const std::vector<int>& it, int nf) {
       cnt[p] = std::max(cnt[p], std::abs(it[(size_t)f * npcg + p]));
   for (int p = 0; p < npcg; ++p) rank[p] = p;
   std::stable_sort(rank.begin(), rank.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
-  C->ranked = true;
   if (rank == C->rank) return SEMX_OK;
   C->rank = rank;
   for (int f = 1; f <= SEMX_MAX_FIELDS; ++f)
@@ -3172,6 +3240,8 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
   if (chip) {
     const ChipDev& C = *H.d.chip;
     const int npcg = (int)H.pcg_plane.size(), W = C.plan.W;
+    H.pcg_onchip = true;
+    H.pcg_known = !H.pcg_counts.empty();
     ChipArgs ca{};
     ca.inst = C.inst; ca.order = C.order[nf]; ca.ticket = C.ticket;
     ca.exch = C.exch; ca.red = C.red;
@@ -3202,6 +3272,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
         return st2 ? st2 : SEMX_E_MAXITER;
       }
       if ((st = chip_rank(H, it, nf))) return st;
+      pcg_counted(H, it, nf);
     }
   } else if (!H.pcg_plane.empty()) {
     PcgArgs pa;
@@ -3217,61 +3288,13 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
     pa.u = nullptr; pa.work = H.d.work; pa.workstride = H.workstride;
     pa.tol = tol_rel; pa.step_max = step_max; pa.inner_tol = H.inner_tol;
     pa.max_outer = H.max_outer; pa.iters = H.d.iters;
-    const int cep = PCG_THREADS / M.npnp;
-    // LDS of every element operator (block-wide, wavefront-level, BF16)
-    size_t lds = RED_DOUBLES * sizeof(double) +
-        (2 * (size_t)M.npnp + 3 * (size_t)cep * M.npnp) * sizeof(double);
-    lds = std::max(lds, RED_DOUBLES * sizeof(double) +
-                        (2 + 3 * (size_t)PCG_WAVES) * M.npnp * sizeof(double));
-    if (H.pcg_prec == SEMX_PCG_BF16_REFINED)
-      lds = std::max(lds, RED_DOUBLES * sizeof(double) + (size_t)PCG_WAVES * 2 * MF_TILE * sizeof(float));
-    auto pcg_fn = [&](int opk) -> const void* {
-      if (H.pcg_prec == SEMX_PCG_FP64)
-        return opk == OPK_WAVE ? (const void*)k_pcg<double, false, OPK_WAVE>
-                               : (const void*)k_pcg<double, false, OPK_BLOCK>;
-      if (H.pcg_prec == SEMX_PCG_BF16_REFINED && opk == OPK_MFMA)
-        return (const void*)k_pcg<float, true, OPK_MFMA>;
-      return opk == OPK_WAVE ? (const void*)k_pcg<float, true, OPK_WAVE>
-                             : (const void*)k_pcg<float, true, OPK_BLOCK>;
-    };
+    const size_t lds = pcg_lds_bytes(H);
     const size_t npcg = H.pcg_plane.size();
-    // Workgroups per plane: enough that the planes of one field fill the
-    // chip's CUs (each 1024-thread workgroup holds a CU), at most 8, each
-    // with at least 8192 vector rows, and only if the whole grid can be
-    // resident (the plane's workgroups wait for each other); SEMX_PCG_WG
-    // sets the count (1: one workgroup per plane).  Once a solve has read
-    // back the planes' iteration counts, a balanced map replaces the
-    // uniform count (pcg_balance).
     int W = 1;
-    const bool bal = H.pcg_nwg > 0 && H.d.pwmap && !getenv("SEMX_PCG_WG");
-    {
-      int cus = 256, dev = 0, per_cu = 0;
-      if (hipGetDevice(&dev) == hipSuccess)
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      W = std::max(1, std::min(8, cus / (int)std::max<size_t>(npcg, 1)));
-      W = std::max(1, std::min(W, H.npts / 8192));
-      if (const char* e = getenv("SEMX_PCG_WG")) W = std::max(1, std::min(8, atoi(e)));
-      if (W > 1) {
-        const void* probe = pcg_fn(H.pcg_opk < 0 ? OPK_BLOCK : H.pcg_opk);
-        if (lds > 64 * 1024)
-          HIPCHK(hipFuncSetAttribute(probe, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds));
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, probe, PCG_THREADS, lds) !=
-                hipSuccess ||
-            (long)per_cu * cus < (long)npcg * W)
-          W = 1;
-      }
-      if ((W > 1 || bal) && (H.pcg_ws < npcg * nf || !H.d.pctr)) {
-        dev_free(H.d.pctr);
-        dev_free(H.d.pslot2);
-        int st2 = dev_upload<unsigned>(&H.d.pctr, nullptr, npcg * nf * 16);
-        if (!st2) st2 = dev_upload<double>(&H.d.pslot2, nullptr, npcg * nf * 4 * PCG_WMAX);
-        if (!st2 && !H.d.err) st2 = dev_upload<int>(&H.d.err, nullptr, 1);
-        if (st2) return st2;
-        H.pcg_ws = npcg * nf;
-      }
-      H.pcg_w = bal ? H.pcg_wtop : W;
-    }
+    bool bal = false;
+    if ((st = pcg_shape(H, nf, W, bal))) return st;
+    H.pcg_w = bal ? H.pcg_wtop : W;
+    H.pcg_onchip = false;
     pa.W = W;
     pa.wmap = bal ? H.d.pwmap : nullptr;
     const unsigned grid = bal ? (unsigned)H.pcg_nwg : (unsigned)(npcg * W);
@@ -3315,7 +3338,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
           pt.step_max = PCG_TUNE_ITERS;
           pt.max_outer = 1;
           pt.wmap = nullptr;
-          const void* fn = pcg_fn(c);
+          const void* fn = pcg_fn(H, c);
           if (lds > 64 * 1024)
             HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
           HIPCHK(hipMemcpyAsync(scr, us[0], nu * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -3339,7 +3362,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
         dev_free(scr);
       }
     }
-    const void* kfn = pcg_fn(H.pcg_opk);
+    const void* kfn = pcg_fn(H, H.pcg_opk);
     if (lds > 64 * 1024)
       HIPCHK(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     for (int i = 0; i < nf; ++i) {
@@ -3373,9 +3396,10 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
         const int st = helm_check(H, s);
         return st ? st : SEMX_E_MAXITER;
       }
+      // the next map at once: the next solve may be captured into a graph
       if (!getenv("SEMX_PCG_WG")) {
-        const int st = pcg_balance(H, it, nf, kfn, lds);
-        if (st) return st;
+        pcg_counted(H, it, nf);
+        if ((st = pcg_shape(H, nf, W, bal))) return st;
       }
     }
   }
@@ -3620,6 +3644,25 @@ int semx_helm_sweep_info(semx_helm helm, int* info) {
   for (int f = 1; f <= SEMX_MAX_FIELDS; ++f) info[f] = H.band_pick[f];
   info[4] = H.coop_w;
   info[5] = H.pcg_w;
+  if (H.pcg_onchip) {
+    const int opk = H.pcg_prec == SEMX_PCG_BF16_REFINED ? OPK_MFMA : OPK_BLOCK;
+    const void* fn = pcg_fn(H, opk);
+    const size_t lds = pcg_lds_bytes(H);
+    if (lds > 64 * 1024)
+      HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    std::vector<int> Wp;
+    info[5] = H.pcg_known && pcg_split(H, fn, lds, Wp)
+                  ? std::max(2, *std::max_element(Wp.begin(), Wp.end()))
+                  : pcg_uniform(H, fn, lds);
+  }
+  return SEMX_OK;
+}
+
+int semx_helm_pcg_info(semx_helm helm, int* info) {
+  if (!helm || !info) return SEMX_E_ARG;
+  const Helm& H = helm->H;
+  info[0] = H.pcg_onchip;
+  info[1] = H.pcg_onchip ? H.d.chip->plan.W : H.pcg_w;
   return SEMX_OK;
 }
 
@@ -4135,6 +4178,12 @@ int semx_helm_set_pcg(semx_helm helm, int precision, double inner_tol, int max_o
   if (H.pcg_prec != precision) H.pcg_opk = -1;
   H.pcg_prec = precision;
   if (refine) { H.inner_tol = inner_tol; H.max_outer = max_outer; }
+  // after on-chip solves, what k_pcg will need: its first solve may be captured
+  if (H.pcg_onchip && precision == SEMX_PCG_BF16_REFINED) {
+    int W = 1;
+    bool bal = false;
+    return pcg_shape(H, H.nf_cap, W, bal);
+  }
   return SEMX_OK;
 }
 
