@@ -294,13 +294,16 @@ int semx_batch_create (int count, const semx_helm* helms, semx_batch* batch);
 int semx_batch_destroy (semx_batch batch);
 /* The element operator each problem's inner iteration uses (opk[count]:
  * 0 block-wide scalar, 1 wavefront-level scalar, 2 BF16 matrix cores; -1
- * before the first solve) and the host time the batch tuner took (ms).
- * The first semx_batch_solve tunes: per class of problems with the same np
- * and element count it times each operator the precision allows on the
- * class's first problem (40 iterations, into a scratch solution) and keeps
- * the fastest per iteration; it synchronises the stream, so make it before
- * capturing a graph.  SEMX_BATCH_OP=block|wave|mfma forces one operator
- * (the BF16 batch offers wave and mfma).                                 */
+ * before the first solve) and the host time the batch tuner took (ms).  A
+ * batch whose vectors are held on chip (every problem as in
+ * semx_helm_pcg_info) has one operator, wavefront-level scalar, and no tuner
+ * (0 ms).  For the others the first semx_batch_solve tunes: per class of
+ * problems with the same np and element count it times each operator the
+ * precision allows on the class's first problem (40 iterations, into a
+ * scratch solution) and keeps the fastest per iteration; it synchronises the
+ * stream, so make it before capturing a graph.  SEMX_BATCH_OP=block|wave|mfma
+ * forces one operator (the BF16 batch offers wave and mfma), and with it the
+ * kernel that is not on chip.                                              */
 int semx_batch_info (semx_batch batch, int* opk, double* tune_ms);
 int semx_batch_solve (semx_batch batch, const double* const* f,
                       const double* const* bc, double* const* u, double tol_rel,

@@ -300,7 +300,8 @@ class Batch:
 
     def info(self):
         """(element operator per problem -- 'block', 'wave' or 'mfma', None
-        before the first solve -- and the tuner's host time in ms)."""
+        before the first solve -- and the tuner's host time in ms, 0 for a
+        batch held on chip, which has the one operator 'wave')."""
         n = len(self.systems)
         opk = np.zeros(n, dtype=np.int32)
         ms = C.c_double(0.0)

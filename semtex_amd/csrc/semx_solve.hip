@@ -3716,7 +3716,7 @@ int semx_helm_solve_fields(semx_helm helm, int nfield, double* const* f, const d
 struct semx_batch_s {
   std::vector<semx_helm> helms;
   std::vector<PcgInst> hinst;      // host copy of inst
-  bool tuned = false;              // element operators chosen
+  bool tuned = false;              // element operators chosen (on chip: solved once)
   double tune_ms = 0.0;            // host time the choice took
   PcgInst* inst = nullptr;         // device, one per problem
   double* work = nullptr;
@@ -3883,7 +3883,6 @@ static int batch_chip_setup(semx_batch_s* b) {
   b->nexch = nex; b->nred = nrd;
   b->lds = lds;
   b->chip = true;
-  b->tuned = true;
   return batch_chip_order(b, its);
 }
 
@@ -4086,6 +4085,7 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
     ca.bf = b.ptrs; ca.bbc = b.ptrs + b.count; ca.bu = (double* const*)(b.ptrs + 2 * b.count);
     if (const int st = chip_launch(ca, 0, b.prec != SEMX_PCG_FP64, b.nwg, b.lds, b.nexch, b.nred, s))
       return st;
+    b.tuned = true;
   }
   PcgBatchArgs a;
   a.wmap = b.wmap; a.pctr = b.pctr; a.pslot = b.pslot; a.err = b.err;
@@ -4160,7 +4160,8 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
 int semx_batch_info(semx_batch batch, int* opk, double* tune_ms) {
   if (!batch) return SEMX_E_ARG;
   if (opk)
-    for (int i = 0; i < batch->count; ++i) opk[i] = batch->tuned ? batch->hinst[i].opk : -1;
+    for (int i = 0; i < batch->count; ++i)
+      opk[i] = !batch->tuned ? -1 : batch->chip ? OPK_WAVE : batch->hinst[i].opk;
   if (tune_ms) *tune_ms = batch->tune_ms;
   return SEMX_OK;
 }
