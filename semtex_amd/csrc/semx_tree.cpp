@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <numeric>
 #include <thread>
@@ -280,11 +281,13 @@ void tree_plan(Helm& H) {
       // children: descendants at depth p, or elements above it; an already
       // passed-through region keeps the child it stands for
       std::vector<int> ch, st{t};
+      std::vector<char> merge;
       while (!st.empty()) {
         const int q = st.back(); st.pop_back();
+        if (q < 0) { merge.push_back(1); continue; }
         const bool stop = bt[q].l < 0 || (q != t && bt[q].depth >= p);
-        if (stop) { ch.push_back(q); continue; }
-        st.push_back(bt[q].r); st.push_back(bt[q].l);
+        if (stop) { ch.push_back(q); merge.push_back(0); continue; }
+        st.push_back(-1); st.push_back(bt[q].r); st.push_back(bt[q].l);
       }
       for (int q = bt[t].lo; q < bt[t].hi; ++q)
         for (int i = 0; i < next; ++i) {
@@ -294,6 +297,7 @@ void tree_plan(Helm& H) {
       std::vector<int> U, key{-7};
       std::vector<std::vector<int>> src;
       TreeType ty;
+      ty.merge = merge;
       ty.cptr.push_back(0);
       for (int c : ch) {
         const bool leaf = bt[c].l < 0;
@@ -385,47 +389,53 @@ constexpr int FB = 48;    // block size of the triangular steps
 
 typedef double v8d __attribute__((vector_size(64)));
 
-// C (m x n) -= A (m x k) B (k x n)
+// C (m x n) -= A (m x k) B (k x n), in columns of 16 (the last ones through a
+// padded copy of B's) so that a column block of B stays in the L1 cache.
 __attribute__((target_clones("avx512f", "fma", "default")))
 void gemm_sub(int m, int n, int k, const double* __restrict__ A, int lda,
               const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc) {
-  int i = 0;
-  for (; i + 4 <= m; i += 4) {
-    const double *a0 = A + (size_t)i * lda, *a1 = a0 + lda, *a2 = a1 + lda, *a3 = a2 + lda;
-    int j = 0;
-    for (; j + 16 <= n; j += 16) {
-      double* c = C + (size_t)i * ldc + j;
+  for (int j = 0; j < n; j += 16) {
+    const int w = std::min(16, n - j);
+    const double* b = B + j;
+    int sb = ldb;
+    static thread_local std::vector<double> pad;
+    if (w < 16) {
+      pad.assign((size_t)k * 16, 0.0);
+      for (int p = 0; p < k; ++p) memcpy(&pad[(size_t)p * 16], b + (size_t)p * ldb, w * sizeof(double));
+      b = pad.data();
+      sb = 16;
+    }
+    for (int i = 0; i < m; i += 4) {
+      const int h = std::min(4, m - i);
+      const double *a0 = A + (size_t)i * lda, *a1 = h > 1 ? a0 + lda : a0,
+                   *a2 = h > 2 ? a0 + 2 * (size_t)lda : a0, *a3 = h > 3 ? a0 + 3 * (size_t)lda : a0;
       v8d c00 = {}, c01 = {}, c10 = {}, c11 = {}, c20 = {}, c21 = {}, c30 = {}, c31 = {};
       for (int p = 0; p < k; ++p) {
         v8d b0, b1;
-        memcpy(&b0, B + (size_t)p * ldb + j, sizeof b0);
-        memcpy(&b1, B + (size_t)p * ldb + j + 8, sizeof b1);
+        memcpy(&b0, b + (size_t)p * sb, sizeof b0);
+        memcpy(&b1, b + (size_t)p * sb + 8, sizeof b1);
         c00 += a0[p] * b0; c01 += a0[p] * b1;
         c10 += a1[p] * b0; c11 += a1[p] * b1;
         c20 += a2[p] * b0; c21 += a2[p] * b1;
         c30 += a3[p] * b0; c31 += a3[p] * b1;
       }
-      for (int q = 0; q < 8; ++q) {
-        c[q] -= c00[q]; c[q + 8] -= c01[q];
-        c[ldc + q] -= c10[q]; c[ldc + q + 8] -= c11[q];
-        c[2 * (size_t)ldc + q] -= c20[q]; c[2 * (size_t)ldc + q + 8] -= c21[q];
-        c[3 * (size_t)ldc + q] -= c30[q]; c[3 * (size_t)ldc + q + 8] -= c31[q];
+      const v8d t[4][2] = {{c00, c01}, {c10, c11}, {c20, c21}, {c30, c31}};
+      for (int r = 0; r < h; ++r) {
+        double* c = C + (size_t)(i + r) * ldc + j;
+        if (w == 16) {
+          v8d x, y;
+          memcpy(&x, c, sizeof x);
+          memcpy(&y, c + 8, sizeof y);
+          x -= t[r][0];
+          y -= t[r][1];
+          memcpy(c, &x, sizeof x);
+          memcpy(c + 8, &y, sizeof y);
+        } else {
+          for (int q = 0; q < w; ++q) c[q] -= t[r][q >> 3][q & 7];
+        }
       }
     }
-    for (; j < n; ++j)
-      for (int r = 0; r < 4; ++r) {
-        double s = 0.0;
-        for (int p = 0; p < k; ++p) s += A[(size_t)(i + r) * lda + p] * B[(size_t)p * ldb + j];
-        C[(size_t)(i + r) * ldc + j] -= s;
-      }
   }
-  for (; i < m; ++i)
-    for (int p = 0; p < k; ++p) {
-      const double a = A[(size_t)i * lda + p];
-      const double* b = B + (size_t)p * ldb;
-      double* c = C + (size_t)i * ldc;
-      for (int j = 0; j < n; ++j) c[j] -= a * b[j];
-    }
 }
 
 // A^T block (rows r0.., cols c0..) packed row-major: out (cols x rows)
@@ -530,7 +540,7 @@ void chunk_backward(int ni, int i0, const double* LT, double* T) {
   }
 }
 
-struct ElimWork { std::vector<double> U, W, LT, tmp; };
+struct ElimWork { std::vector<double> U, W, LT, tmp; RawDoubles XE, G, Z; };
 
 // fn(i) for i < n on up to nth threads
 template <class F>
@@ -600,18 +610,149 @@ int eliminate(int ni, int nb, ElimWork& E, int nth) {
   return SEMX_OK;
 }
 
-template <class F>
-void pack_matrix(int rows, int cols, double* out, F at) {
-  const int mt = tree_mt(rows), kp = tree_kp(cols);
-  for (int t = 0; t < mt; ++t)
-    for (int k = 0; k < kp; ++k) {
-      double* o = out + ((size_t)t * kp + k) * 128;
-      for (int l = 0; l < 64; ++l)
-        for (int j = 0; j < 2; ++j) {
-          const int r = 16 * t + (l & 15), c = 8 * k + 4 * j + (l >> 4);
-          o[2 * l + j] = (r < rows && c < cols) ? at(r, c) : 0.0;
-        }
+// A part of a region: its eliminated unknowns I and boundary unknowns B (the
+// region's numbers; cnt: how many of the region's child entries each of B
+// stands for), A_II^-1, X = A_II^-1 A_IB and the Schur complement on B.
+struct Part {
+  std::vector<int> I, B, cnt;
+  RawDoubles inv, X;
+  std::vector<double> S;
+};
+
+// Two parts (or one alone) merged: the unknowns that no other part holds are
+// eliminated.  With e of them, n eliminated before and the parts' matrices,
+//   A_EE^-1, Y = A_EE^-1 A_EB, S = A_BB - A_BE Y          (eliminate)
+//   X   = [X_B - X_E Y; Y]
+//   inv = [blockdiag(inv) + X_E A_EE^-1 X_E^T, -X_E A_EE^-1; sym., A_EE^-1]
+// which is n^2 e / 2 multiply-adds for the inverse where a factorisation of
+// the whole region takes (n + e)^3 / 2.  total: entries of each unknown; pin:
+// the unknown to drop (-1: none); pos: scratch, -1 everywhere.
+int merge_parts(Part* a, Part* b, int nelim, const std::vector<int>& total, int pin,
+                std::vector<int>& pos, ElimWork& E, int nth, Part& out) {
+  Part* parts[2] = {a, b};
+  const int np = b ? 2 : 1;
+  std::vector<int> U, cnt;
+  for (int k = 0; k < np; ++k)
+    for (size_t i = 0; i < parts[k]->B.size(); ++i) {
+      const int u = parts[k]->B[i];
+      if (pos[u] < 0) { pos[u] = (int)U.size(); U.push_back(u); cnt.push_back(0); }
+      cnt[pos[u]] += parts[k]->cnt[i];
     }
+  std::vector<int> el;
+  for (size_t i = 0; i < U.size(); ++i) {
+    if (U[i] < nelim && cnt[i] == total[U[i]]) el.push_back(U[i]);
+    else { out.B.push_back(U[i]); out.cnt.push_back(cnt[i]); }
+  }
+  const int e = (int)el.size(), nb = (int)out.B.size(), nu = e + nb;
+  for (int i = 0; i < e; ++i) pos[el[i]] = i;
+  for (int i = 0; i < nb; ++i) pos[out.B[i]] = e + i;
+  E.U.assign((size_t)nu * nu, 0.0);
+  for (int k = 0; k < np; ++k) {
+    const Part& q = *parts[k];
+    const int m = (int)q.B.size();
+    for (int i = 0; i < m; ++i) {
+      double* row = &E.U[(size_t)pos[q.B[i]] * nu];
+      for (int j = 0; j < m; ++j) row[pos[q.B[j]]] += q.S[(size_t)i * m + j];
+    }
+  }
+  // the pinned node of a singular mode is dropped (src/matrix.cpp:167-169):
+  // decoupled here, its rows and columns of the results zeroed below
+  const int ip = pin >= 0 && pos[pin] >= 0 && pos[pin] < e ? pos[pin] : -1;
+  if (ip >= 0) {
+    for (int k = 0; k < nu; ++k) E.U[(size_t)ip * nu + k] = E.U[(size_t)k * nu + ip] = 0.0;
+    E.U[(size_t)ip * nu + ip] = 1.0;
+  }
+  if (e)
+    if (const int st = eliminate(e, nb, E, nth)) return st;
+  const double* W = E.W.data();
+  if (ip >= 0) {
+    for (int k = 0; k < nu; ++k) E.W[(size_t)ip * nu + k] = 0.0;
+    for (int r = 0; r < e; ++r) E.W[(size_t)r * nu + nb + ip] = 0.0;
+  }
+  out.S.resize((size_t)nb * nb);
+  for (int r = 0; r < nb; ++r)
+    std::copy_n(&E.U[(size_t)(e + r) * nu + e], nb, &out.S[(size_t)r * nb]);
+  int n = 0;
+  for (int k = 0; k < np; ++k) n += (int)parts[k]->I.size();
+  const int ni = n + e;
+  out.inv.resize((size_t)ni * ni);
+  out.X.resize((size_t)ni * nb);
+  E.XE.resize((size_t)n * e);
+  if ((long long)n * (ni + e) < 200000) nth = 1;
+  const int split = np > 1 ? (int)a->I.size() : n;
+  for (int k = 0; k < np; ++k) out.I.insert(out.I.end(), parts[k]->I.begin(), parts[k]->I.end());
+  out.I.insert(out.I.end(), el.begin(), el.end());
+  std::vector<int> col[2];
+  for (int k = 0; k < np; ++k)
+    for (int u : parts[k]->B) col[k].push_back(pos[u]);
+  for (int u : U) pos[u] = -1;
+  // the parts' rows: their inverses with zeros to their right, their X split
+  // into the eliminated and the other columns
+  const int nblk = (n + FC - 1) / FC;
+  spread(nblk, nth, [&](int j) {
+    for (int r = j * FC; r < std::min((j + 1) * FC, n); ++r) {
+      const int k = r >= split, r0 = k ? split : 0;
+      const Part& q = *parts[k];
+      const int m = (int)q.I.size(), mb = (int)q.B.size();
+      double* v = &out.inv[(size_t)r * ni];
+      std::copy_n(&q.inv[(size_t)(r - r0) * m], m, v + r0);
+      std::fill(v + r0 + m, v + n, 0.0);
+      const double* x = q.X.data() + (size_t)(r - r0) * mb;
+      double *xe = E.XE.data() + (size_t)r * e, *xb = out.X.data() + (size_t)r * nb;
+      std::fill_n(xe, e, 0.0);
+      std::fill_n(xb, nb, 0.0);
+      for (int c = 0; c < mb; ++c) {
+        const int at = col[k][c];
+        (at < e ? xe[at] : xb[at - e]) = x[c];
+      }
+    }
+  });
+  if (e) {
+    E.G.resize((size_t)n * e);
+    E.Z.resize((size_t)n * e);
+    pack_t(E.XE.data(), e, n, e, E.Z.data());      // e x n
+    spread(nblk, nth, [&](int j) {
+      const int s = j * FC, m = std::min(FC, n - s);
+      const double* x = &E.XE[(size_t)s * e];
+      double* g = &E.G[(size_t)s * e];
+      std::fill_n(g, (size_t)m * e, 0.0);
+      gemm_sub(m, nb, e, x, e, W, nu, out.X.data() + (size_t)s * nb, nb);
+      gemm_sub(m, e, e, x, e, W + nb, nu, g, e);
+      gemm_sub(m, n - s, e, g, e, &E.Z[s], n, &out.inv[(size_t)s * ni + s], ni);
+      for (int r = s; r < s + m; ++r) std::copy_n(&E.G[(size_t)r * e], e, &out.inv[(size_t)r * ni + n]);
+    });
+    for (int r = 0; r < e; ++r) {
+      std::copy_n(W + (size_t)r * nu, nb, out.X.data() + (size_t)(n + r) * nb);
+      std::copy_n(W + (size_t)r * nu + nb, e, &out.inv[(size_t)(n + r) * ni + n]);
+    }
+  }
+  // the rows below the diagonal: mirrored, by blocks
+  spread((ni + 31) / 32, nth, [&](int b) {
+    const int i = 32 * b;
+    for (int j = 0; j <= i; j += 32)
+      for (int r = i; r < std::min(i + 32, ni); ++r)
+        for (int c = j; c < std::min(j + 32, r); ++c)
+          out.inv[(size_t)r * ni + c] = out.inv[(size_t)c * ni + r];
+  });
+  return SEMX_OK;
+}
+
+// Packs a matrix of which row(r, buf) writes row r.
+template <class F>
+void pack_matrix(int rows, int cols, double* out, int nth, F row) {
+  const int mt = tree_mt(rows), kp = tree_kp(cols);
+  if ((long long)rows * cols < 100000) nth = 1;
+  spread(mt, nth, [&](int t) {
+    std::vector<double> buf((size_t)16 * kp * 8, 0.0);
+    for (int r = 16 * t; r < std::min(16 * t + 16, rows); ++r) row(r, &buf[(size_t)(r - 16 * t) * kp * 8]);
+    double* o = out + (size_t)t * kp * 128;
+    for (int k = 0; k < kp; ++k, o += 128)
+      for (int l = 0; l < 64; ++l) {
+        const double* b = &buf[(size_t)(l & 15) * kp * 8 + 8 * k + (l >> 4)];
+        o[2 * l] = b[0];
+        o[2 * l + 1] = b[4];
+      }
+  });
 }
 
 }  // namespace
@@ -623,7 +764,7 @@ int tree_factor(Helm& H) {
   std::vector<int> dm;
   for (int m = 0; m < H.nmodes; ++m) if (H.modes[m].kind == SEMX_DIRECT) dm.push_back(m);
   const int nd = (int)dm.size(), nt = (int)T.type.size();
-  T.mat.assign((size_t)nd * T.mstride, 0.0);
+  T.mat.resize((size_t)nd * T.mstride);   // packed whole below
   std::vector<std::vector<double>> S((size_t)nd * nt);
   // how many types of later stages still read a type's S
   std::vector<std::atomic<int>> uses((size_t)nd * nt);
@@ -633,50 +774,93 @@ int tree_factor(Helm& H) {
       if (c >= 0) for (int i = 0; i < nd; ++i) uses[(size_t)i * nt + c]++;
   std::atomic<int> status{SEMX_OK};
   auto work = [&](int im, int t, ElimWork& E, int nth) {
-    std::vector<double>&U = E.U, &W = E.W;
     const TreeType& ty = T.type[t];
     const int m = dm[im], ni = ty.ni, nb = ty.nb, nu = ni + nb;
-    U.assign((size_t)nu * nu, 0.0);
-    for (size_t c = 0; c < ty.child.size(); ++c) {
-      const int id = ty.child[c], n = ty.cptr[c + 1] - ty.cptr[c];
-      const int* mp = &ty.cmap[ty.cptr[c]];
-      if (id < 0) {
-        const TreeLeaf& L = T.leaf[-1 - id];
-        const double* hbb = &H.hbb[((size_t)m * nset + L.set) * next * next];
-        for (int i = 0; i < n; ++i)
-          for (int k = 0; k < n; ++k)
-            U[(size_t)mp[i] * nu + mp[k]] += hbb[(size_t)L.loc[i] * next + L.loc[k]];
-      } else {
-        const std::vector<double>& s = S[(size_t)im * nt + id];
-        for (int i = 0; i < n; ++i)
-          for (int k = 0; k < n; ++k) U[(size_t)mp[i] * nu + mp[k]] += s[(size_t)i * n + k];
-        if (--uses[(size_t)im * nt + id] == 0) std::vector<double>().swap(S[(size_t)im * nt + id]);
+    std::vector<int> total(nu, 0), pos(nu, -1);
+    for (int u : ty.cmap) total[u]++;
+    const int pin = H.modes[m].singular ? ty.pin : -1;
+    // merge by merge, as the bisection did: parts in the order the children
+    // come in, the halves of a large region on threads of their own
+    struct Half { int child, l, r, size; };
+    std::vector<Half> half;
+    {
+      std::vector<int> st;
+      int c = 0;
+      for (char op : ty.merge) {
+        if (!op) {
+          half.push_back({c++, -1, -1, 1});
+        } else {
+          const int r = st.back(), l = st[st.size() - 2];
+          st.resize(st.size() - 2);
+          half.push_back({-1, l, r, half[l].size + half[r].size});
+        }
+        st.push_back((int)half.size() - 1);
       }
     }
-    // the pinned node of a singular mode is dropped (src/matrix.cpp:167-169):
-    // decoupled here, its rows and columns of the results zeroed below
-    const int pin = H.modes[m].singular ? ty.pin : -1;
-    if (pin >= 0) {
-      for (int k = 0; k < nu; ++k) U[(size_t)pin * nu + k] = U[(size_t)k * nu + pin] = 0.0;
-      U[(size_t)pin * nu + pin] = 1.0;
+    std::function<int(int, int, ElimWork&, std::vector<int>&, Part&)> build =
+        [&](int h, int threads, ElimWork& W, std::vector<int>& pos, Part& out) {
+      const Half& q = half[h];
+      if (q.child >= 0) {
+        const int id = ty.child[q.child], n = ty.cptr[q.child + 1] - ty.cptr[q.child];
+        const int* mp = &ty.cmap[ty.cptr[q.child]];
+        out.B.assign(mp, mp + n);
+        out.cnt.assign(n, 1);
+        if (id < 0) {
+          const TreeLeaf& L = T.leaf[-1 - id];
+          const double* hbb = &H.hbb[((size_t)m * nset + L.set) * next * next];
+          out.S.resize((size_t)n * n);
+          for (int i = 0; i < n; ++i)
+            for (int k = 0; k < n; ++k) out.S[(size_t)i * n + k] = hbb[(size_t)L.loc[i] * next + L.loc[k]];
+        } else {
+          std::vector<double>& s = S[(size_t)im * nt + id];
+          out.S = s;
+          if (--uses[(size_t)im * nt + id] == 0) std::vector<double>().swap(s);
+        }
+        return SEMX_OK;
+      }
+      Part l, r;
+      int sl = SEMX_OK, sr;
+      if (threads > 1 && q.size >= 16) {
+        std::thread left([&]() {
+          ElimWork Wl;
+          std::vector<int> pl(nu, -1);
+          sl = build(q.l, threads / 2, Wl, pl, l);
+        });
+        sr = build(q.r, threads - threads / 2, W, pos, r);
+        left.join();
+      } else {
+        sl = build(q.l, threads, W, pos, l);
+        sr = build(q.r, threads, W, pos, r);
+      }
+      if (sl || sr) return sl ? sl : sr;
+      return merge_parts(&l, &r, ni, total, pin, pos, W, threads, out);
+    };
+    Part R;
+    int fail = build((int)half.size() - 1, nth, E, pos, R);
+    if (!fail && half.size() == 1) {
+      Part one;
+      std::swap(one, R);
+      fail = merge_parts(&one, nullptr, ni, total, pin, pos, E, nth, R);
     }
-    if (eliminate(ni, nb, E, nth)) { status = SEMX_E_NOT_SPD; return; }
-    const int ldw = nu;
-    if (pin >= 0) {
-      for (int k = 0; k < ldw; ++k) W[(size_t)pin * ldw + k] = 0.0;
-      for (int r = 0; r < ni; ++r) W[(size_t)r * ldw + nb + pin] = 0.0;
-    }
-    // forward: -X (nb x ni); backward: [inv | -X^T] (ni x (ni + nb))
+    if (fail) { status = SEMX_E_NOT_SPD; return; }
+    std::vector<int> pi(ni), pb(nb);        // the region's numbers -> rows and columns
+    for (int i = 0; i < ni; ++i) pi[R.I[i]] = i;
+    for (int i = 0; i < nb; ++i) pb[R.B[i] - ni] = i;
+    // forward: -X^T (nb x ni); backward: [inv | -X] (ni x (ni + nb))
     double* out = &T.mat[(size_t)im * T.mstride];
-    pack_matrix(nb, ni, out + ty.off_f, [&](int r, int c) { return -W[(size_t)c * ldw + r]; });
-    pack_matrix(ni, nu, out + ty.off_b, [&](int r, int c) {
-      return c < ni ? W[(size_t)r * ldw + nb + c] : -W[(size_t)r * ldw + c - ni];
+    pack_matrix(nb, ni, out + ty.off_f, nth, [&](int r, double* o) {
+      for (int q = 0; q < ni; ++q) o[q] = -R.X[(size_t)pi[q] * nb + pb[r]];
+    });
+    pack_matrix(ni, nu, out + ty.off_b, nth, [&](int r, double* o) {
+      const double *v = &R.inv[(size_t)pi[r] * ni], *x = R.X.data() + (size_t)pi[r] * nb;
+      for (int q = 0; q < ni; ++q) o[q] = v[pi[q]];
+      for (int q = 0; q < nb; ++q) o[ni + q] = -x[pb[q]];
     });
     if (nb) {
       std::vector<double>& s = S[(size_t)im * nt + t];
       s.resize((size_t)nb * nb);
       for (int r = 0; r < nb; ++r)
-        memcpy(&s[(size_t)r * nb], &U[(size_t)(ni + r) * nu + ni], nb * sizeof(double));
+        for (int k = 0; k < nb; ++k) s[(size_t)r * nb + k] = R.S[(size_t)pb[r] * nb + pb[k]];
     }
   };
   // types of a stage are independent of each other
@@ -686,11 +870,11 @@ int tree_factor(Helm& H) {
     for (int t = 0; t < nt; ++t) if (T.type[t].stage == st) list.push_back(t);
     const int total = (int)list.size() * nd;
     std::atomic<int> nextj{0};
-    // one worker per region and mode at a time; few of them share the threads
-    const int n = std::min(nth, total), inner = n ? std::max(1, nth / n) : 1;
-    spread(n, n, [&](int) {
+    // one worker per region and mode at a time; the last of them share the threads
+    spread(std::min(nth, total), nth, [&](int) {
       ElimWork E;
-      for (int j; (j = nextj++) < total && status == SEMX_OK;) work(j % nd, list[j / nd], E, inner);
+      for (int j; (j = nextj++) < total && status == SEMX_OK;)
+        work(j % nd, list[j / nd], E, std::max(1, nth / (total - j)));
     });
   }
   return status;

@@ -7,11 +7,22 @@
 // recovers its eliminated unknowns from its boundary values).
 #pragma once
 
+#include <memory>
 #include <vector>
 
 namespace semx {
 
 struct Helm;
+
+// Doubles that a resize leaves as they are: large matrices are written whole,
+// by the threads that compute them, and would only be touched twice.
+template <class T>
+struct NoInit : std::allocator<T> {
+  template <class U> struct rebind { typedef NoInit<U> other; };
+  template <class U> void construct(U*) noexcept {}
+  template <class U, class V> void construct(U* p, const V& v) { *p = v; }
+};
+typedef std::vector<double, NoInit<double>> RawDoubles;
 
 // A region type: regions built the same way from the same child types
 // share their matrices (translated copies on uniform meshes).
@@ -20,6 +31,8 @@ struct TreeType {
   int ni = 0, nb = 0;            // eliminated unknowns, boundary unknowns
   int pin = -1;                  // eliminated unknown that a singular mode pins
   std::vector<int> child;        // child types; -1-l: leaf (element) type l
+  std::vector<char> merge;       // how the bisection merges them: 0 the next child,
+                                 // 1 the last two parts
   std::vector<int> cptr, cmap;   // child's boundary entry -> unknown (0..ni+nb)
   long long off_f = 0, off_b = 0;  // packed matrices within a mode's block
 };
@@ -47,7 +60,7 @@ struct Tree {
   std::vector<int> rowptr, src;  // contributions to each: element-boundary slots
                                  // [0, nel*next), then child slots from there on
   long long mstride = 0;         // doubles per direct mode
-  std::vector<double> mat;       // direct modes' packed matrices, released on upload
+  RawDoubles mat;                // direct modes' packed matrices, released on upload
 };
 
 // A matrix (rows x cols) in the order the matrix cores take it: 16-row

@@ -268,7 +268,7 @@ int tree_upload(Helm& H) {
   if ((st = dev_upload(&D->gid, T.gid.data(), T.gid.size()))) return st;
   if ((st = dev_upload(&D->rowptr, T.rowptr.data(), T.rowptr.size()))) return st;
   if ((st = dev_upload(&D->src, T.src.data(), T.src.size()))) return st;
-  std::vector<double>().swap(T.mat);
+  RawDoubles().swap(T.mat);
   return SEMX_OK;
 }
 
