@@ -74,7 +74,7 @@ constexpr int END_FEW = 2;      // the same for groups of at most 2 columns a wa
 
 struct EndArgs {
   int np, npnp, next, nint, nel, planeSize, nline, nsolve, nplanes, nset, nbe, ld, npl, nrhs;
-  int solstride;
+  int solstride, ngrp, lds;         // lds: doubles of a group (W = 1)
   const int4* grp;
   const int* elist;
   const int* bidx;
@@ -120,6 +120,18 @@ struct EndCols {
             __builtin_amdgcn_readlane(ib, c)};
   }
 };
+
+// LDS order within a group of W wavefronts
+template <int W>
+__device__ inline void end_sync() {
+  if constexpr (W > 1) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
 
 __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
@@ -259,11 +271,16 @@ __global__ __launch_bounds__(ET) void k_force(EndArgs a, const int* __restrict__
 
 // A wavefront brings in whole columns (NJ nodes per lane, EU columns in
 // flight; the column's field, plane and element sit in scalar registers).
-template <int CT, int NJ, int EU>
+// A group is worked on by W wavefronts: the workgroup's, or one of them (see
+// end_launch).
+template <int CT, int NJ, int EU, int W>
 __global__ __launch_bounds__(ET) void k_cond(EndArgs a) {
-  extern __shared__ double vs[];
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int4 g = a.grp[blockIdx.x];
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, wave = W > 1 ? wave_id() : 0;
+  const int gi = W > 1 ? blockIdx.x : blockIdx.x * EW + wave_id();
+  if (W == 1 && gi >= a.ngrp) return;
+  double* vs = lds + (W > 1 ? 0 : wave_id() * a.lds);
+  const int4 g = a.grp[gi];
   const int im = blockIdx.y, m = a.dmode[im];
   const EndCols cols(a, m, g);
   const int npnp = a.npnp, next = a.next, ld = a.ld, N = g.y * a.nrhs;
@@ -279,20 +296,20 @@ __global__ __launch_bounds__(ET) void k_cond(EndArgs a) {
     q4[j] = -a.G[((size_t)set * G_N + G_Q4) * npnp + pt[j]];
     b[j] = a.pmap[pt[j]];
   }
-  for (int c0 = wave; c0 < N; c0 += EW * EU) {
+  for (int c0 = wave; c0 < N; c0 += W * EU) {
     // loads without a condition (lanes past the last node repeat it), so
     // that all of them are in flight together
     double f[EU][NJ], l[EU][NJ];
 #pragma unroll
     for (int u = 0; u < EU; ++u) {
-      const EndCols::Col q = cols.col(min(c0 + u * EW, N - 1));
+      const EndCols::Col q = cols.col(min(c0 + u * W, N - 1));
       const double* fp = a.f[q.fld] + (size_t)q.k * a.planeSize + (size_t)q.e * npnp;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) f[u][j] = fp[pt[j]];
     }
 #pragma unroll
     for (int u = 0; u < EU; ++u) {
-      const EndCols::Col q = cols.col(min(c0 + u * EW, N - 1));
+      const EndCols::Col q = cols.col(min(c0 + u * W, N - 1));
       const double* lp = a.L + q.fld * a.LF + ((size_t)q.p * a.nbe + q.ib) * npnp;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) l[u][j] = 0.0;
@@ -302,17 +319,17 @@ __global__ __launch_bounds__(ET) void k_cond(EndArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < EU; ++u)
-      if (c0 + u * EW < N) {
-        const bool on = cols.col(c0 + u * EW).p >= 0;
+      if (c0 + u * W < N) {
+        const bool on = cols.col(c0 + u * W).p >= 0;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
           if (lane + 64 * j < npnp)
-            vs[(c0 + u * EW) * ld + b[j]] = on ? q4[j] * f[u][j] + l[u][j] : 0.0;
-        if (lane < ld - npnp) vs[(c0 + u * EW) * ld + npnp + lane] = 0.0;
+            vs[(c0 + u * W) * ld + b[j]] = on ? q4[j] * f[u][j] + l[u][j] : 0.0;
+        if (lane < ld - npnp) vs[(c0 + u * W) * ld + npnp + lane] = 0.0;
       }
   }
-  __syncthreads();
-  for (int t = wave; t < MT * npair; t += EW) {
+  end_sync<W>();
+  for (int t = wave; t < MT * npair; t += W) {
     const int rt = t / npair, c0 = (t - rt * npair) * CT * 16;
     elem_d4 acc[CT];
     end_product<CT>(mat, rt, KP, vs + next, ld, c0, N, acc);
@@ -327,19 +344,22 @@ __global__ __launch_bounds__(ET) void k_cond(EndArgs a) {
       }
     }
   }
-  __syncthreads();
-  for (int c = wave; c < N; c += EW) {
+  end_sync<W>();
+  for (int c = wave; c < N; c += W) {
     const EndCols::Col q = cols.col(c);
     if (q.p >= 0 && lane < next)
       a.Fb[q.fld * a.FbF + ((size_t)q.p * a.nel + q.e) * next + lane] = vs[c * ld + lane];
   }
 }
 
-template <int CT, int NJ, int EU>
+template <int CT, int NJ, int EU, int W>
 __global__ __launch_bounds__(ET) void k_back(EndArgs a) {
-  extern __shared__ double vs[];
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int4 g = a.grp[blockIdx.x];
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, wave = W > 1 ? wave_id() : 0;
+  const int gi = W > 1 ? blockIdx.x : blockIdx.x * EW + wave_id();
+  if (W == 1 && gi >= a.ngrp) return;
+  double* vs = lds + (W > 1 ? 0 : wave_id() * a.lds);
+  const int4 g = a.grp[gi];
   const int im = blockIdx.y, m = a.dmode[im], n = a.mode_n[m];
   const EndCols cols(a, m, g);
   const int npnp = a.npnp, next = a.next, ld = a.ld, N = g.y * a.nrhs;
@@ -355,14 +375,14 @@ __global__ __launch_bounds__(ET) void k_back(EndArgs a) {
     q4[j] = -a.G[((size_t)set * G_N + G_Q4) * npnp + pt[j]];
     b[j] = a.pmap[pt[j]];
   }
-  for (int c0 = wave; c0 < N; c0 += EW * EU) {
+  for (int c0 = wave; c0 < N; c0 += W * EU) {
     double f[EU][NJ], v[EU][NJ];
     int gid[EU][NJ];
     // forcing and node numbers, then the solved values of boundary nodes (a
     // pinned node holds zero); loads without a condition, see k_cond
 #pragma unroll
     for (int u = 0; u < EU; ++u) {
-      const EndCols::Col q = cols.col(min(c0 + u * EW, N - 1));
+      const EndCols::Col q = cols.col(min(c0 + u * W, N - 1));
       const double* fp = a.f[q.fld] + (size_t)q.k * a.planeSize + (size_t)q.e * npnp;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
@@ -372,32 +392,32 @@ __global__ __launch_bounds__(ET) void k_back(EndArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < EU; ++u) {
-      const EndCols::Col q = cols.col(min(c0 + u * EW, N - 1));
+      const EndCols::Col q = cols.col(min(c0 + u * W, N - 1));
       const double* sp = a.sol + q.fld * a.solF + (size_t)max(q.p, 0) * a.solstride;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) v[u][j] = sp[gid[u][j] < n ? gid[u][j] : 0];
     }
 #pragma unroll
     for (int u = 0; u < EU; ++u)
-      if (c0 + u * EW < N) {
-        const EndCols::Col q = cols.col(c0 + u * EW);
+      if (c0 + u * W < N) {
+        const EndCols::Col q = cols.col(c0 + u * W);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           if (gid[u][j] >= n) v[u][j] = 0.0;
           if (q.ib >= 0 && gid[u][j] >= a.nsolve)
             v[u][j] = a.bc[q.fld][(size_t)q.k * a.nline + a.ess_src[gid[u][j] - a.nsolve]];
           if (b[j] >= next) v[u][j] = q4[j] * f[u][j];
-          if (lane + 64 * j < npnp) vs[(c0 + u * EW) * ld + b[j]] = q.p >= 0 ? v[u][j] : 0.0;
+          if (lane + 64 * j < npnp) vs[(c0 + u * W) * ld + b[j]] = q.p >= 0 ? v[u][j] : 0.0;
         }
-        if (lane < ld - npnp) vs[(c0 + u * EW) * ld + npnp + lane] = 0.0;
+        if (lane < ld - npnp) vs[(c0 + u * W) * ld + npnp + lane] = 0.0;
       }
   }
-  __syncthreads();
+  end_sync<W>();
   const int lo = a.nint | 1;
   // the products read the interior values of every row tile: results go to
   // the part of LDS after the columns
   double* out = vs + (size_t)N * ld;
-  for (int t = wave; t < MT * npair; t += EW) {
+  for (int t = wave; t < MT * npair; t += W) {
     const int rt = t / npair, c0 = (t - rt * npair) * CT * 16;
     elem_d4 acc[CT];
     end_product<CT>(mat, rt, KP, vs, ld, c0, N, acc);
@@ -411,8 +431,8 @@ __global__ __launch_bounds__(ET) void k_back(EndArgs a) {
       }
     }
   }
-  __syncthreads();
-  for (int c = wave; c < N; c += EW) {
+  end_sync<W>();
+  for (int c = wave; c < N; c += W) {
     const EndCols::Col q = cols.col(c);
     if (q.p < 0) continue;
     double* up = a.u[q.fld] + (size_t)q.k * a.planeSize + (size_t)q.e * npnp;
@@ -420,6 +440,46 @@ __global__ __launch_bounds__(ET) void k_back(EndArgs a) {
     for (int j = 0; j < NJ; ++j)
       if (lane + 64 * j < npnp)
         up[lane + 64 * j] = b[j] < next ? vs[c * ld + b[j]] : out[c * lo + (b[j] - next)];
+  }
+}
+
+// np = 3: eight boundary nodes and one interior one, a thread per node and
+// right-hand side; the same matrices.
+template <bool BACK>
+__global__ __launch_bounds__(ET) void k_end3(EndArgs a) {
+  const int idx = blockIdx.x * ET + threadIdx.x;
+  if (idx >= a.nel * 9) return;
+  const int e = idx / 9, pt = idx - 9 * e, im = blockIdx.y, m = a.dmode[im];
+  const int fld = blockIdx.z / a.npl, p = a.mode_plane[2 * m + blockIdx.z % a.npl];
+  if (p < 0) return;
+  const int k = a.plane_of[p], b = a.pmap[pt], set = a.eset[e], ib = a.bidx[e];
+  const double* q4 = a.G + ((size_t)set * G_N + G_Q4) * 9;
+  const double* f = a.f[fld] + (size_t)k * a.planeSize + (size_t)e * 9;
+  const double fi = -(q4[4] * f[4]);               // the interior node
+  if constexpr (!BACK) {
+    if (b == 8) return;
+    const double* L = a.L + fld * a.LF + ((size_t)p * a.nbe + max(ib, 0)) * 9;
+    const double lb = ib >= 0 ? L[b] : 0.0, li = ib >= 0 ? L[8] : 0.0;
+    const double h = a.mat[((size_t)im * a.nset + set) * 128 + 2 * b];
+    a.Fb[fld * a.FbF + ((size_t)p * a.nel + e) * 8 + b] = (lb - q4[pt] * f[pt]) - h * (fi + li);
+  } else {
+    const int n = a.mode_n[m];
+    const double* sol = a.sol + fld * a.solF + (size_t)p * a.solstride;
+    const double* bc = a.bc[fld] + (size_t)k * a.nline;
+    auto node = [&](int c) {                       // a pinned one holds zero
+      const int gid = a.btog[e * 8 + c];
+      return gid < n ? sol[gid] : gid >= a.nsolve ? bc[a.ess_src[gid - a.nsolve]] : 0.0;
+    };
+    double v = 0.0;
+    if (b < 8) {
+      v = node(b);
+    } else {
+      const double* A = a.mat + ((size_t)im * a.nset + set) * 256;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v += A[32 * (c & 3) + (c >> 2)] * node(c);
+      v += A[128] * fi;
+    }
+    a.u[fld][(size_t)k * a.planeSize + (size_t)e * 9 + pt] = v;
   }
 }
 
@@ -449,24 +509,53 @@ __global__ void k_end_pack(const double* __restrict__ hbi, const double* __restr
   }
 }
 
-// The kernel for npnp nodes, groups of ncol columns and a matrix of mt row
-// tiles.  Two column tiles per product (each matrix operand used twice) where
-// that leaves no wavefront with more work than single tiles would; few
+// k_cond or k_back for npnp nodes, groups of ncol columns and a matrix of mt
+// row tiles.  Two column tiles per product (each matrix operand used twice)
+// where that leaves no wavefront with more work than single tiles would; few
 // columns (elements of their own geometry) load no repeats of them.
 const void* end_kernel(bool back, int ncol, int mt, int npnp) {
   int ct = ncol > 16 ? 2 : 1;
   if (2 * ((mt + EW - 1) / EW) > (2 * mt + EW - 1) / EW) ct = 1;
   const void* fn = nullptr;
 #define SEMX_END_PICK(K_, NJ_)                                                              \
-  (ncol <= EW * END_FEW ? (const void*)K_<1, NJ_, END_FEW>                                  \
-   : ct == 1            ? (const void*)K_<1, NJ_, end_cols(NJ_)>                            \
-                        : (const void*)K_<2, NJ_, end_cols(NJ_)>)
+  (ncol <= EW * END_FEW ? (const void*)K_<1, NJ_, END_FEW, EW>                              \
+   : ct == 1            ? (const void*)K_<1, NJ_, end_cols(NJ_), EW>                        \
+                        : (const void*)K_<2, NJ_, end_cols(NJ_), EW>)
 #define SEMX_END(NJ_)                                                                       \
   if ((npnp + 63) / 64 == NJ_) fn = back ? SEMX_END_PICK(k_back, NJ_) : SEMX_END_PICK(k_cond, NJ_)
   SEMX_END(1); SEMX_END(2); SEMX_END(3); SEMX_END(4);
 #undef SEMX_END
 #undef SEMX_END_PICK
   return fn;
+}
+
+// Condensation or recovery of every group and direct mode.  np = 3 takes a
+// thread per node: nine of a wavefront's lanes would work.  np = 4 and 5 with
+// geometries of their own take one wavefront per group, four groups per
+// workgroup: both matrices are one row tile, so three of the workgroup's
+// wavefronts would only load.  Measured, whole solves, us, a workgroup per
+// group -> this (the band sweeps' element kernels, a thread per row): 32x32
+// distorted np=3 Nz=128 420 -> 187 (204), Nz=32 119 -> 72 (98); 16x16
+// distorted np=4 Nz=64 69 -> 54 (64), np=5 82 -> 66 (97); 16x16 uniform np=3
+// Nz=128 59 -> 47 (55).
+int end_launch(bool back, EndArgs& a, const Mesh& M, const ElemList& l, unsigned nd, hipStream_t s) {
+  void* kargs[] = {&a};
+  if (M.np == 3) {
+    const dim3 grid((M.nel * 9 + ET - 1) / ET, nd, a.nrhs);
+    HIPCHK(hipLaunchKernel(back ? (const void*)k_end3<true> : (const void*)k_end3<false>, grid,
+                           dim3(ET), kargs, 0, s));
+    return SEMX_OK;
+  }
+  const bool one = tree_mt(M.next) == 1 && tree_mt(M.nint) == 1 && l.ncol <= 2 * SEMX_MAX_FIELDS;
+  const void* fn = one ? back ? (const void*)k_back<1, 1, END_FEW, 1> : (const void*)k_cond<1, 1, END_FEW, 1>
+                       : end_kernel(back, l.ncol, tree_mt(back ? M.nint : M.next), M.npnp);
+  a.ngrp = l.ngrp;
+  a.lds = l.ncol * (a.ld + (back ? M.nint | 1 : 0));
+  const size_t lds = (size_t)a.lds * (one ? EW : 1) * sizeof(double);
+  if (lds > 64 * 1024)
+    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  HIPCHK(hipLaunchKernel(fn, dim3(one ? (l.ngrp + EW - 1) / EW : l.ngrp, nd), dim3(ET), kargs, lds, s));
+  return SEMX_OK;
 }
 
 }  // namespace
@@ -653,13 +742,8 @@ int elem_condense(Helm& H, int nf, double* const* fs, const double* const* bcs, 
   if (!H.dmode.empty()) {
     const ElemList& l = D.list[nf];
     a.mat = D.cond;
-    const size_t lds = (size_t)l.ncol * a.ld * sizeof(double);
-    const void* fn = end_kernel(false, l.ncol, tree_mt(M.next), M.npnp);
-    if (lds > 64 * 1024)
-      HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    void* kargs[] = {&a};
     prof_begin(s, &ev);
-    HIPCHK(hipLaunchKernel(fn, dim3(l.ngrp, (unsigned)H.dmode.size()), dim3(ET), kargs, lds, s));
+    if (const int st = end_launch(false, a, M, l, (unsigned)H.dmode.size(), s)) return st;
     prof_end(s, "k_condense", ev);
   }
   if (!H.pcg_plane.empty()) {
@@ -680,14 +764,9 @@ int elem_backsub(Helm& H, int nf, double* const* fs, const double* const* bcs, d
   EndArgs a = end_args(H, nf, fs, bcs, us, pFb, pFi, psol);
   const ElemList& l = D.list[nf];
   a.mat = D.back;
-  const void* fn = end_kernel(true, l.ncol, tree_mt(M.nint), M.npnp);
-  const size_t lds = (size_t)l.ncol * (a.ld + (M.nint | 1)) * sizeof(double);
-  if (lds > 64 * 1024)
-    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipEvent_t ev;
-  void* kargs[] = {&a};
   prof_begin(s, &ev);
-  HIPCHK(hipLaunchKernel(fn, dim3(l.ngrp, (unsigned)H.dmode.size()), dim3(ET), kargs, lds, s));
+  if (const int st = end_launch(true, a, M, l, (unsigned)H.dmode.size(), s)) return st;
   prof_end(s, "k_backsub", ev);
   return SEMX_OK;
 }
