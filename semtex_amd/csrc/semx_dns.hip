@@ -1256,10 +1256,9 @@ void extrapolation(int n, double* c) {
 // ===========================================================================
 
 // The buffer roles of the DNS state: which allocation each field of the
-// step uses.  The step permutes them (transform output <-> spare,
-// swapData, the rolled time levels) and returns to a given assignment only
-// after a full cycle of steps (88 steps for N_TIME = 3 with the
-// skew-symmetric terms, 182 with the alternating form).
+// step uses.  The step permutes them (swapData, the rolled time levels) and
+// returns to a given assignment only after a full cycle of steps
+// (rotate_spares).
 struct DnsRoles {
   double* U[3];
   double* P;
@@ -1450,12 +1449,17 @@ void roll(double* lev[3][3], int nord, int ncom) {
   }
 }
 
-// Between steps Us[0], Uf[0], tmp and spare hold nothing; which of those
-// buffers a step takes for what is free.  They are exchanged here (and, for
-// the skew-symmetric form, before the viscous solves) so that the roles recur
-// after 88 steps of that form and 182 of the alternating one at N_TIME = 3:
-// the number of step graphs that programs which capture a full cycle count on.
+// The step's swaps and rolled levels return to one assignment of roles after
+// 2 N_TIME + 1 steps (twice that with the alternating form).  Between steps
+// Us[0], Uf[0], tmp and spare hold nothing; with planes and N_TIME = 3 those are
+// exchanged as well (here and, for the skew-symmetric form, before the viscous
+// solves), so that the roles recur after 88 steps of that form and 182 of the
+// alternating one, the number of step graphs that programs which capture a
+// full cycle count on there.
+bool long_cycle(const semx_dns_s& D) { return D.nz > 2 && D.nord == 3; }
+
 void rotate_spares(semx_dns_s& D) {
+  if (!long_cycle(D)) return;
   if (D.advection == 0) {
     std::swap(D.Uf[0][2], D.tmp);
     std::swap(D.Us[0][0], D.spare);
@@ -1506,7 +1510,7 @@ int dns_step(semx_dns_s& D, hipStream_t s) {
   // systems (JACPCG) while step < N_TIME; iterative ones start from the old
   // velocity, direct ones only leave parts of it in place.
   Helm* V = (D.step < nord) ? D.start[D.step - 1] : D.vel;
-  if (D.advection == 0) {   // spare buffers: see rotate_spares
+  if (D.advection == 0 && long_cycle(D)) {   // spare buffers: see rotate_spares
     std::swap(D.Uf[0][0], D.Uf[0][1]);
     std::swap(D.Uf[0][0], D.spare);
   }
@@ -1565,8 +1569,8 @@ void set_roles(semx_dns_s& D, const DnsRoles& r) {
 }
 
 // A step from a HIP graph.  Start-up steps (order < N_TIME, JACPCG
-// systems) and the first steady step (which runs the band-sweep autotuner
-// and allocates the solve scratch) run eagerly, as do all steps while
+// systems) and the first steady step (which allocates the solve scratch and,
+// where the band sweeps are selected, times them) run eagerly, as do all steps while
 // kernel timing is on.  A steady step whose role assignment has not been
 // met is captured on the library's capture stream (the host state
 // advances as in an eager step), instantiated and launched on the caller's
