@@ -3321,7 +3321,10 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       } else if (env) {
         const std::string v(env);
         if (v != "block" && v != "wave") return SEMX_E_ARG;
+        if (v == "wave" && M.npnp > 64 * PCG_NPT) return SEMX_E_UNSUPPORTED;
         H.pcg_opk = v == "block" ? OPK_BLOCK : OPK_WAVE;
+      } else if (M.npnp > 64 * PCG_NPT) {   // more nodes than a wavefront's lanes hold
+        H.pcg_opk = OPK_BLOCK;
       } else {
         double* scr = nullptr;
         const size_t nu = (size_t)H.nz * M.planeSize;
