@@ -125,8 +125,8 @@ def main():
             sx.solve(msys, tf, tb, tu, tol_rel=tol, iters=False)
         torch.cuda.synchronize()
         prof = {}
-        for name in ("k_ess_gather", "k_condense", "k_assemble", "k_tree", "k_band_solve",
-                     "k_backsub", "k_pcg"):
+        for name in ("k_ess_gather", "k_lift", "k_condense", "k_assemble", "k_tree",
+                     "k_band_solve", "k_backsub", "k_pcg"):
             tot = C.c_double(); cnt = C.c_longlong()
             L.semx_profile_query(name.encode(), C.byref(tot), C.byref(cnt))
             if cnt.value:
@@ -330,11 +330,11 @@ def main():
     print(json.dumps(result), flush=True)
 
 
-# inner-iteration bytes per PCG iteration per plane: s (3 nPlane + 17 npts),
-# the BLAS-1 and gather/scatter traffic of semtex's loop (src/field.cpp:
-# 676-703) with s bytes per vector value (the BF16 operator reads FP32
-# vectors, so s = 4 for it too)
-PCG_VALUE_BYTES = {"fp64": 8, "fp32_refined": 4, "bf16_refined": 4}
+# vector bytes of the inner iteration of k_pcg, which keeps its vectors in
+# memory: s (3 nPlane + 17 npts) per iteration and plane, the BLAS-1 and
+# gather/scatter traffic of semtex's loop (src/field.cpp:676-703) with s = 4
+# (the BF16 operator reads FP32 vectors)
+PCG_VALUE_BYTES = 4
 
 
 def config2_bench(args, torch, sx, L):
@@ -372,7 +372,8 @@ def config2_bench(args, torch, sx, L):
                        "Dirichlet, seeded smooth solutions; MIXED: mode 0 FP64 DIRECT, modes "
                        "1..63 Jacobi-PCG to |r| <= 1e-10 |b|",
            "dof_per_plane": npts, "planes": nplanes, "setup_s": round(t_setup, 2),
-           "bytes_per_iteration_per_plane_formula": "s*(3*nPlane + 17*npts), s = value bytes"}
+           "bytes_per_iteration_per_plane_formula": "4*(3*nPlane + 17*npts), where the vectors "
+                                                    "are in memory (k_pcg)"}
     for label, (prec, itol, mo) in settings.items():
         S.set_pcg(prec, inner_tol=itol, max_outer=mo)
         progress(f"config2 {label}")
@@ -400,13 +401,14 @@ def config2_bench(args, torch, sx, L):
         L.semx_profile_query(b"k_pcg", C.byref(tot), C.byref(cnt))
         L.semx_profile_enable(0)
         pcg_ms = tot.value / max(cnt.value, 1)
-        sb = PCG_VALUE_BYTES[label]
-        byts = float(np.abs(pits).sum()) * sb * (3 * P.nPlane + 17 * npts)
+        where = S.pcg_info()
         out[label] = {"ms_per_step": ms, "value": npts * nplanes / (ms * 1e-3),
                       "iterations_max": it, "iterations_sum": int(np.abs(pits).sum()),
-                      "rel_l2_vs_fp64_pcg_1e-13": err, "k_pcg_ms": pcg_ms,
-                      "k_pcg_inner_bytes": byts,
-                      "k_pcg_inner_gb_s": byts / (pcg_ms * 1e-3) / 1e9}
+                      "rel_l2_vs_fp64_pcg_1e-13": err, "k_pcg_ms": pcg_ms, "pcg": where}
+        if not where["on_chip"]:   # the vectors pass through memory every iteration
+            byts = float(np.abs(pits).sum()) * PCG_VALUE_BYTES * (3 * P.nPlane + 17 * npts)
+            out[label]["k_pcg_inner_bytes"] = byts
+            out[label]["k_pcg_inner_gb_s"] = byts / (pcg_ms * 1e-3) / 1e9
     for label in ("fp32_refined", "bf16_refined"):
         out[label]["speedup_vs_fp64_pcg"] = out["fp64"]["ms_per_step"] / out[label]["ms_per_step"]
     return out
@@ -494,18 +496,18 @@ def batch_bench(args, torch, sx, L):
         "dtype": "f32 inner PCG, f64 refinement",
         "workload": f"{args.batch} independent 2D problems, K x K quads K~U{{4..16}}, "
                     "np~U{5..11}, lambda2~U[0.1,100], seed 4, Dirichlet, Jacobi-PCG to 1e-10, "
-                    "one launch (the largest problems on up to 8 workgroups each, the "
-                    "rest on one)",
+                    "one launch (a problem on the fewest workgroups that hold its vectors)",
         "dof_total": dofs,
         "iterations_max": it32,
         "fp64_pcg_ms_per_step": ms64,
         "fp64_pcg_value": dofs / (ms64 * 1e-3),
         "rel_l2_vs_fp64": rel,
         "speedup_vs_fp64_pcg": ms64 / ms32,
-        "tuner": {"fp64": tuner(B64), "fp32_refined": tuner(B32), "bf16_refined": tuner(B16),
+        "tuner": {"bf16_refined": tuner(B16),
                   "what": "element operator per (np, element count) class chosen by the batch "
-                          "tuner on the first solve (block-wide or wavefront-level scalar, or "
-                          "BF16 matrix cores)"},
+                          "tuner on the first solve (wavefront-level scalar or BF16 matrix "
+                          "cores); the FP64 and FP32 refined batches are held on chip and have "
+                          "one operator"},
         "bf16_refined": {"ms_per_step": ms16, "value": dofs / (ms16 * 1e-3),
                          "iterations_max": it16, "rel_l2_vs_fp64": rel16,
                          "speedup_vs_fp64_pcg": ms64 / ms16,
@@ -550,8 +552,8 @@ def dns_bench(args, torch, sx, L):
     D.run(args.dns_steps, u, v, w, p)
     torch.cuda.synchronize()
     prof = {}
-    for name in ("k_tree", "k_condense", "k_assemble", "k_backsub", "k_dft_z",
-                 "k_grad_xy", "k_grad_nl", "k_grad_z", "k_smooth", "dns_nonlinear"):
+    for name in ("k_tree", "k_lift", "k_condense", "k_backsub", "k_dft_z", "k_grad_nl",
+                 "k_smooth", "k_wave_div", "k_project", "dns_nonlinear"):
         tot = C.c_double(); cnt = C.c_longlong()
         L.semx_profile_query(name.encode(), C.byref(tot), C.byref(cnt))
         if cnt.value:
