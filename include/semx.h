@@ -255,8 +255,8 @@ int semx_helm_iters (semx_helm helm, int* iters, void* stream);
  * the velocity components u, v, w do in semtex (the MatrixSys cache,
  * src/matrix.cpp:85-91, and Solve per component, dns/integrate.cpp:
  * 365-395).  f, bc, u: host arrays of nfield device pointers, each as in
- * semx_helm_solve (bc may be NULL on a mesh without boundaries).  The band
- * factor of each mode is streamed once for all fields' planes.            */
+ * semx_helm_solve (bc may be NULL on a mesh without boundaries).  The
+ * matrices of each mode are read once for all fields' planes.             */
 int semx_helm_solve_fields (semx_helm helm, int nfield, double* const* f,
                             const double* const* bc, double* const* u,
                             double tol_rel, int step_max, int* iters,
@@ -284,9 +284,12 @@ int semx_helm_set_pcg (semx_helm helm, int precision, double inner_tol,
  * are solved together in one launch; the workgroups of a problem do all
  * of Field::solve's JACPCG branch (src/field.cpp:564-725) for its plane:
  * -(M f + H g) + <h,w>, x0 from u, the iteration, essential re-imposition.
- * A problem whose expected cost exceeds the batch's per-CU share gets
- * several workgroups (up to 8; SEMX_BATCH_WG=1: one each), launched first;
- * the rest one workgroup each, largest first.
+ * Where every problem can be held on chip (semx_helm_pcg_info) each takes
+ * the fewest workgroups that hold it, the longest problems first.  Otherwise,
+ * and with SEMX_BATCH_WG or SEMX_BATCH_OP set, a problem whose expected cost
+ * exceeds the batch's per-CU share gets several workgroups (up to 8;
+ * SEMX_BATCH_WG=1: one each), launched first; the rest one workgroup each,
+ * largest first.
  * f, bc, u: host arrays of count device pointers (bc[i] may be NULL when
  * mesh i has no boundary); iters as in semx_helm_solve.  The systems must
  * outlive the batch.                                                      */

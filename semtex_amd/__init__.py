@@ -241,8 +241,8 @@ def helm_check(msys, stream=None):
 
 
 def solve_fields(msys, fs, bcs, us, tol_rel=1e-12, step_max=10000, stream=None, iters=True):
-    """Field::solve for up to 3 fields sharing msys (as u, v, w do): one
-    sweep of each mode's factor for all of them.  Lists of device tensors;
+    """Field::solve for up to 3 fields sharing msys (as u, v, w do): each
+    mode's matrices are read once for all of them.  Lists of device tensors;
     bcs may be None on a mesh without boundaries."""
     import torch
     M = msys.mesh
@@ -269,8 +269,8 @@ def solve_fields(msys, fs, bcs, us, tol_rel=1e-12, step_max=10000, stream=None, 
 
 class Batch:
     """Independent 2D JACPCG problems (systems made with nz=1, nmodes=1,
-    method JACPCG, equal set_pcg settings) solved in one launch, one
-    workgroup per problem."""
+    method JACPCG, equal set_pcg settings) solved in one launch, one or
+    several workgroups per problem."""
 
     def __init__(self, systems):
         self.systems = list(systems)

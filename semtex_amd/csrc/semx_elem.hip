@@ -10,6 +10,7 @@
 //   k_back   direct modes: u_i = hii F_i - hbi^T u_b, essential values
 //            re-imposed (Element::global2localSC, src/element.cpp:398-438)
 //   k_force  PCG modes: F alone, boundary and interior parts
+//   k_end3   k_cond and k_back for np = 3
 //
 // Condensation and recovery are products of one small matrix per mode and
 // geometric set with as many columns as there are elements of that set,

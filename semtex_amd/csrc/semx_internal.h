@@ -35,7 +35,6 @@ struct MeshDev {
   int* emap = nullptr;       // npnp
   int* pmap = nullptr;       // npnp, inverse of emap
   int* btog = nullptr;       // nel*next
-  int* emask = nullptr;      // nel
   double* ops = nullptr;     // DV DT SDV SDT, 4*npnp
   int* asm_ptr = nullptr;    // nglobal+1
   int* asm_idx = nullptr;    // nel*next

@@ -383,9 +383,9 @@ __device__ inline void elem_apply(const Fac& F, const T (&p)[NP], T (&out)[NP], 
 }
 
 // A thread's column: its element, and the roles of its nodes as bit masks
-// over the rows -- on the element boundary, solved, counted in dot products
-// (the first copy of a node).
-struct Place { int e, el, j, slot0; bool act; unsigned bnd, msk, own; };
+// over the rows -- solved, counted in dot products (the first copy of a
+// node).
+struct Place { int e, el, j, slot0; bool act; unsigned msk, own; };
 
 template <typename T, int NP, bool GREG>
 __device__ inline ElemFac<T, NP, GREG> elem_fac(const ChipMesh& M, const ChipInst& I, const Place& P) {
@@ -553,7 +553,7 @@ __device__ __forceinline__ void chip_solve(const ChipArgs& a, const ChipInst& I,
   if (!P.act) P.el = 0;
   P.e = pt.elo + P.el;
   P.slot0 = P.el * NX;
-  P.bnd = P.msk = P.own = 0;
+  P.msk = P.own = 0;
   if (P.act)
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -562,7 +562,6 @@ __device__ __forceinline__ void chip_solve(const ChipArgs& a, const ChipInst& I,
         P.msk |= 1u << i;
         P.own |= 1u << i;
       } else {
-        P.bnd |= 1u << i;
         if (M.btog[P.e * NX + b] < I.n) {
           P.msk |= 1u << i;
           if (G.tab[P.slot0 + b].x == P.slot0 + b) P.own |= 1u << i;

@@ -14,9 +14,11 @@
 //                   the default; the band sweeps above serve their own
 //                   switches and systems a tree does not fit
 //   k_back          interior recovery and essential re-imposition (semx_elem.hip)
-//   k_pcg           JACPCG, persistent workgroups, one or several per plane
-//                   (FP64, or FP32 / BF16-matrix-core inner PCG with FP64
-//                   refinement)
+//   k_pcg_chip      JACPCG with the vectors held on chip (semx_pcg.hip), the
+//                   default for np 4 to 12 in FP64 and FP32 refined
+//   k_pcg           JACPCG with the vectors in memory, persistent workgroups,
+//                   one or several per plane: BF16-matrix-core refinement,
+//                   other np, larger meshes, and behind its own switches
 //   k_pcg_batch     the same for many independent 2D problems in one launch,
 //                   right-hand side built in the problem's workgroups
 #include <hip/hip_runtime.h>
@@ -1405,8 +1407,9 @@ __global__ __launch_bounds__((coop_bt<NB, NR>())) void k_band_xcoop(CoopArgs a) 
 
 // ===========================================================================
 // Jacobi-preconditioned CG, persistent workgroups (one per plane, or W
-// sharing a plane, below): semtex's JACPCG branch of Field::solve (src/field.cpp:627-720) with the global
-// operator of Field::HelmholtzOperator (src/field.cpp:771-856).
+// sharing a plane, below), vectors in memory: semtex's JACPCG branch of
+// Field::solve (src/field.cpp:627-720) with the global operator of
+// Field::HelmholtzOperator (src/field.cpp:771-856).
 // Vectors are globally numbered: nglobal element-boundary nodes, then the
 // element interiors in emap order.  Rows of essential (and pinned) nodes are
 // held at zero.  T is the precision of the iteration vectors; with
@@ -2441,7 +2444,6 @@ int mesh_upload(Mesh& M) {
   if ((st = dev_upload(&M.d.emap, M.ops.emap.data(), M.ops.emap.size()))) return st;
   if ((st = dev_upload(&M.d.pmap, M.ops.pmap.data(), M.ops.pmap.size()))) return st;
   if ((st = dev_upload(&M.d.btog, M.btog.data(), M.btog.size()))) return st;
-  if ((st = dev_upload(&M.d.emask, M.emask.data(), M.emask.size()))) return st;
   if ((st = dev_upload(&M.d.ops, ops.data(), ops.size()))) return st;
   if ((st = dev_upload(&M.d.asm_ptr, M.asm_ptr.data(), M.asm_ptr.size()))) return st;
   if ((st = dev_upload(&M.d.asm_idx, M.asm_idx.data(), M.asm_idx.size()))) return st;
@@ -2458,7 +2460,7 @@ int mesh_upload(Mesh& M) {
 void mesh_release(Mesh& M) {
   dev_free(M.d.G); dev_free(M.d.eset); dev_free(M.d.emap); dev_free(M.d.pmap);
   dev_free(M.d.btog);
-  dev_free(M.d.emask); dev_free(M.d.ops); dev_free(M.d.asm_ptr); dev_free(M.d.asm_idx);
+  dev_free(M.d.ops); dev_free(M.d.asm_ptr); dev_free(M.d.asm_idx);
   dev_free(M.d.ess_src); dev_free(M.d.nat_ptr); dev_free(M.d.nat_b); dev_free(M.d.bside);
   dev_free(M.d.barea); dev_free(M.d.imass);
   M.on_device = false;

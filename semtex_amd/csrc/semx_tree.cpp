@@ -96,10 +96,12 @@ void tree_plan(Helm& H) {
   for (const ModeSys& S : H.modes)
     if (S.kind == SEMX_DIRECT) { ++nd; pinned |= S.singular != 0; }
   if (nd == 0 || M.nsolve < 2) return;
-  // The tree was faster than the band sweeps on every system measured, from
-  // one 8x8 plane (23 against 47 us) to 32x32 np=11 (0.27 against 4.19 ms),
-  // so only the sweeps' own switches and SEMX_TREE=0 select them -- and
-  // systems with a region too large for a workgroup's LDS (below).
+  // The tree is faster than the band sweeps were on the systems measured (the
+  // figures in semx_tree.hip), but for small meshes with 64 modes, where both
+  // are chains of short launches (8x8 np=5 Nz=128 43 against 40 us, 32x3 np=6
+  // Nz=64 46 against 44).  So only the sweeps' own switches and SEMX_TREE=0
+  // select them -- and systems with a region too large for a workgroup's LDS
+  // (below).
   for (const char* v : {"SEMX_AUTOTUNE", "SEMX_BAND_COOP", "SEMX_BAND_XCOOP", "SEMX_BAND_PARTS"})
     if (getenv(v)) return;
   if (const char* e = getenv("SEMX_TREE")) if (atoi(e) == 0) return;

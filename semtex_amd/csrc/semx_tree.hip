@@ -9,12 +9,12 @@
 // doubles twice.  The tree's matrices are 2.5-8 times fewer bytes (fill
 // grows with the separators, not with the band), are shared by translated
 // copies of a region, and every region of a stage and every mode is
-// independent.  Measured, whole solves (band sweeps -> tree): 16x16 quads
-// np=9 Nz=64 292 -> 150 us (matrices 110 MB against 444 MB of factor);
-// 32x32 np=11 Nz=16 4190 -> 271 us; three fields on 20x12 np=8 Nz=32
-// periodic in x 394 -> 183 us; 8x8 np=8 one plane 47 -> 23 us; 11x7 np=6
-// Nz=36 all elements distinct 48 -> 42 us; two DNS steps on 24x24 np=9
-// Nz=96 12.7 -> 6.0 ms.
+// independent.  Measured, whole solves, us (band sweeps with the element
+// kernels of semx_elem.hip -> tree with them): 16x16 quads np=9 Nz=64 267 ->
+// 113 (matrices 110 MB against 444 MB of factor; 156 MB of HBM traffic a
+// solve); 32x32 np=11 Nz=16 4124 -> 180; three fields on 20x12 np=8 Nz=32
+// periodic in x 305 -> 128; 8x8 np=8 one plane 47 -> 25; 11x7 np=6 Nz=36 all
+// elements distinct 45 -> 38.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
