@@ -682,7 +682,7 @@ int elem_scratch(Helm& H, int nf) {
   ElemDev* D = H.d.elem;
   int st;
   if (nf <= D->nf_cap) return SEMX_OK;
-  dev_free(D->L);
+  retire(H, D->L);
   D->nf_cap = 0;
   if ((st = dev_upload<double>(&D->L, nullptr, (size_t)H.nplanes * nf * D->nbe * H.M->npnp))) return st;
   for (int f = 1; f <= nf; ++f)

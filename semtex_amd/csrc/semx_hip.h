@@ -42,6 +42,15 @@ inline void dev_free(T*& p) {
   p = nullptr;
 }
 
+// Gives back scratch that a larger one replaces, or keeps it until the system
+// is released where a solve has been captured: the graph goes on using it.
+template <class T>
+inline void retire(Helm& H, T*& p) {
+  if (p && H.pcg_frozen) H.d.retired.push_back((void*)p);
+  else if (p) (void)hipFree((void*)p);
+  p = nullptr;
+}
+
 // Field::solve over all planes of one system (the body of semx_helm_solve).
 int helm_solve(Helm& H, double* f, const double* bc, double* u, double tol_rel, int step_max,
                int* iters, hipStream_t s);

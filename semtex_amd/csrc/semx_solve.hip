@@ -2595,6 +2595,8 @@ void helm_release(Helm& H) {
   dev_free(H.d.err);
   dev_free(H.d.spk); dev_free(H.d.spk_off); dev_free(H.d.prow); dev_free(H.d.pslot);
   dev_free(H.d.pctr); dev_free(H.d.pslot2); dev_free(H.d.pwmap);
+  for (void*& p : H.d.retired) dev_free(p);
+  H.d.retired.clear();
   elem_release(H);
   tree_release(H);
   if (ChipDev* C = H.d.chip) {
@@ -2620,8 +2622,8 @@ int helm_scratch(Helm& H, int nf, hipStream_t s) {
   if (H.tree.on)
     if (const int st = tree_scratch(H, nf)) return st;
   if (const int st = elem_scratch(H, nf)) return st;
-  dev_free(H.d.Fb); dev_free(H.d.Fi); dev_free(H.d.g); dev_free(H.d.sol);
-  dev_free(H.d.work); dev_free(H.d.iters);
+  retire(H, H.d.Fb); retire(H, H.d.Fi); retire(H, H.d.g); retire(H, H.d.sol);
+  retire(H, H.d.work); retire(H, H.d.iters);
   const size_t np_ = (size_t)H.nplanes * nf;
   const int nzero = M.nglobal - M.nsolve;
   int st;
@@ -2771,8 +2773,8 @@ int pcg_shape(Helm& H, int nf, int& W, bool& bal) {
   W = pcg_uniform(H, fn, lds);
   bal = H.pcg_nwg > 0 && H.d.pwmap && !getenv("SEMX_PCG_WG");
   if ((W > 1 || bal) && (H.pcg_ws < npcg * nf || !H.d.pctr)) {
-    dev_free(H.d.pctr);
-    dev_free(H.d.pslot2);
+    retire(H, H.d.pctr);
+    retire(H, H.d.pslot2);
     int st = dev_upload<unsigned>(&H.d.pctr, nullptr, npcg * nf * 16);
     if (!st) st = dev_upload<double>(&H.d.pslot2, nullptr, npcg * nf * 4 * PCG_WMAX);
     if (!st && !H.d.err) st = dev_upload<int>(&H.d.err, nullptr, 1);
@@ -2822,7 +2824,7 @@ int chip_prepare(Helm& H, int nf) {
   const int W = C->plan.W;
   if (nf > C->nf_cap || C->work != H.d.work) {
     nf = std::max(nf, C->nf_cap);
-    dev_free(C->inst); dev_free(C->exch); dev_free(C->red);
+    retire(H, C->inst); retire(H, C->exch); retire(H, C->red);
     C->nf_cap = 0;
     const size_t np_ = (size_t)npcg * nf;
     if ((st = dev_upload<double>(&C->exch, nullptr, np_ * 4 * C->plan.nif))) return st;

@@ -340,7 +340,7 @@ int tree_scratch(Helm& H, int nf) {
   TreeDev* D = H.d.tree;
   int st;
   if (nf <= D->nf_cap) return SEMX_OK;
-  dev_free(D->C); dev_free(D->Y);
+  retire(H, D->C); retire(H, D->Y);
   D->nf_cap = 0;
   const size_t np = (size_t)H.nplanes * nf;
   if ((st = dev_upload<double>(&D->C, nullptr, np * T.nslot_c))) return st;

@@ -108,3 +108,30 @@ def test_fewer_fields_captured(cuda, method):
     for nf in (1, 2):
         _capture_and_replay(
             torch, lambda us: sx.solve_fields(S, fs[:nf], bs[:nf], us, iters=False), ref[:nf])
+
+
+@pytest.mark.parametrize("method", [sx.DIRECT, sx.JACPCG, sx.MIXED], ids=["direct", "jacpcg", "mixed"])
+def test_captured_solve_outlives_larger_ones(cuda, method):
+    """A solve of one field captured, then solves of two and three fields,
+    which need larger scratch: the graph keeps its own."""
+    import torch
+    print(f"[capture] outgrown scratch, method {method}", flush=True)
+    P, ins = _case(17, 9, 6, 8, [3, 4, 5])
+    S = sx.ModalMatrixSys(P, 2.0, 1.2, 0, 4, 8, method)
+    fs, bs = [i[0] for i in ins], [i[1] for i in ins]
+    ref = [torch.zeros_like(f) for f in fs]
+    sx.solve(S, fs[0], bs[0], ref[0], iters=False)
+    u = torch.zeros_like(fs[0])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        u.zero_()
+        sx.solve(S, fs[0], bs[0], u, iters=False)
+    for nf in (2, 3):
+        vs = [torch.zeros_like(f) for f in fs[:nf]]
+        sx.solve_fields(S, fs[:nf], bs[:nf], vs, iters=False)
+        keep = torch.full((1 << 22,), 7.0, dtype=torch.float64, device="cuda:0")   # reuse what was freed
+        u.fill_(1.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(u, ref[0]) and torch.equal(vs[0], ref[0])
+        assert float(keep.min()) == 7.0 and float(keep.max()) == 7.0
