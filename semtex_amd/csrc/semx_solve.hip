@@ -4065,6 +4065,15 @@ int semx_batch_destroy(semx_batch batch) {
   return SEMX_OK;
 }
 
+struct PtrBlock {
+  static constexpr int N = 256;      // 2 KB of kernel arguments
+  const double* p[N];
+};
+
+static __global__ void k_set_ptrs(const double** dst, PtrBlock b, int n) {
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = b.p[threadIdx.x];
+}
+
 int semx_batch_solve(semx_batch batch, const double* const* f, const double* const* bc,
                      double* const* u, double tol_rel, int step_max, int* iters,
                      void* stream) {
@@ -4080,9 +4089,20 @@ int semx_batch_solve(semx_batch batch, const double* const* f, const double* con
     ptrs[b.count + i] = bc ? bc[i] : nullptr;
     ptrs[2 * b.count + i] = u[i];
   }
-  if (stream_capturing(s)) b.frozen = true;   // a graph keeps the layout's buffers
-  HIPCHK(hipMemcpyAsync(b.ptrs, ptrs.data(), ptrs.size() * sizeof(double*),
-                        hipMemcpyHostToDevice, s));
+  if (stream_capturing(s)) {
+    // a graph keeps the layout's buffers, and the pointers by value: a copy
+    // recorded from ptrs would be made from it at every replay
+    b.frozen = true;
+    for (size_t i = 0; i < ptrs.size(); i += PtrBlock::N) {
+      PtrBlock pb;
+      const int n = (int)std::min<size_t>(PtrBlock::N, ptrs.size() - i);
+      std::copy_n(&ptrs[i], n, pb.p);
+      hipLaunchKernelGGL(k_set_ptrs, dim3(1), dim3(PtrBlock::N), 0, s, b.ptrs + i, pb, n);
+    }
+  } else {
+    HIPCHK(hipMemcpyAsync(b.ptrs, ptrs.data(), ptrs.size() * sizeof(double*),
+                          hipMemcpyHostToDevice, s));
+  }
   if (b.chip) {
     ChipArgs ca{};
     ca.inst = b.cinst; ca.order = b.order; ca.ticket = b.ticket;

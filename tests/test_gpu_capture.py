@@ -135,3 +135,25 @@ def test_captured_solve_outlives_larger_ones(cuda, method):
         torch.cuda.synchronize()
         assert torch.equal(u, ref[0]) and torch.equal(vs[0], ref[0])
         assert float(keep.min()) == 7.0 and float(keep.max()) == 7.0
+
+
+@pytest.mark.parametrize("prec", [sx.PCG_FP64, sx.PCG_BF16_REFINED], ids=["fp64", "bf16r"])
+def test_batch_captured(cuda, prec):
+    """A batch's solve captured (100 problems: more pointers than one block of
+    them), replayed between eager solves into other buffers."""
+    import torch
+    print(f"[capture] batch, precision {prec}", flush=True)
+    hs, fs, bs, keep = [], [], [], []
+    for i in range(100):
+        P, [(f, b)] = _case(2 + i % 4, 2 + i % 3, 4 + i % 5, 1, [i])
+        S = sx.ModalMatrixSys(P, 2.0, 1.2, 0, 1, 1, sx.JACPCG)
+        if prec == sx.PCG_BF16_REFINED:
+            S.set_pcg(prec, inner_tol=1e-2, max_outer=80)
+        keep.append(P)
+        hs.append(S)
+        fs.append(f)
+        bs.append(b)
+    B = sx.Batch(hs)
+    ref = [torch.zeros_like(f) for f in fs]
+    B.solve(fs, bs, ref)
+    _capture_and_replay(torch, lambda us: B.solve(fs, bs, us, iters=False), ref)
