@@ -801,7 +801,13 @@ int chip_workgroups(const Mesh& M) {
   for (int g = 0; g < M.nglobal; ++g)
     if (M.asm_ptr[g + 1] - M.asm_ptr[g] > 4) return 0;
   const int W = (M.nel + elems_per_wg(M.np) - 1) / elems_per_wg(M.np);
-  return W <= CHIP_WMAX ? W : 0;
+  // a problem's workgroups wait for each other, each on a CU of its own: all of
+  // them have to be resident (fewer than 256 CUs on a partitioned device)
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  return W <= std::min(CHIP_WMAX, cus) ? W : 0;
 }
 
 int chip_plan(Mesh& M, ChipPlan& P, const ChipMesh** dev) {
