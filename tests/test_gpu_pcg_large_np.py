@@ -41,3 +41,38 @@ def test_large_np(cuda, np_, monkeypatch):
     else:
         ug, _ = gpu_solve(torch, P, S, f, b)
         assert rel(solved(P, ug), solved(P, uo)) <= 1e-9
+
+
+@pytest.mark.parametrize("np_", [14, 16])
+def test_dns_start_up_with_large_np(cuda, np_, monkeypatch):
+    """The first steps of N_TIME = 3, whose velocity systems are JACPCG, against
+    the CPU oracle: relative L2 <= 1e-10 after five steps at TOL_REL 1e-13."""
+    import ctypes as C
+
+    import numpy as np
+    import torch
+    for v in ("SEMX_PCG_WG", "SEMX_PCG_OP", "SEMX_PCG_CHIP"):
+        monkeypatch.delenv(v, raising=False)
+    print(f"[dns large np] {np_}", flush=True)
+    m = rect_mesh(3, 2, 0, 2 * np.pi, 0, 2 * np.pi, periodic_x=True, periodic_y=True)
+    P, Q = sx.Mesh(np_, m), O.Mesh(np_, m)
+    nz, f = 4, []
+    for c in range(4):
+        a = np.zeros((nz, P.planeSize))
+        for k in (0, 2, 3):
+            q = np.random.default_rng(10 * c + k).standard_normal(3)
+            a[k, :P.nPlane] = 0.3 * q[0] * np.sin(P.x + q[1]) * np.cos(P.y + q[2]) * (c < 3)
+        f.append(a)
+    t = [torch.from_numpy(a.reshape(-1).copy()).to("cuda:0") for a in f]
+    D = sx.DNS(P, nz, 1.0, 2e-3, 0.05, norder=3, tol_rel=1e-13, step_max=5000)
+    D.run(5, *t)
+    o = [np.ascontiguousarray(a.copy()) for a in f]
+    Do = O.lib().orc_dns_create(C.c_void_p(Q.h), nz, 1.0, 2e-3, 0.05, 3, 0, 1e-13, 5000, 0)
+    tm = C.c_double()
+    O.lib().orc_dns_run(C.c_void_p(Do), 5, *(O.dp(a) for a in o), C.byref(tm))
+    O.lib().orc_dns_destroy(C.c_void_p(Do))
+    keep = [0, 2, 3]
+    for name, g, r in zip("uvw", t, o):
+        e = rel(g.cpu().numpy().reshape(r.shape)[keep, :P.nPlane], r[keep, :P.nPlane])
+        print(f"  {name}: rel L2 {e:.2e}", flush=True)
+        assert e <= 1e-10
