@@ -45,7 +45,7 @@ namespace semx {
 typedef double elem_d4 __attribute__((ext_vector_type(4)));
 
 struct ElemList {               // element groups for one field count
-  int4* grp = nullptr;          // first entry of elist, elements, set
+  size_t first = 0;             // of its groups
   int ngrp = 0, ncol = 1;
 };
 
@@ -62,6 +62,7 @@ struct ElemDev {
   int nbe = 0;
   double* L = nullptr;          // their boundary terms: field, plane, entry, node
   int nf_cap = 0;
+  int4* grp = nullptr;          // groups: first entry of elist, elements, set
   ElemList list[SEMX_MAX_FIELDS + 1];
 };
 
@@ -629,7 +630,7 @@ void elem_release(Helm& H) {
   if (!D) return;
   dev_free(D->cond); dev_free(D->back); dev_free(D->elist); dev_free(D->bidx); dev_free(D->blist);
   dev_free(D->bsrc); dev_free(D->L);
-  for (ElemList& l : D->list) dev_free(l.grp);
+  dev_free(D->grp);
   delete D;
   H.d.elem = nullptr;
 }
@@ -643,7 +644,7 @@ static int end_ld(const Mesh& M) {
 // The element groups of nf fields: two column tiles (32 columns) per
 // workgroup, or one where two would leave fewer than 512 workgroups (two per
 // CU).
-static int elem_list(Helm& H, int nf, ElemList& l) {
+static void elem_list(const Helm& H, int nf, ElemList& l, std::vector<int4>& groups) {
   const Mesh& M = *H.M;
   int npl = 1;
   for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) npl = 2;
@@ -673,7 +674,8 @@ static int elem_list(Helm& H, int nf, ElemList& l) {
   for (const int4& q : g) nmax = std::max(nmax, q.y * nrhs);
   l.ncol = nmax;                        // np <= 16: at most 32 x 4 KB
   l.ngrp = (int)g.size();
-  return dev_upload(&l.grp, g.data(), g.size());
+  l.first = groups.size();
+  groups.insert(groups.end(), g.begin(), g.end());
 }
 
 // Boundary-term scratch for nf fields and the element groups of every field
@@ -685,8 +687,12 @@ int elem_scratch(Helm& H, int nf) {
   retire(H, D->L);
   D->nf_cap = 0;
   if ((st = dev_upload<double>(&D->L, nullptr, (size_t)H.nplanes * nf * D->nbe * H.M->npnp))) return st;
-  for (int f = 1; f <= nf; ++f)
-    if (!D->list[f].grp && !H.dmode.empty() && (st = elem_list(H, f, D->list[f]))) return st;
+  if (!H.dmode.empty()) {
+    retire(H, D->grp);
+    std::vector<int4> groups;
+    for (int f = 1; f <= nf; ++f) elem_list(H, f, D->list[f], groups);
+    if ((st = dev_upload(&D->grp, groups.data(), groups.size()))) return st;
+  }
   D->nf_cap = nf;
   return SEMX_OK;
 }
@@ -703,7 +709,7 @@ static EndArgs end_args(Helm& H, int nf, double* const* fs, const double* const*
   for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) a.npl = 2;
   a.nrhs = a.npl * nf;
   a.solstride = H.solstride;
-  a.grp = D.list[nf].grp; a.elist = D.elist; a.bidx = D.bidx;
+  a.grp = D.grp + D.list[nf].first; a.elist = D.elist; a.bidx = D.bidx;
   a.eset = M.d.eset; a.pmap = M.d.pmap; a.btog = M.d.btog;
   a.ess_src = M.d.ess_src; a.G = M.d.G; a.L = D.L;
   a.dmode = H.d.dmode; a.mode_plane = H.d.mode_plane; a.plane_of = H.d.plane_of;

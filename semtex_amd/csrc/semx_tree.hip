@@ -48,7 +48,7 @@ struct TreeDev {
   int nf_cap = 0;
   // launch lists per field count: forward stages, then backward stages
   std::vector<TreeList> list[SEMX_MAX_FIELDS + 1];
-  TreeTask* task[SEMX_MAX_FIELDS + 1] = {nullptr};
+  TreeTask* task = nullptr;     // their tasks
 };
 
 namespace {
@@ -333,8 +333,8 @@ static int tree_lists(const Tree& T, int nrhs, std::vector<TreeList>& out,
 }
 
 // Contribution scratch for nf fields and the launch lists of every field
-// count up to that (one allocation each): a solve of fewer fields may be
-// captured into a graph without a call of its own before it.
+// count up to that (their tasks in one allocation): a solve of fewer fields
+// may be captured into a graph without a call of its own before it.
 int tree_scratch(Helm& H, int nf) {
   Tree& T = H.tree;
   TreeDev* D = H.d.tree;
@@ -347,14 +347,13 @@ int tree_scratch(Helm& H, int nf) {
   if ((st = dev_upload<double>(&D->Y, nullptr, np * T.nslot_y))) return st;
   int npl = 1;
   for (int m : H.dmode) if (H.mode_plane[2 * m + 1] >= 0) npl = 2;
+  retire(H, D->task);
+  std::vector<TreeTask> tasks;
   for (int f = 1; f <= nf; ++f) {
-    if (D->task[f]) continue;
-    std::vector<TreeTask> tasks;
-    std::vector<TreeList> list;
-    if ((st = tree_lists(T, npl * f, list, tasks))) return st;
-    if ((st = dev_upload(&D->task[f], tasks.data(), tasks.size()))) return st;
-    D->list[f] = list;
+    D->list[f].clear();
+    if ((st = tree_lists(T, npl * f, D->list[f], tasks))) return st;
   }
+  if ((st = dev_upload(&D->task, tasks.data(), tasks.size()))) return st;
   D->nf_cap = nf;
   return SEMX_OK;
 }
@@ -364,7 +363,7 @@ void tree_release(Helm& H) {
   if (!D) return;
   dev_free(D->mat); dev_free(D->type); dev_free(D->node); dev_free(D->gid);
   dev_free(D->rowptr); dev_free(D->src); dev_free(D->C); dev_free(D->Y);
-  for (TreeTask*& t : D->task) dev_free(t);
+  dev_free(D->task);
   delete D;
   H.d.tree = nullptr;
 }
@@ -403,7 +402,7 @@ int tree_solve(Helm& H, int nf, size_t pFb, size_t psol, hipStream_t s) {
       fn = l.ct == 1 ? (const void*)k_tree_down<1, false>
                      : l.ct == 2 ? (const void*)k_tree_down<2, false> : (const void*)k_tree_down<3, false>;
     if (!l.ntask) continue;
-    a.task = D->task[nf] + l.first; a.wk = l.wk; a.ldn = l.ldn;
+    a.task = D->task + l.first; a.wk = l.wk; a.ldn = l.ldn;
     if (l.lds > 64 * 1024)
       HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
     void* kargs[] = {&a, &nleaf};
