@@ -2687,7 +2687,7 @@ bool pcg_split(const Helm& H, const void* kfn, size_t lds, std::vector<int>& Wp)
 }
 
 // The workgroup map of that split.
-int pcg_balance(Helm& H, int nf, const void* kfn, size_t lds) {
+int pcg_balance(Helm& H, const void* kfn, size_t lds) {
   const int npcg = (int)H.pcg_plane.size();
   std::vector<int> Wp;
   H.pcg_stale = false;
@@ -2758,10 +2758,11 @@ int pcg_uniform(const Helm& H, const void* fn, size_t lds) {
   return W;
 }
 
-// What a k_pcg launch for nf fields needs: its uniform workgroup count W,
-// and, once a solve has read back the planes' iteration counts -- k_pcg's own
+// What a k_pcg launch needs, for as many fields as the system's scratch holds:
+// its uniform workgroup count W, and, once a solve has read back the planes' iteration counts -- k_pcg's own
 // or the on-chip iteration's --, the balanced map in its place (bal).
-int pcg_shape(Helm& H, int nf, int& W, bool& bal) {
+int pcg_shape(Helm& H, int& W, bool& bal) {
+  const int nf = H.nf_cap;
   const int opk = H.pcg_opk >= 0 ? H.pcg_opk
                   : H.pcg_prec == SEMX_PCG_BF16_REFINED ? OPK_MFMA : OPK_BLOCK;
   const void* fn = pcg_fn(H, opk);
@@ -2769,7 +2770,7 @@ int pcg_shape(Helm& H, int nf, int& W, bool& bal) {
   if (lds > 64 * 1024)
     HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   if (H.pcg_stale && !H.pcg_frozen && !getenv("SEMX_PCG_WG"))
-    if (const int st = pcg_balance(H, nf, fn, lds)) return st;
+    if (const int st = pcg_balance(H, fn, lds)) return st;
   W = pcg_uniform(H, fn, lds);
   bal = H.pcg_nwg > 0 && H.d.pwmap && !getenv("SEMX_PCG_WG");
   if ((W > 1 || bal) && (H.pcg_ws < npcg * nf || !H.d.pctr)) {
@@ -2794,15 +2795,16 @@ std::vector<int2> chip_order(const ChipDev& C, int npcg, int nf) {
   return o;
 }
 
-// The on-chip PCG of a system's planes for nf fields: tables on first use,
-// slots for the largest field count met, and the order the planes are taken
+// The on-chip PCG of a system's planes: tables on first use, slots for as many
+// fields as the system's scratch holds, and the order the planes are taken
 // in: as listed (low modes, which take the most iterations, first), or by
 // the iteration counts of the last solve that read them back.  H.d.chip
 // stays null where the on-chip iteration does not take the system; its own
 // switches (SEMX_PCG_WG, SEMX_PCG_OP, SEMX_PCG_CHIP=0) and BF16 refinement
 // select k_pcg.
-int chip_prepare(Helm& H, int nf) {
+int chip_prepare(Helm& H) {
   Mesh& M = *H.M;
+  const int nf = H.nf_cap;
   const int npcg = (int)H.pcg_plane.size();
   int st;
   if (!H.d.chip_tried) {
@@ -2823,7 +2825,6 @@ int chip_prepare(Helm& H, int nf) {
   if (!C) return SEMX_OK;
   const int W = C->plan.W;
   if (nf > C->nf_cap || C->work != H.d.work) {
-    nf = std::max(nf, C->nf_cap);
     retire(H, C->inst); retire(H, C->exch); retire(H, C->red);
     C->nf_cap = 0;
     const size_t np_ = (size_t)npcg * nf;
@@ -3238,7 +3239,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
               !getenv("SEMX_PCG_WG") && !getenv("SEMX_PCG_OP") &&
               !(getenv("SEMX_PCG_CHIP") && atoi(getenv("SEMX_PCG_CHIP")) == 0);
   if (chip) {
-    if ((st = chip_prepare(H, nf))) return st;
+    if ((st = chip_prepare(H))) return st;
     chip = H.d.chip != nullptr;
   }
   if (chip) {
@@ -3296,7 +3297,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
     const size_t npcg = H.pcg_plane.size();
     int W = 1;
     bool bal = false;
-    if ((st = pcg_shape(H, nf, W, bal))) return st;
+    if ((st = pcg_shape(H, W, bal))) return st;
     H.pcg_w = bal ? H.pcg_wtop : W;
     H.pcg_onchip = false;
     pa.W = W;
@@ -3406,7 +3407,7 @@ int helm_solve_fields(Helm& H, int nf, double* const* fs, const double* const* b
       // the next map at once: the next solve may be captured into a graph
       if (!getenv("SEMX_PCG_WG")) {
         pcg_counted(H, it, nf);
-        if ((st = pcg_shape(H, nf, W, bal))) return st;
+        if ((st = pcg_shape(H, W, bal))) return st;
       }
     }
   }
@@ -4210,7 +4211,7 @@ int semx_helm_set_pcg(semx_helm helm, int precision, double inner_tol, int max_o
   if (H.pcg_onchip && precision == SEMX_PCG_BF16_REFINED) {
     int W = 1;
     bool bal = false;
-    return pcg_shape(H, H.nf_cap, W, bal);
+    return pcg_shape(H, W, bal);
   }
   return SEMX_OK;
 }

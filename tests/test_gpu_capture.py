@@ -157,3 +157,32 @@ def test_batch_captured(cuda, prec):
     ref = [torch.zeros_like(f) for f in fs]
     B.solve(fs, bs, ref)
     _capture_and_replay(torch, lambda us: B.solve(fs, bs, us, iters=False), ref)
+
+
+def test_captured_after_precision_change(cuda):
+    """Three fields solved in one kernel, one field in the other after a change
+    of precision: a solve of two fields is captured in either."""
+    import torch
+    print("[capture] precision changes", flush=True)
+    P, ins = _case(17, 9, 6, 8, [3, 4, 5])
+    fs, bs = [i[0] for i in ins], [i[1] for i in ins]
+    bf16 = dict(precision=sx.PCG_BF16_REFINED, inner_tol=1e-2, max_outer=120)
+    for first, second in ((bf16, {}), ({}, bf16)):
+        S = sx.ModalMatrixSys(P, 2.0, 1.2, 0, 4, 8, sx.JACPCG)
+        S.set_pcg(**first)
+        sx.solve_fields(S, fs, bs, [torch.zeros_like(f) for f in fs], iters=False)
+        S.set_pcg(**second)
+        sx.solve(S, fs[0], bs[0], torch.zeros_like(fs[0]), iters=False)
+        us = [torch.zeros_like(f) for f in fs[:2]]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for u in us:
+                u.zero_()
+            sx.solve_fields(S, fs[:2], bs[:2], us, iters=False)
+        g.replay()
+        torch.cuda.synchronize()
+        for f, b, u in zip(fs, bs, us):
+            v = torch.zeros_like(f)
+            sx.solve(S, f, b, v, iters=False)
+            torch.cuda.synchronize()
+            assert torch.equal(u, v)
